@@ -38,46 +38,13 @@ constexpr int kNrcBlock = 256;
 
 __device__ __forceinline__ __bf16 to_bf16(float x) { return (__bf16)x; }
 
+// max(x, 0) before the rounding to BF16, 0 for a NaN, in one instruction (fmaxf of a matrix-core result
+// takes two: it first quietens a signalling NaN). The upper end only keeps the compiler from turning
+// this into that fmaxf: the largest float rounds to infinity in BF16, as infinity does.
+__device__ __forceinline__ float relu(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 3.402823466e38f); }
+
 __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// feature i of the encoding (see the file comment); d = derived inputs:
-// d[0..2] normalised position, d[3..4] wo angles, d[5..6] normal angles, d[7] roughness, d[8..13] albedos
-__device__ __forceinline__ float feature(int i, const float* d) {
-    const float pi = 3.14159265358979f;
-    if (i < 52) {
-        int a, k, sc;
-        float x;
-        if (i < 36) {
-            a = i / 12;
-            k = (i % 12) >> 1;
-            sc = i & 1;
-            x = d[a];
-        } else {
-            const int r = (i - 36) & 7;
-            a = (i < 44 ? 3 : 5) + (r >> 2);
-            k = (r & 3) >> 1;
-            sc = r & 1;
-            x = d[a];
-        }
-        const float arg = (float)(1 << k) * pi * x;
-        return sc ? cosf(arg) : sinf(arg);
-    }
-    if (i == 52) return 1.0f - expf(-d[7]);
-    if (i < 59) return d[8 + (i - 53)];
-    return i == 59 ? 1.0f : 0.0f;
-}
-
-__device__ __forceinline__ void derive(const NrcBox& box, const float* raw, float* d) {
-    const float pi = 3.14159265358979f;
-    for (int a = 0; a < 3; ++a) d[a] = (raw[a] - box.lo[a]) * box.inv_ext[a];
-    d[3] = acosf(fminf(fmaxf(raw[5], -1.0f), 1.0f)) / pi;
-    d[4] = (atan2f(raw[4], raw[3]) / pi + 1.0f) * 0.5f;
-    d[5] = acosf(fminf(fmaxf(raw[8], -1.0f), 1.0f)) / pi;
-    d[6] = (atan2f(raw[7], raw[6]) / pi + 1.0f) * 0.5f;
-    d[7] = raw[9];
-    for (int k = 0; k < 6; ++k) d[8 + k] = raw[10 + k];
 }
 
 // sin(pi y) and cos(pi y) from the hardware's sine and cosine, whose argument is in revolutions
@@ -91,34 +58,39 @@ __device__ __forceinline__ void sincospi_hw(float y, float* s, float* c) {
     *c = __builtin_amdgcn_cosf(r);
 }
 
-// B operand of the first layer for lane group g: slot (kc, j) holds feature perm(kc, 8g + j)
-// Slots j and j + 1 (j even) hold features i and i + 1 with i even: below 52 these are the sine
-// and cosine of the same argument 2^k pi x, computed together from the exact 2^k x.
+// the four features sin, cos(pi y), sin, cos(2 pi y)
+__device__ __forceinline__ void octaves(float y, float f[4]) {
+    sincospi_hw(y, &f[0], &f[1]);
+    sincospi_hw(2.0f * y, &f[2], &f[3]);
+}
+
+// B operand of the first layer for lane group g: slot (kc, j) holds feature perm(kc, 8g + j), that is,
+// output tile t = 2kc + j/4 of a layer holds features 16t + 4g .. 16t + 4g + 3. A lane computes its own
+// 16 features only: two octaves of one coordinate per tile (their arguments 2^k x are exact), and of
+// the four angles the one that its group needs (g = 1: acos(wo.z), 2: atan2(wo), 3: acos(n.z), 0:
+// atan2(n)), so that a query costs one acos and one atan2 per lane, not four.
 __device__ __forceinline__ void encode(const NrcBox& box, const float* raw, int g, bf16x8 b[2]) {
-    float d[14];
-    derive(box, raw, d);
+    const float pi = 3.14159265358979f;
+    float x[3];
+    for (int a = 0; a < 3; ++a) x[a] = (raw[a] - box.lo[a]) * box.inv_ext[a];
+    const float polar = acosf(fminf(fmaxf(g == 1 ? raw[5] : raw[8], -1.0f), 1.0f)) / pi;
+    const float azimuth = (atan2f(g == 2 ? raw[4] : raw[7], g == 2 ? raw[3] : raw[6]) / pi + 1.0f) * 0.5f;
+    const float angle = (g & 1) ? polar : azimuth;
+    float f[4][4];
+    // features 0..35 are (x, y, z) x octaves 0..5: tile 0 holds x 0-1, x 2-3, x 4-5, y 0-1 for g = 0..3,
+    // tile 1 y 2-3, y 4-5, z 0-1, z 2-3, tile 2 z 4-5 (g = 0)
+    octaves((g == 3 ? x[1] : x[0]) * (g == 1 ? 4.0f : g == 2 ? 16.0f : 1.0f), f[0]);
+    octaves((g < 2 ? x[1] : x[2]) * (g == 1 ? 16.0f : g == 2 ? 1.0f : 4.0f), f[1]);
+    octaves(g == 0 ? x[2] * 16.0f : angle, f[2]);
+    octaves(angle, f[3]);
+    if (g != 0) {  // roughness, albedos, one, zeros
+        f[3][0] = g == 1 ? 1.0f - expf(-raw[9]) : g == 2 ? raw[13] : 0.0f;
+        f[3][1] = g == 1 ? raw[10] : g == 2 ? raw[14] : 0.0f;
+        f[3][2] = g == 1 ? raw[11] : g == 2 ? raw[15] : 0.0f;
+        f[3][3] = g == 1 ? raw[12] : g == 2 ? 1.0f : 0.0f;
+    }
     for (int kc = 0; kc < 2; ++kc)
-        for (int j = 0; j < 8; j += 2) {
-            const int i = (2 * kc + (j >> 2)) * 16 + g * 4 + (j & 3);
-            float f0, f1;
-            if (i < 52) {
-                int a, k;
-                if (i < 36) {
-                    a = i / 12;
-                    k = (i % 12) >> 1;
-                } else {
-                    const int r = (i - 36) & 7;
-                    a = (i < 44 ? 3 : 5) + (r >> 2);
-                    k = (r & 3) >> 1;
-                }
-                sincospi_hw((float)(1 << k) * d[a], &f0, &f1);
-            } else {
-                f0 = feature(i, d);
-                f1 = feature(i + 1, d);
-            }
-            b[kc][j] = to_bf16(f0);
-            b[kc][j + 1] = to_bf16(f1);
-        }
+        for (int j = 0; j < 8; ++j) b[kc][j] = to_bf16(f[2 * kc + (j >> 2)][j & 3]);
 }
 
 // one hidden layer: out = relu(W x) as the next B operand; w = packed fragments [ot][kc][lane][8]
@@ -130,28 +102,31 @@ __device__ __forceinline__ void hidden_layer(const bf16x8* w, int lane, const bf
         for (int kc = 0; kc < 2; ++kc) acc[ot] = mfma(w[(ot * 2 + kc) * 64 + lane], in[kc], acc[ot]);
     }
     for (int kc = 0; kc < 2; ++kc)
-        for (int j = 0; j < 8; ++j) out[kc][j] = to_bf16(fmaxf(acc[2 * kc + (j >> 2)][j & 3], 0.0f));
+        for (int j = 0; j < 8; ++j) out[kc][j] = to_bf16(relu(acc[2 * kc + (j >> 2)][j & 3]));
     if (pre)
         for (int ot = 0; ot < 4; ++ot) pre[ot] = acc[ot];
 }
 
-// hidden_layer for two tiles of 16 queries: each weight fragment read from LDS feeds both
-__device__ __forceinline__ void hidden_layer2(const bf16x8* w, int lane, const bf16x8 in0[2], const bf16x8 in1[2],
+// hidden_layer for two tiles of 16 queries, its 8 weight fragments in registers
+__device__ __forceinline__ void hidden_layer2(const bf16x8* w, const bf16x8 in0[2], const bf16x8 in1[2],
                                               bf16x8 out0[2], bf16x8 out1[2]) {
     f32x4 acc0[4], acc1[4];
+#pragma unroll
     for (int ot = 0; ot < 4; ++ot) {
         acc0[ot] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         acc1[ot] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
         for (int kc = 0; kc < 2; ++kc) {
-            const bf16x8 wf = w[(ot * 2 + kc) * 64 + lane];
-            acc0[ot] = mfma(wf, in0[kc], acc0[ot]);
-            acc1[ot] = mfma(wf, in1[kc], acc1[ot]);
+            acc0[ot] = mfma(w[ot * 2 + kc], in0[kc], acc0[ot]);
+            acc1[ot] = mfma(w[ot * 2 + kc], in1[kc], acc1[ot]);
         }
     }
+#pragma unroll
     for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
         for (int j = 0; j < 8; ++j) {
-            out0[kc][j] = to_bf16(fmaxf(acc0[2 * kc + (j >> 2)][j & 3], 0.0f));
-            out1[kc][j] = to_bf16(fmaxf(acc1[2 * kc + (j >> 2)][j & 3], 0.0f));
+            out0[kc][j] = to_bf16(relu(acc0[2 * kc + (j >> 2)][j & 3]));
+            out1[kc][j] = to_bf16(relu(acc1[2 * kc + (j >> 2)][j & 3]));
         }
 }
 
@@ -169,23 +144,33 @@ __device__ __forceinline__ void load_weights_lds(bf16x8* lds, const bf16x8* __re
 
 // inference over n queries of `stride` floats (first 16 = inputs). kAccumulate: out_rgb[path] +=
 // thr * max(pred, 0) with thr = record[16..18] and path = bits of record[19]; else out[q*3 + c] = pred.
+//
+// Bound by VALU issue (the encoding and the ReLU and rounding between the layers, some 800 instructions
+// per 32 queries and lane, beside 68 matrix instructions). Every wave keeps the whole network's 34
+// weight fragments in registers (136 of its 256: 2 waves per SIMD) and runs through the queries, two
+// tiles of 16 at a time; read from LDS they were 34 KB per 32 queries, as long as the matrix
+// instructions themselves. 1,000,003 queries: 97.7 us with the weights in LDS and every lane encoding
+// all four angles, 61.4 with both changed, 54.3 (610 TFLOP/s) with the one-instruction relu.
 template <bool kAccumulate>
-__global__ __launch_bounds__(kNrcBlock) void k_nrc_infer(const bf16x8* __restrict__ packed, NrcBox box,
-                                                         const float* __restrict__ rec, uint32_t n,
-                                                         const uint32_t* __restrict__ n_dev, uint32_t stride,
-                                                         float* __restrict__ out,
-                                                         const uint32_t* __restrict__ begin_dev) {
-    __shared__ bf16x8 w[kFwdSize / 8];
-    load_weights_lds(w, packed, kFwdSize / 8);
+__global__ __launch_bounds__(kNrcBlock, 2) void k_nrc_infer(const bf16x8* __restrict__ packed, NrcBox box,
+                                                            const float* __restrict__ rec, uint32_t n,
+                                                            const uint32_t* __restrict__ n_dev, uint32_t stride,
+                                                            float* __restrict__ out,
+                                                            const uint32_t* __restrict__ begin_dev) {
     if (n_dev) n = min(n, *n_dev);  // count written by an earlier kernel on the stream
     const uint32_t begin = begin_dev ? min(*begin_dev, n) : 0u;
     const int lane = threadIdx.x & 63, g = lane >> 4;
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const uint32_t n_waves = (gridDim.x * blockDim.x) >> 6;
     const uint32_t pairs = (n - begin + 31) / 32;  // two tiles of 16 queries per wave and step
+    if (wave >= pairs) return;
+    bf16x8 w[kFwdSize / 512];
+#pragma unroll
+    for (int i = 0; i < kFwdSize / 512; ++i) w[i] = packed[i * 64 + lane];
     for (uint32_t t = wave; t < pairs; t += n_waves) {
         uint32_t q[2];
         bf16x8 a[2][2], b[2][2];
+#pragma unroll
         for (int h = 0; h < 2; ++h) {
             q[h] = begin + t * 32 + 16 * h + (lane & 15);
             float raw[16];
@@ -205,12 +190,14 @@ __global__ __launch_bounds__(kNrcBlock) void k_nrc_infer(const bf16x8* __restric
             }
             encode(box, raw, g, a[h]);
         }
-        hidden_layer2(w + 0 * (kFwdLayer / 8), lane, a[0], a[1], b[0], b[1]);
-        hidden_layer2(w + 1 * (kFwdLayer / 8), lane, b[0], b[1], a[0], a[1]);
-        hidden_layer2(w + 2 * (kFwdLayer / 8), lane, a[0], a[1], b[0], b[1]);
-        hidden_layer2(w + 3 * (kFwdLayer / 8), lane, b[0], b[1], a[0], a[1]);
+        hidden_layer2(w, a[0], a[1], b[0], b[1]);
+        hidden_layer2(w + 8, b[0], b[1], a[0], a[1]);
+        hidden_layer2(w + 16, a[0], a[1], b[0], b[1]);
+        hidden_layer2(w + 24, b[0], b[1], a[0], a[1]);
+#pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const f32x4 o = output_layer(w + 4 * (kFwdLayer / 8), lane, a[h]);
+            f32x4 o{0.0f, 0.0f, 0.0f, 0.0f};  // lane group 0 gets the 3 outputs of query lane % 16
+            for (int kc = 0; kc < 2; ++kc) o = mfma(w[32 + kc], a[h][kc], o);
             if (g == 0 && q[h] < n) {
                 if (kAccumulate) {
                     const float* r = rec + (size_t)q[h] * stride;
@@ -512,7 +499,7 @@ int nrc_infer(cupbr_nrc* c, const float* rec, uint32_t n, const uint32_t* n_dev,
               bool accumulate, hipStream_t stream, const uint32_t* begin_dev) {
     if (n == 0) return CUPBR_OK;
     const uint32_t pairs = (n + 31) / 32;  // a wave takes two 16-query tiles at a time
-    const int blocks = (int)std::max<uint32_t>(1, std::min<uint32_t>((pairs + 3) / 4, (uint32_t)device_cu_count() * 4));
+    const int blocks = (int)std::max<uint32_t>(1, std::min<uint32_t>((pairs + 3) / 4, (uint32_t)device_cu_count() * 2));
     if (accumulate)
         hipLaunchKernelGGL(k_nrc_infer<true>, dim3(blocks), dim3(kNrcBlock), 0, stream, c->packed_fwd.as<bf16x8>(),
                            c->box, rec, n, n_dev, stride, out, begin_dev);
