@@ -23,9 +23,9 @@ struct cupbr_nrc {
     cupbr::NrcBox box{};
     cupbr::DevBuf w, m, v;                   // FP32 weights and Adam moments
     cupbr::DevBuf packed_fwd, packed_bwd;    // BF16 matrix-core fragments of W and W^T
-    cupbr::DevBuf acts, partial;             // training scratch: activations, per-slice weight gradients
-    uint32_t acts_cleared_for = 0;
-    uint32_t step = 0;
+    cupbr::DevBuf acts, losses, sums;        // training scratch: activations and gradients, per-block losses,
+                                             // weight-gradient sums per slice of the batch
+    cupbr::DevBuf state, bias;               // step numbers; Adam's bias corrections by step
     float beta1 = 0.9f, beta2 = 0.99f, eps = 1e-10f;
 };
 
@@ -43,8 +43,10 @@ int nrc_infer(cupbr_nrc* c, const float* rec, uint32_t n, const uint32_t* n_dev,
               bool accumulate, hipStream_t stream, const uint32_t* begin_dev = nullptr);
 // D = A B (16x32 by 32x16) through one matrix-core instruction with the cache's fragment layout
 int nrc_mfma_product(const float* a, const float* b, float* d);
-// `steps` Adam steps on batches of `batch` rows drawn from rows[0, n_rows) (stride kNrcRowStride)
+// `steps` Adam steps on batches of `batch` rows (a multiple of 512) drawn from rows[0, n_rows) (stride
+// kNrcRowStride); with n_rows_dev from the first min(n_rows, *n_rows_dev) rows (a count on the device),
+// and no step when that is 0
 int nrc_train(cupbr_nrc* c, const float* rows, uint32_t n_rows, uint32_t batch, uint32_t steps, float lr,
-              float* loss_dev, hipStream_t stream);
+              float* loss_dev, hipStream_t stream, const uint32_t* n_rows_dev = nullptr);
 
 }  // namespace cupbr

@@ -137,11 +137,6 @@ __device__ __forceinline__ f32x4 output_layer(const bf16x8* w5, int lane, const 
     return acc;
 }
 
-__device__ __forceinline__ void load_weights_lds(bf16x8* lds, const bf16x8* __restrict__ packed, int n_frag) {
-    for (int i = threadIdx.x; i < n_frag; i += blockDim.x) lds[i] = packed[i];
-    __syncthreads();
-}
-
 // inference over n queries of `stride` floats (first 16 = inputs). kAccumulate: out_rgb[path] +=
 // thr * max(pred, 0) with thr = record[16..18] and path = bits of record[19]; else out[q*3 + c] = pred.
 //
@@ -225,151 +220,249 @@ __device__ __forceinline__ uint32_t hash32(uint32_t x) {
     return x;
 }
 
-// activations of the batch for the weight gradients: X[layer][feature][query] (inputs of layers
-// 1..5) and G[layer][feature][query] (loss gradient at the outputs of layers 1..5, after the ReLU
-// mask), both BF16; batch row b uses training row rows[(hash(seed + b)) % n_rows]
-__device__ __forceinline__ void store_feats(__bf16* base, uint32_t B, uint32_t q, int g, const bf16x8 v[2]) {
-    for (int kc = 0; kc < 2; ++kc)
-        for (int j = 0; j < 8; ++j) base[(size_t)((2 * kc + (j >> 2)) * 16 + g * 4 + (j & 3)) * B + q] = v[kc][j];
+// Training state on the device: steps taken since the weights were set, and the number of the step at
+// hand (each written by one thread of a launch that does not read it).
+struct TrainState {
+    uint32_t taken, step;
+};
+
+// Step s of a call: forward, loss and backward for one training batch of B rows (a multiple of 64), 64
+// rows per tile. Batch row q is rows[hash(seed + q) % n_rows], its seed from the step number.
+//
+// A wave takes 16 rows through the network in registers (the weights of both directions in LDS). The
+// weight gradients dW[o][i] = sum_q G[o][q] X[i][q] of k_nrc_weight_sums then need the batch rows as the K
+// dimension: the inputs X of the five layers and the loss gradients G at their outputs go through LDS
+// as [feature][row] (rows of 64 + 8 values, so that the 16 lanes of an operand load read all 64 banks
+// once) and from there to memory as matrix operands, acts[row / 512][operand][row % 512 / 32][lane] of 16
+// bytes: operands 0..19 are X[layer][16 features], 20..35 G[hidden layer][16 outputs], 36 the output
+// layer's G.
+// Bound by the latency of one 16-row chain per SIMD and the 20 MB of operands. 16,384 rows: 26.7 us when
+// every value went to memory as a 2-byte store and the weights to LDS one load after the other, now
+// 11.3; 16.7 with operands 16 KB apart, 14.6 with a slice's tiles on all XCDs.
+constexpr int kTrainRows = 64;
+constexpr int kTrainStride = kTrainRows + 8;
+constexpr uint32_t kOperands = 37;
+constexpr uint32_t kSlice = 512;                         // batch rows whose gradients are added up first
+// 16-byte values of one operand of a slice, and 1 KB between operands: 16 KB apart, the pieces that a
+// block writes of every operand would share memory channels
+constexpr uint32_t kSliceOperand = kSlice / 32 * 64 + 64;
+constexpr uint32_t kSliceTiles = kSlice / kTrainRows;
+// The u-th tile of a batch: a slice's tiles are 8 apart, so that (blocks going round the XCDs) one XCD
+// makes all of a slice, the one on which k_nrc_weight_sums reads it.
+__device__ __forceinline__ uint32_t tile_at(uint32_t u) {
+    return ((u / (8u * kSliceTiles)) * 8u + (u & 7u)) * kSliceTiles + (u >> 3) % kSliceTiles;
 }
 
-__global__ __launch_bounds__(kNrcBlock) void k_nrc_forward_backward(const bf16x8* __restrict__ pf,
-                                                                    const bf16x8* __restrict__ pb, NrcBox box,
-                                                                    const float* __restrict__ rows, uint32_t n_rows,
-                                                                    uint32_t B, uint32_t seed, __bf16* __restrict__ X,
-                                                                    __bf16* __restrict__ G, float* loss) {
+__device__ __forceinline__ void store_rows(__bf16* base, int row, int g, const bf16x8 v[2]) {
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) base[((2 * kc + (j >> 2)) * 16 + g * 4 + (j & 3)) * kTrainStride + row] = v[kc][j];
+}
+
+__global__ __launch_bounds__(kNrcBlock, 1) void k_nrc_train(const bf16x8* __restrict__ pf, const bf16x8* __restrict__ pb,
+                                                            NrcBox box, const float* __restrict__ rows, uint32_t n_rows,
+                                                            const uint32_t* __restrict__ n_rows_dev, uint32_t B,
+                                                            TrainState* state, uint32_t s, bf16x8* __restrict__ acts,
+                                                            float* __restrict__ losses) {
     __shared__ bf16x8 wf[kFwdSize / 8];
     __shared__ bf16x8 wb[kBwdSize / 8];
-    for (int i = threadIdx.x; i < kBwdSize / 8; i += blockDim.x) wb[i] = pb[i];
-    load_weights_lds(wf, pf, kFwdSize / 8);
-    const int lane = threadIdx.x & 63, g = lane >> 4;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t n_waves = (gridDim.x * blockDim.x) >> 6;
-    const size_t layer = (size_t)64 * B;
+    // [layer][feature][row]: X of the 5 layers, then G of the 4 hidden ones
+    __shared__ __attribute__((aligned(16))) __bf16 xg[9][64 * kTrainStride];
+    __shared__ __attribute__((aligned(16))) __bf16 g5[16 * kTrainStride];
+    __shared__ float loss_s[kNrcBlock / 64];
+    const int lane = threadIdx.x & 63, g = lane >> 4, wave = threadIdx.x >> 6;
+    const int col = wave * 16 + (lane & 15);
+    // the weights, the counts and then the first row: their loads in flight together (the weights one
+    // after the other take 7 us more)
+    constexpr int nf = (kFwdSize / 8 + kNrcBlock - 1) / kNrcBlock, nb = (kBwdSize / 8 + kNrcBlock - 1) / kNrcBlock;
+    bf16x8 f[nf], b[nb];
+#pragma unroll
+    for (int k = 0; k < nf; ++k) f[k] = pf[min((int)threadIdx.x + k * kNrcBlock, kFwdSize / 8 - 1)];
+#pragma unroll
+    for (int k = 0; k < nb; ++k) b[k] = pb[min((int)threadIdx.x + k * kNrcBlock, kBwdSize / 8 - 1)];
+    if (n_rows_dev) n_rows = min(n_rows, *n_rows_dev);
+    const uint32_t step = state->taken + s + 1u;
+    if (n_rows == 0) return;
+    if (tile_at(blockIdx.x) >= B / kTrainRows) {  // the last slices of a batch that is no multiple of 4096 rows
+        if (threadIdx.x == 0) losses[blockIdx.x] = 0.0f;
+        return;
+    }
+    const uint32_t seed = step * 0x9E3779B9u + 0x51ED270Bu;
+    float raw[19];
+    auto load_row = [&](uint32_t t) {
+        const float* r = rows + (size_t)(hash32(seed + t * kTrainRows + col) % n_rows) * kNrcRowStride;
+#pragma unroll
+        for (int k = 0; k < 19; ++k) raw[k] = r[k];
+    };
+    load_row(tile_at(blockIdx.x));
+#pragma unroll
+    for (int k = 0; k < nf; ++k)
+        if ((int)threadIdx.x + k * kNrcBlock < kFwdSize / 8) wf[threadIdx.x + k * kNrcBlock] = f[k];
+#pragma unroll
+    for (int k = 0; k < nb; ++k)
+        if ((int)threadIdx.x + k * kNrcBlock < kBwdSize / 8) wb[threadIdx.x + k * kNrcBlock] = b[k];
+    __syncthreads();
     float loss_acc = 0.0f;
-    for (uint32_t t = wave; t < B / 16; t += n_waves) {
-        const uint32_t q = t * 16 + (lane & 15);
-        const uint32_t row = hash32(seed + q) % n_rows;
-        const float* r = rows + (size_t)row * kNrcRowStride;
-        float raw[16];
-        for (int k = 0; k < 16; ++k) raw[k] = r[k];
+    for (uint32_t u = blockIdx.x; tile_at(u) < B / kTrainRows; u += gridDim.x) {  // gridDim.x: a multiple of 64
+        const uint32_t t = tile_at(u);
+        if (u != blockIdx.x) load_row(t);
         bf16x8 x[5][2];
         f32x4 pre[4][4];
         encode(box, raw, g, x[0]);
+#pragma unroll
         for (int L = 0; L < 4; ++L) hidden_layer(wf + L * (kFwdLayer / 8), lane, x[L], x[L + 1], pre[L]);
         const f32x4 o = output_layer(wf + 4 * (kFwdLayer / 8), lane, x[4]);
         // relative L2: sum_c (o_c - y_c)^2 / (o_c^2 + 0.01), o_c detached in the denominator
-        bf16x8 dy[2];
+        bf16x8 cur[2];
+#pragma unroll
         for (int kc = 0; kc < 2; ++kc)
-            for (int j = 0; j < 8; ++j) dy[kc][j] = to_bf16(0.0f);
-        float d5[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int j = 0; j < 8; ++j) cur[kc][j] = to_bf16(0.0f);
         if (g == 0) {
+#pragma unroll
             for (int c = 0; c < 3; ++c) {
                 const float den = o[c] * o[c] + 0.01f;
-                const float e = o[c] - r[16 + c];
+                const float e = o[c] - raw[16 + c];
                 loss_acc += e * e / den;
-                d5[c] = 2.0f * e / den;
-                dy[0][c] = to_bf16(d5[c]);
+                cur[0][c] = to_bf16(2.0f * e / den);
             }
         }
-        for (int L = 0; L < 5; ++L) store_feats(X + L * layer, B, q, g, x[L]);
-        // G[4] holds rows 0..2 of the output gradient (rows 3..63 stay zero)
-        if (g == 0)
-            for (int c = 0; c < 3; ++c) G[4 * layer + (size_t)c * B + q] = dy[0][c];
+#pragma unroll
+        for (int L = 0; L < 5; ++L) store_rows(xg[L], col, g, x[L]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) g5[(g * 4 + j) * kTrainStride + col] = g == 0 ? cur[0][j] : to_bf16(0.0f);
         // backward through W5^T, then W4^T..W2^T, masking with the ReLU of each hidden layer
-        bf16x8 cur[2] = {dy[0], dy[1]};
+#pragma unroll
         for (int L = 3; L >= 0; --L) {
             f32x4 acc[4];
+#pragma unroll
             for (int it = 0; it < 4; ++it) {
                 acc[it] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 if (L == 3) {
                     acc[it] = mfma(wb[3 * (kFwdLayer / 8) + it * 64 + lane], cur[0], acc[it]);
                 } else {
+#pragma unroll
                     for (int kc = 0; kc < 2; ++kc)
                         acc[it] = mfma(wb[L * (kFwdLayer / 8) + (it * 2 + kc) * 64 + lane], cur[kc], acc[it]);
                 }
             }
-            bf16x8 nxt[2];
+#pragma unroll
             for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const int ot = 2 * kc + (j >> 2), v = j & 3;
-                    nxt[kc][j] = to_bf16(pre[L][ot][v] > 0.0f ? acc[ot][v] : 0.0f);
+                    cur[kc][j] = to_bf16(pre[L][ot][v] > 0.0f ? acc[ot][v] : 0.0f);
                 }
-            store_feats(G + L * layer, B, q, g, nxt);
-            cur[0] = nxt[0];
-            cur[1] = nxt[1];
+            store_rows(xg[5 + L], col, g, cur);
         }
-    }
-    if (loss) {
-        for (int off = 32; off > 0; off >>= 1) loss_acc += __shfl_xor(loss_acc, off);
-        if (lane == 0) atomicAdd(loss, loss_acc);
-    }
-}
-
-// weight gradients of one layer over one slice of the batch: dW[o][i] = sum_q G[o][q] X[i][q],
-// written (not accumulated) to partial[slice][param offset]
-template <int kOutTiles>  // 4: hidden layers W1..W4; 1: output layer W5
-__device__ __forceinline__ void weight_grad_layer(int layer, const __bf16* __restrict__ X,
-                                                  const __bf16* __restrict__ G, uint32_t B, uint32_t slice,
-                                                  float* __restrict__ partial) {
-    const uint32_t s = blockIdx.x;          // slice index
-    const int lane = threadIdx.x, g = lane >> 4;
-    constexpr int n_ot = kOutTiles;
-    const __bf16* Xl = X + (size_t)layer * 64 * B;
-    const __bf16* Gl = G + (size_t)layer * 64 * B;
-    f32x4 acc[kOutTiles][4];
-#pragma unroll
-    for (int a = 0; a < kOutTiles; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t q0 = s * slice; q0 < (s + 1) * slice; q0 += 32) {
-        const uint32_t qq = q0 + 8 * g;
-        bf16x8 bx[4];
-        for (int it = 0; it < 4; ++it)
-            bx[it] = *reinterpret_cast<const bf16x8*>(Xl + (size_t)(it * 16 + (lane & 15)) * B + qq);
-        for (int ot = 0; ot < n_ot; ++ot) {
-            const bf16x8 ag = *reinterpret_cast<const bf16x8*>(Gl + (size_t)(ot * 16 + (lane & 15)) * B + qq);
-            for (int it = 0; it < 4; ++it) acc[ot][it] = mfma(ag, bx[it], acc[ot][it]);
+        __syncthreads();
+        // operand rows: lane l holds row l % 16 of its 16 features, batch rows 32 half + 8 (l / 16) .. + 7
+        const int at = (lane & 15) * kTrainStride + 8 * g;
+        bf16x8* to = acts + (size_t)(t / kSliceTiles) * kOperands * kSliceOperand +
+                     t % kSliceTiles * (kTrainRows / 32 * 64) + lane;
+        for (uint32_t k = wave; k < 2 * kOperands; k += kNrcBlock / 64) {
+            const uint32_t half = k & 1u, op = k >> 1;
+            const __bf16* from = op < 36u ? xg[op >> 2] + (op & 3u) * 16u * kTrainStride : g5;
+            to[op * kSliceOperand + half * 64u] = *reinterpret_cast<const bf16x8*>(from + at + 32 * half);
         }
+        __syncthreads();
     }
-    float* out = partial + (size_t)s * kNrcParams;
-    for (int ot = 0; ot < n_ot; ++ot)
-        for (int it = 0; it < 4; ++it)
-            for (int v = 0; v < 4; ++v) {
-                const int o = ot * 16 + g * 4 + v, i = it * 16 + (lane & 15);
-                if (layer == 4) {
-                    if (o < 3) out[4 * 4096 + o * 64 + i] = acc[ot][it][v];
-                } else {
-                    out[layer * 4096 + o * 64 + i] = acc[ot][it][v];
-                }
-            }
-}
-
-// all five layers in one launch: blockIdx.x = slice, blockIdx.y = layer (4: the output layer)
-__global__ __launch_bounds__(64) void k_nrc_weight_grad(const __bf16* __restrict__ X, const __bf16* __restrict__ G,
-                                                        uint32_t B, uint32_t slice, float* __restrict__ partial) {
-    if (blockIdx.y < 4)
-        weight_grad_layer<4>((int)blockIdx.y, X, G, B, slice, partial);
-    else
-        weight_grad_layer<1>(4, X, G, B, slice, partial);
+    for (int off = 32; off > 0; off >>= 1) loss_acc += __shfl_xor(loss_acc, off);
+    if (lane == 0) loss_s[wave] = loss_acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float sum = 0.0f;
+        for (int k = 0; k < kNrcBlock / 64; ++k) sum += loss_s[k];
+        losses[blockIdx.x] = sum;
+        if (blockIdx.x == 0) state->step = step;
+    }
 }
 
 __device__ __forceinline__ void pack_weight(uint32_t p, float w, __bf16* __restrict__ pf, __bf16* __restrict__ pb);
 
-// sum of the slice partials, Adam, and the packed BF16 copies for the next forward/backward
-__global__ void k_nrc_adam(const float* __restrict__ partial, uint32_t n_slices, float inv_b, float* __restrict__ w,
-                           float* __restrict__ m, float* __restrict__ v, float lr, float b1, float b2, float eps,
-                           float bc1, float bc2, __bf16* __restrict__ pf, __bf16* __restrict__ pb) {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kNrcParams) return;
+// Weight gradients of slices of 512 batch rows: one wave takes a slice of one 16 x 16 tile of a layer's
+// weights through 16 matrix instructions in row order, all 32 operand loads in flight together. The
+// order of the rows, and of the slices in k_nrc_adam, is fixed: it decides the last bits of the gradients,
+// and with them when a BF16 weight or a ReLU tips over in later steps.
+// A block holds the four tiles of 16 outputs of a layer, which share the G operand; the 17 blocks of a
+// slice run on one XCD (ids 8 apart), so that its 629 KB of operands reach one L2. Bound by the latency of
+// those loads (16,384 rows: 5.1 us; 10.7 with a slice's tiles on all XCDs; 12.1 in 160 waves that took all
+// 16 tiles of a layer through their chunks one load after the other).
+// sums[tile][slice][lane]: lane 16 a + i holds outputs 4 a .. 4 a + 3 of input i.
+constexpr uint32_t kWeightTiles = 68;  // 4 layers of 4 x 4, and 4 of the output layer
+__global__ __launch_bounds__(kNrcBlock) __attribute__((amdgpu_waves_per_eu(1, 3)))
+void k_nrc_weight_sums(const bf16x8* __restrict__ acts, uint32_t n_slices, f32x4* __restrict__ sums, uint32_t n_rows,
+                       const uint32_t* __restrict__ n_rows_dev) {
+    if (n_rows_dev && min(n_rows, *n_rows_dev) == 0u) return;
+    const int lane = threadIdx.x & 63;
+    const uint32_t r = blockIdx.x >> 3, s = r / 17u * 8u + (blockIdx.x & 7u), L = r % 17u >> 2, ot = r % 17u & 3u;
+    if (s >= n_slices) return;
+    const uint32_t it = threadIdx.x >> 6, tile = L * 16u + ot * 4u + it;  // L = 4, ot = 0: the output layer
+    const bf16x8* base = acts + (size_t)s * kOperands * kSliceOperand + lane;
+    const bf16x8* ga = base + (20u + L * 4u + ot) * kSliceOperand;
+    const bf16x8* xa = base + (L * 4u + it) * kSliceOperand;
+    bf16x8 a[kSlice / 32], x[kSlice / 32];
+#pragma unroll
+    for (uint32_t k = 0; k < kSlice / 32; ++k) {
+        a[k] = ga[k * 64u];
+        x[k] = xa[k * 64u];
+    }
+    f32x4 acc{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (uint32_t k = 0; k < kSlice / 32; ++k) acc = mfma(a[k], x[k], acc);
+    sums[((size_t)tile * n_slices + s) * 64 + lane] = acc;
+}
+
+// The sum of the slices in order, Adam, and the packed BF16 copies for the next batch: a block per
+// weight tile (thread 64 a + 4 i + v: output 4 a + v, input i), and one that adds up the loss. Bound by
+// latency: the loads of up to 32 slices are in flight together (16,384 rows: 9.8 us with one load and add
+// after the other, now 3.6).
+constexpr uint32_t kBiasSteps = 2048;  // from here on 1 - beta^t is 1 in FP32
+__global__ __launch_bounds__(kNrcBlock) void k_nrc_adam(const f32x4* __restrict__ sums, uint32_t n_slices,
+                                                        const float* __restrict__ losses, uint32_t n_losses, float inv_b,
+                                                        float* __restrict__ w, float* __restrict__ m,
+                                                        float* __restrict__ v, float lr, float b1, float b2, float eps,
+                                                        const float2* __restrict__ bias, uint32_t n_rows,
+                                                        const uint32_t* __restrict__ n_rows_dev, TrainState* state,
+                                                        uint32_t add_taken, float* loss, __bf16* __restrict__ pf,
+                                                        __bf16* __restrict__ pb) {
+    const uint32_t tile = blockIdx.x;
+    if (n_rows_dev && min(n_rows, *n_rows_dev) == 0u) return;
+    if (tile == kWeightTiles) {
+        const uint32_t lane = threadIdx.x;
+        if (lane >= 64u) return;
+        float sum = 0.0f;
+        for (uint32_t k = lane; k < n_losses; k += 64) sum += losses[k];
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+        if (lane == 0) {
+            if (loss) *loss += sum;
+            state->taken += add_taken;  // after the call's last batch: no launch in flight reads it
+        }
+        return;
+    }
+    const uint32_t a = threadIdx.x >> 6, i = (threadIdx.x >> 2) & 15u, k4 = threadIdx.x & 3u;
+    const uint32_t o = (tile < 64u ? (tile >> 2) & 3u : 0u) * 16u + a * 4u + k4;
+    if (tile >= 64u && o >= 3u) return;
+    const uint32_t p = (tile >> 4) * 4096u + o * 64u + (tile & 3u) * 16u + i;
+    const float* mine = reinterpret_cast<const float*>(sums + (size_t)tile * n_slices * 64 + a * 16u + i) + k4;
+    const float m0 = m[p], v0 = v[p], w0 = w[p];
+    const float2 bc = bias[min(state->step, kBiasSteps - 1u)];
     float gsum = 0.0f;
-    for (uint32_t s = 0; s < n_slices; ++s) gsum += partial[(size_t)s * kNrcParams + p];
+    for (uint32_t s = 0; s < n_slices; s += 32) {
+        float q[32];
+#pragma unroll
+        for (uint32_t k = 0; k < 32; ++k) q[k] = mine[(size_t)min(s + k, n_slices - 1u) * 256];
+#pragma unroll
+        for (uint32_t k = 0; k < 32; ++k)
+            if (s + k < n_slices) gsum += q[k];
+    }
     const float gr = gsum * inv_b;
-    const float mm = b1 * m[p] + (1.0f - b1) * gr;
-    const float vv = b2 * v[p] + (1.0f - b2) * gr * gr;
+    const float mm = b1 * m0 + (1.0f - b1) * gr;
+    const float vv = b2 * v0 + (1.0f - b2) * gr * gr;
     m[p] = mm;
     v[p] = vv;
-    const float wn = w[p] - lr * (mm / bc1) / (sqrtf(vv / bc2) + eps);
+    const float wn = w0 - lr * (mm / bc.x) / (sqrtf(vv / bc.y) + eps);
     w[p] = wn;
     pack_weight(p, wn, pf, pb);
 }
@@ -456,7 +549,7 @@ int nrc_set_weights(cupbr_nrc* c, const float* host) {
     CUPBR_HIP_CHECK(hipMemcpy(c->w.ptr, host, kNrcParams * 4, hipMemcpyHostToDevice));
     CUPBR_HIP_CHECK(hipMemset(c->m.ptr, 0, kNrcParams * 4));
     CUPBR_HIP_CHECK(hipMemset(c->v.ptr, 0, kNrcParams * 4));
-    c->step = 0;
+    CUPBR_HIP_CHECK(hipMemset(c->state.ptr, 0, sizeof(TrainState)));
     return nrc_pack(c, nullptr);
 }
 
@@ -476,7 +569,8 @@ int nrc_create(const float lo[3], const float hi[3], uint32_t seed, cupbr_nrc** 
     }
     int rc;
     if ((rc = c->w.ensure(kNrcParams * 4)) || (rc = c->m.ensure(kNrcParams * 4)) || (rc = c->v.ensure(kNrcParams * 4)) ||
-        (rc = c->packed_fwd.ensure(kFwdSize * 2)) || (rc = c->packed_bwd.ensure(kBwdSize * 2))) {
+        (rc = c->packed_fwd.ensure(kFwdSize * 2)) || (rc = c->packed_bwd.ensure(kBwdSize * 2)) ||
+        (rc = c->state.ensure(sizeof(TrainState))) || (rc = c->bias.ensure(kBiasSteps * sizeof(float2)))) {
         delete c;
         return rc;
     }
@@ -485,6 +579,14 @@ int nrc_create(const float lo[3], const float hi[3], uint32_t seed, cupbr_nrc** 
         hipMemset(c->packed_bwd.ptr, 0, kBwdSize * 2) != hipSuccess) {
         delete c;
         return set_error(CUPBR_ERR_HIP, "hipMemset failed");
+    }
+    // Adam's bias corrections, one pair per step number
+    std::vector<float2> bias(kBiasSteps);
+    for (uint32_t k = 0; k < kBiasSteps; ++k)
+        bias[k] = make_float2(1.0f - std::pow(c->beta1, (float)k), 1.0f - std::pow(c->beta2, (float)k));
+    if (hipMemcpy(c->bias.ptr, bias.data(), kBiasSteps * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess) {
+        delete c;
+        return set_error(CUPBR_ERR_HIP, "hipMemcpy failed");
     }
     if ((rc = nrc_init_weights(c, seed))) {
         delete c;
@@ -510,47 +612,31 @@ int nrc_infer(cupbr_nrc* c, const float* rec, uint32_t n, const uint32_t* n_dev,
     return CUPBR_OK;
 }
 
-__global__ void k_nrc_zero(uint4* __restrict__ p, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        p[i] = make_uint4(0u, 0u, 0u, 0u);
-}
-
 int nrc_train(cupbr_nrc* c, const float* rows, uint32_t n_rows, uint32_t batch, uint32_t steps, float lr,
-              float* loss_dev, hipStream_t stream) {
+              float* loss_dev, hipStream_t stream, const uint32_t* n_rows_dev) {
     if (n_rows == 0 || steps == 0) return CUPBR_OK;
-    const uint32_t slice = 512;
-    const uint32_t n_slices = batch / slice;
+    // a block per 64 rows, in groups of 8 slices, at most about one per CU (its 149 KB of LDS allow no second one)
+    const uint32_t n_slices = batch / kSlice, groups = (n_slices + 7) / 8;
+    const uint32_t blocks = 64 * std::min<uint32_t>(groups, std::max(1u, (uint32_t)device_cu_count() / 64));
     int rc;
-    if ((rc = c->acts.ensure((size_t)2 * 5 * 64 * batch * 2)) ||
-        (rc = c->partial.ensure((size_t)n_slices * kNrcParams * 4)))
+    if ((rc = c->acts.ensure((size_t)n_slices * kOperands * kSliceOperand * 16)) || (rc = c->losses.ensure((size_t)blocks * 4)) ||
+        (rc = c->sums.ensure((size_t)kWeightTiles * (batch / kSlice) * 1024)))
         return rc;
-    __bf16* X = c->acts.as<__bf16>();
-    __bf16* G = X + (size_t)5 * 64 * batch;
-    // rows 3..63 of the output-layer gradient are never written: clear them once per size (by a
-    // kernel rather than a memset, so that a caller may capture the call in a graph)
-    if (c->acts_cleared_for != batch) {
-        const size_t n4 = (size_t)2 * 5 * 64 * batch * 2 / 16;
-        hipLaunchKernelGGL(k_nrc_zero, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096)), dim3(256), 0, stream,
-                           c->acts.as<uint4>(), n4);
-        CUPBR_HIP_CHECK(hipGetLastError());
-        c->acts_cleared_for = batch;
-    }
-    const int blocks = (int)std::max<uint32_t>(1, std::min<uint32_t>(batch / 64, (uint32_t)device_cu_count() * 2));
+    const uint32_t sum_blocks = groups * 8 * (kWeightTiles / 4);
+    TrainState* state = c->state.as<TrainState>();
     for (uint32_t s = 0; s < steps; ++s) {
-        ++c->step;
-        const uint32_t seed = c->step * 0x9E3779B9u + 0x51ED270Bu;
-        hipLaunchKernelGGL(k_nrc_forward_backward, dim3(blocks), dim3(kNrcBlock), 0, stream, c->packed_fwd.as<bf16x8>(),
-                           c->packed_bwd.as<bf16x8>(), c->box, rows, n_rows, batch, seed, X, G,
-                           loss_dev ? loss_dev + s : nullptr);
+        hipLaunchKernelGGL(k_nrc_train, dim3(blocks), dim3(kNrcBlock), 0, stream, c->packed_fwd.as<bf16x8>(),
+                           c->packed_bwd.as<bf16x8>(), c->box, rows, n_rows, n_rows_dev, batch, state, s,
+                           c->acts.as<bf16x8>(), c->losses.as<float>());
         CUPBR_HIP_CHECK(hipGetLastError());
-        hipLaunchKernelGGL(k_nrc_weight_grad, dim3(n_slices, 5), dim3(64), 0, stream, X, G, batch, slice,
-                           c->partial.as<float>());
+        hipLaunchKernelGGL(k_nrc_weight_sums, dim3(sum_blocks), dim3(kNrcBlock), 0, stream, c->acts.as<bf16x8>(), n_slices,
+                           c->sums.as<f32x4>(), n_rows, n_rows_dev);
         CUPBR_HIP_CHECK(hipGetLastError());
-        const float b1 = c->beta1, b2 = c->beta2;
-        const float bc1 = 1.0f - std::pow(b1, (float)c->step), bc2 = 1.0f - std::pow(b2, (float)c->step);
-        hipLaunchKernelGGL(k_nrc_adam, dim3((kNrcParams + 255) / 256), dim3(256), 0, stream, c->partial.as<float>(),
-                           n_slices, 1.0f / (float)batch, c->w.as<float>(), c->m.as<float>(), c->v.as<float>(), lr, b1,
-                           b2, c->eps, bc1, bc2, c->packed_fwd.as<__bf16>(), c->packed_bwd.as<__bf16>());
+        hipLaunchKernelGGL(k_nrc_adam, dim3(kWeightTiles + 1), dim3(kNrcBlock), 0, stream, c->sums.as<f32x4>(), n_slices,
+                           c->losses.as<float>(), blocks, 1.0f / (float)batch, c->w.as<float>(), c->m.as<float>(),
+                           c->v.as<float>(), lr, c->beta1, c->beta2, c->eps, c->bias.as<float2>(), n_rows, n_rows_dev,
+                           state, s + 1 == steps ? steps : 0u, loss_dev ? loss_dev + s : nullptr,
+                           c->packed_fwd.as<__bf16>(), c->packed_bwd.as<__bf16>());
         CUPBR_HIP_CHECK(hipGetLastError());
     }
     return CUPBR_OK;
