@@ -497,7 +497,6 @@ int cupbr_render(cupbr_renderer* r, const cupbr_camera* cam, uint32_t spp) {
     if (int rc = scene_upload(r->scene)) return rc;
     if (cam->moved) r->frame_index = 0;  // :174-177
     r->stats = cupbr_render_stats{};
-    r->nrc_queries_total = r->nrc_rows_total = 0;
     r->timer.used = 0;
     CUPBR_HIP_CHECK(hipEventRecord(r->ev_start, r->stream));
     int rc = CUPBR_OK;
@@ -528,9 +527,9 @@ int cupbr_renderer_get_stats(const cupbr_renderer* cr, cupbr_render_stats* out) 
     CUPBR_HIP_CHECK(hipStreamSynchronize(r->stream));
     float ms = 0.0f;
     if (hipEventElapsedTime(&ms, r->ev_start, r->ev_stop) == hipSuccess) r->stats.milliseconds = ms;
+    Counters c{};
+    if (r->wf.counters.ptr) CUPBR_HIP_CHECK(hipMemcpy(&c, r->wf.counters.ptr, sizeof c, hipMemcpyDeviceToHost));
     if (r->wf.counters.ptr && (r->method == CUPBR_PATHTRACER || r->method == CUPBR_VOLUME || r->method == CUPBR_GRADIENTDOMAIN)) {
-        Counters c;
-        CUPBR_HIP_CHECK(hipMemcpy(&c, r->wf.counters.ptr, sizeof c, hipMemcpyDeviceToHost));
         r->stats.extension_rays = c.extension_rays;
         r->stats.shadow_rays = c.shadow_rays;
         r->stats.extension_node_visits = c.ext_nodes;
@@ -539,8 +538,8 @@ int cupbr_renderer_get_stats(const cupbr_renderer* cr, cupbr_render_stats* out) 
         r->stats.shadow_prim_tests = c.shadow_prims;
         r->stats.refill_launches = c.refill_launches;
     }
-    r->stats.cache_queries = r->nrc_queries_total;
-    r->stats.cache_training_rows = r->nrc_rows_total;
+    r->stats.cache_queries = c.cache_queries;
+    r->stats.cache_training_rows = c.cache_rows;
     for (int k = 0; k < 4; ++k) { r->stats.stage_ms[k] = 0.0; r->stats.stage_launches[k] = 0; }
     for (size_t i = 1; i < r->timer.used; ++i) {
         const int st = r->timer.stage[i];

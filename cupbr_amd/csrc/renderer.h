@@ -33,6 +33,7 @@ struct Counters {
     unsigned long long shadow_rays;
     unsigned long long ext_nodes, ext_prims, shadow_nodes, shadow_prims;  // traversal counting
     unsigned long long refill_launches;  // trace launches that handed rays to idle lanes
+    unsigned long long cache_queries, cache_rows;  // radiance-cache queries and training rows of the call
 };
 
 // HIP events recorded between consecutive launches on the renderer's stream;
@@ -109,7 +110,6 @@ struct cupbr_renderer {
     // second stream for cache inference that overlaps the training paths' later bounces
     hipStream_t side_stream = nullptr;
     hipEvent_t ev_queries = nullptr, ev_side_done = nullptr;
-    uint64_t nrc_queries_total = 0, nrc_rows_total = 0;  // of the last cupbr_render call
 };
 
 namespace cupbr {
