@@ -10,8 +10,8 @@
 //   final trace the last bounce's shadow rays
 //   accumulate  the reference running mean, frame by frame             (:162-168)
 // Queue lengths live on the device, so no host round trip happens between bounces.
-// trace is a persistent grid whose waves take 64-ray chunks from 8 work counters, one
-// per XCD group (traversal cost varies per ray; one launch per bounce keeps the GPU full
+// trace is a persistent grid whose waves take pieces of their XCD's rays from its work counter
+// (traversal cost varies per ray; one launch per bounce keeps the GPU full
 // where the shadow queue alone is short); shade walks its queue with a static grid stride and
 // appends to the next queues with one atomic per 256-entry block (ballot + LDS prefix).
 // Extension and shadow queues alternate by bounce parity.
@@ -37,6 +37,13 @@
 #ifndef CUPBR_REFILL_IDLE
 #define CUPBR_REFILL_IDLE 32
 #endif
+// Rays per lane of the persistent grid from which a trace launch refills its lanes; below, every wave
+// traces one 64-ray chunk, whose end waits for one tail, not for two (extension rays, then shadow
+// rays). 1080p / 1M triangles at 1 spp with 1, 2 and 4 rays: 4.00, 4.09 and 4.27 ms (the volume renderer,
+// 512x512, 16 spp: 2.63, 2.62, 2.58).
+#ifndef CUPBR_REFILL_MIN
+#define CUPBR_REFILL_MIN 1u
+#endif
 
 namespace cupbr {
 
@@ -45,13 +52,8 @@ constexpr int kPtWaves = kPtBlock / 64;
 // traversal stack entries per lane kept in LDS (16 KB per 256-thread block: the trace kernel's 61
 // VGPRs, not LDS, then bound its occupancy at 8 waves per SIMD; deeper entries spill to memory)
 constexpr int kPtLds = 16;
-
-// one wave-uniform ticket per call
-__device__ __forceinline__ uint32_t wave_fetch(uint32_t* counter) {
-    uint32_t base = 0;
-    if (__lane_id() == 0) base = atomicAdd(counter, 1u);
-    return __shfl(base, 0);
-}
+// consecutive rays of a trace queue that belong to one XCD
+constexpr uint32_t kGranule = 1024;
 
 // Block-wide append: every thread of the block calls it; lanes with `want` get consecutive
 // slots of the queue whose length is *count (one atomic per block).
@@ -383,33 +385,74 @@ __device__ __forceinline__ void shadow_result(bool occluded, const float4 d4, co
     rad[p] = make_float4(L.x, L.y, L.z, R.w);
 }
 
-// One queue of the trace kernel, n rays, with per-lane refill: the queue is split into 8
-// contiguous groups, group h's rays handed out by counter[h]. A wave starts on group g0 (its
-// block's XCD), moves to the next group once its counter has passed the group's end, and gives
-// fresh rays to its idle lanes whenever at least CUPBR_REFILL_IDLE (32) of them are idle (or all are), so that a
-// lane whose ray ended does not wait for the slowest ray of a 64-ray chunk. finish(i, hit, r)
+// A wave's share of one queue of n rays. The queue is cut into granules of kGranule rays, granule k
+// belonging to XCD k % 8 (the blocks b with b % 8 = k % 8), so that the XCDs have equal work without
+// taking rays from each other. An XCD's rays, numbered through its granules, go to its waves in
+// pieces: a wave's first piece is dealt by its index, the next ones come from the XCD's counter.
+// What bounds the handing out is the counters: one 128-byte line serves an add with a return value
+// every 13 ns when only its own XCD uses it, and other XCDs' reads in between hold every add up. With
+// one add per refill of some 40 rays, the 20 M rays of a Cornell box bounce were 0.85 ms of counting
+// in a launch of 1.76 ms; with waves that tried all 8 counters before they ended, a launch took at
+// least 115 us however few rays it had, and one that refilled some 300 us. Hence the XCD's own counter
+// only, and pieces of 64 to 256 rays: as many as leave each of the XCD's waves two more, so that they
+// shrink towards the end. Gradient domain (Cornell box, 512x512, 16 spp) 9.5 -> 7.4 ms, volume
+// renderer (512x512, 16 spp) 3.85 -> 2.63 ms, 1080p / 1M triangles / 64 spp 113.5 -> 109.8 ms. Granules
+// of 256, 4096, 16384 and 65536 rays: 110.0, 109.6, 109.9, 110.6 ms; pieces of up to 64, 512 and 1024
+// rays 3% slower, the same, the same.
+struct RayShare {
+    CounterLine* counter;    // the XCD's
+    uint32_t g, waves;       // the XCD and its number of waves
+    uint32_t len, dealt;     // its rays, and those of the first pieces
+    uint32_t at, end;        // the wave's piece
+    __device__ __forceinline__ uint32_t piece(uint32_t left) const {
+        return min(max(left / (2u * waves) & ~63u, 64u), 256u);
+    }
+    __device__ __forceinline__ void begin(CounterLine* c, uint32_t n) {
+        g = blockIdx.x & 7u;
+        counter = c + g;
+        waves = (gridDim.x >> 3) * kPtWaves;
+        const uint32_t rest = n % (8u * kGranule), mine = rest - min(rest, g * kGranule);
+        len = n / (8u * kGranule) * kGranule + min(mine, kGranule);
+        const uint32_t size = piece(len);
+        dealt = min(size * waves, len);
+        at = __builtin_amdgcn_readfirstlane(min(((blockIdx.x >> 3) * kPtWaves + (threadIdx.x >> 6)) * size, len));
+        end = min(at + size, len);
+    }
+    // a new piece; false when there is none (wave-uniform: the whole wave calls it)
+    __device__ __forceinline__ bool refill() {
+        if (dealt == len) return false;
+        const uint32_t size = piece(len - end);
+        uint32_t base = 0;
+        if (__lane_id() == 0u) base = atomicAdd(&counter->v, size);
+        at = __builtin_amdgcn_readfirstlane(base) + dealt;
+        end = min(at + size, len);
+        return at < len;
+    }
+    // the queue index of the XCD's ray r < len
+    __device__ __forceinline__ uint32_t index(uint32_t r) const { return (r / kGranule * 8u + g) * kGranule + r % kGranule; }
+};
+
+// One queue of the trace kernel, n rays, with per-lane refill: a wave gives fresh rays of its share
+// (RayShare) to its idle lanes whenever at least CUPBR_REFILL_IDLE (32) of them are idle (or all are), so
+// that a lane whose ray ended does not wait for the slowest ray of a 64-ray chunk. finish(i, hit, r)
 // consumes the result of ray i.
 template <bool kAny, class Load, class Finish>
-__device__ __forceinline__ void trace_queue(const DevScene& S, uint32_t n, uint32_t g0, CounterLine* counter,
+__device__ __forceinline__ void trace_queue(const DevScene& S, uint32_t n, CounterLine* counter,
                                             LaneStack<kPtLds>& st, Load load, Finish finish) {
     const uint32_t lane = __lane_id();
-    uint32_t k = 0, h = g0;
-    uint32_t r0 = h * n / 8u, rl = (h + 1u) * n / 8u - r0;
     bool active = false, pool = true, hit = false;
     uint32_t my = 0;
+    RayShare share;
+    share.begin(counter, n);
     RayState rs;
     for (;;) {
         const unsigned long long idle = __ballot(!active);
         if (pool && (__popcll(idle) >= CUPBR_REFILL_IDLE || idle == ~0ull)) {
-            const uint32_t need = (uint32_t)__popcll(idle);
-            const uint32_t leader = (uint32_t)__builtin_ctzll(idle);
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(&counter[h].v, need);
-            base = (uint32_t)__shfl((int)base, (int)leader);
+            if (share.at >= share.end) pool = share.refill();
             if (!active) {
-                const uint32_t idx = base + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                if (idx < rl) {  // ray r0 + idx < (h + 1) n / 8 <= n
-                    my = r0 + idx;
+                const uint32_t idx = share.at + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+                if (idx < share.end) {
+                    my = share.index(idx);
                     v3 o, d;
                     float dist;
                     load(my, o, d, dist);
@@ -417,14 +460,7 @@ __device__ __forceinline__ void trace_queue(const DevScene& S, uint32_t n, uint3
                     if (!active) finish(my, hit, rs.best);
                 }
             }
-            if (base + need >= rl) {  // group h has handed out all of its rays
-                if (++k == 8) pool = false;
-                else {
-                    h = (g0 + k) & 7u;
-                    r0 = h * n / 8u;
-                    rl = (h + 1u) * n / 8u - r0;
-                }
-            }
+            share.at = min(share.at + (uint32_t)__popcll(idle), share.end);
         }
         const unsigned long long am = __ballot(active);
         if (am == 0ull) {
@@ -452,8 +488,8 @@ __device__ __forceinline__ void trace_queue(const DevScene& S, uint32_t n, uint3
 }
 
 // One bounce's extension rays (queue cur), then the previous bounce's shadow rays (parity cur ^ 1),
-// each queue handed out by 8 group counters (trace_queue; short launches and the visit-counting
-// instantiation hand out 64-ray chunks instead, one ray per lane until the chunk is done).
+// each queue handed out by one counter per XCD (trace_queue; short launches and the visit-counting
+// instantiation deal out 64-ray chunks instead, one ray per lane until the chunk is done).
 // amdgpu_waves_per_eu(8, 8): the compiler keeps the kernel within the SGPR budget of 8 waves per
 // SIMD (spilling a few SGPRs into VGPR lanes); without it 104 SGPRs held the kernel to 6 resident
 // waves per SIMD and a quarter of the persistent blocks only started when the queue was empty.
@@ -476,21 +512,15 @@ void k_pt_trace(DevScene S, int cur, const float4* __restrict__ q_o, const float
     }
     LaneStack<kPtLds> st{lds + threadIdx.x, kPtBlock, spill ? spill + gtid : nullptr, spill_stride};
     TravCount te, ts;
-    // Each queue is split into 8 groups: group h owns its h-th eighth. Workgroups are dispatched
-    // to the 8 XCDs round-robin, so the waves of block b start on group b % 8: each XCD traces
-    // neighbouring queue entries (neighbouring pixels and hit points) and its own L2 holds the
-    // nodes they share. A group that runs dry takes rays from the next groups in turn; every ray
-    // is handed out once, whatever XCD a block runs on.
+    // Workgroups are dispatched to the 8 XCDs round-robin: block b runs on XCD b % 8 (only the speed
+    // depends on it)
     const uint32_t g0 = blockIdx.x & 7u;
-    // Refill pays off once every lane of the persistent grid has several rays to trace; a short
-    // launch (deep bounces, one-frame calls) ends sooner with the one tail of 64-ray chunks than
-    // with the two tails of the refill (extension rays, then shadow rays). The decision is the
-    // same for every wave (n_ext and n_sh are read at the start).
-    const bool refill = !kCount && n_ext + n_sh >= 4u * gridDim.x * kPtBlock;
+    // the same decision for every wave (n_ext and n_sh are read at the start)
+    const bool refill = !kCount && n_ext + n_sh >= CUPBR_REFILL_MIN * gridDim.x * kPtBlock;
     if (refill && gtid == 0) c->refill_launches += 1;
     if (refill) {
         trace_queue<false>(
-            S, n_ext, g0, c->work, st,
+            S, n_ext, c->work, st,
             [&](uint32_t i, v3& o, v3& d, float& dist) {
                 const float4 o4 = q_o[i], d4 = q_d[i];
                 o = mk(o4.x, o4.y, o4.z);
@@ -499,7 +529,7 @@ void k_pt_trace(DevScene S, int cur, const float4* __restrict__ q_o, const float
             },
             [&](uint32_t i, bool, const TraceResult& r) { q_hit[i] = make_float2(r.t, __uint_as_float(r.prim)); });
         trace_queue<true>(
-            S, n_sh, g0, c->swork, st,
+            S, n_sh, c->swork, st,
             [&](uint32_t j, v3& o, v3& d, float& dist) {
                 const float4 o4 = s_o[j], d4 = s_d[j];
                 o = mk(o4.x, o4.y, o4.z);
@@ -508,34 +538,31 @@ void k_pt_trace(DevScene S, int cur, const float4* __restrict__ q_o, const float
             },
             [&](uint32_t j, bool occluded, const TraceResult&) { shadow_result(occluded, s_d[j], s_c, j, rad); });
     } else {
-        // 64-ray chunks, one ray per lane until the chunk is done (and the visit-counting pass):
-        // group h's counter hands out its extension chunks, then its shadow chunks
-        const uint32_t e_chunks = (n_ext + 63u) >> 6, s_chunks = (n_sh + 63u) >> 6;
-        for (uint32_t k = 0; k < 8; ++k) {
-            const uint32_t h = (g0 + k) & 7u;
-            const uint32_t e0 = h * e_chunks / 8u, e_len = (h + 1u) * e_chunks / 8u - e0;
-            const uint32_t s0 = h * s_chunks / 8u, s_len = (h + 1u) * s_chunks / 8u - s0;
-            for (;;) {
-                const uint32_t q = wave_fetch(&c->work[h].v);
-                if (q >= e_len + s_len) break;
-                if (q < e_len) {
-                    const uint32_t i = ((e0 + q) << 6) + __lane_id();
-                    if (i < n_ext) {
-                        const float4 o4 = q_o[i], d4 = q_d[i];
-                        TraceResult r;
-                        traverse<false, kPtLds, kCount>(S, mk(o4.x, o4.y, o4.z), mk(d4.x, d4.y, d4.z), 0.0f, st, r,
-                                                        &te);
-                        q_hit[i] = make_float2(r.t, __uint_as_float(r.prim));
-                    }
-                } else {
-                    const uint32_t j = ((s0 + q - e_len) << 6) + __lane_id();
-                    if (j < n_sh) {
-                        const float4 o4 = s_o[j], d4 = s_d[j];
-                        TraceResult r;
-                        const bool occluded = traverse<true, kPtLds, kCount>(S, mk(o4.x, o4.y, o4.z),
-                                                                              mk(d4.x, d4.y, d4.z), o4.w, st, r, &ts);
-                        shadow_result(occluded, d4, s_c, j, rad);
-                    }
+        // 64-ray chunks, one ray per lane until the chunk is done (and the visit-counting pass). The
+        // chunks, extension then shadow, are dealt out by wave: XCD x (blocks b % 8 = x) takes the
+        // x-th eighth of them, its waves one after the other. No counters: a wave has one chunk (in the
+        // visit-counting pass as many as it takes). Cornell box, 256x256, 1 spp: 730 -> 238 us a frame.
+        // Chunks of 32, 16 or 8 rays on more waves gave 247, 249 and 256 us.
+        const uint32_t e_chunks = (n_ext + 63u) >> 6, chunks = e_chunks + ((n_sh + 63u) >> 6);
+        const uint32_t first = g0 * chunks / 8u, last = (g0 + 1u) * chunks / 8u;
+        const uint32_t waves = (gridDim.x >> 3) * kPtWaves;  // per XCD; gridDim.x is a multiple of 8
+        for (uint32_t q = first + (blockIdx.x >> 3) * kPtWaves + (threadIdx.x >> 6); q < last; q += waves) {
+            if (q < e_chunks) {
+                const uint32_t i = (q << 6) + __lane_id();
+                if (i < n_ext) {
+                    const float4 o4 = q_o[i], d4 = q_d[i];
+                    TraceResult r;
+                    traverse<false, kPtLds, kCount>(S, mk(o4.x, o4.y, o4.z), mk(d4.x, d4.y, d4.z), 0.0f, st, r, &te);
+                    q_hit[i] = make_float2(r.t, __uint_as_float(r.prim));
+                }
+            } else {
+                const uint32_t j = ((q - e_chunks) << 6) + __lane_id();
+                if (j < n_sh) {
+                    const float4 o4 = s_o[j], d4 = s_d[j];
+                    TraceResult r;
+                    const bool occluded = traverse<true, kPtLds, kCount>(S, mk(o4.x, o4.y, o4.z),
+                                                                          mk(d4.x, d4.y, d4.z), o4.w, st, r, &ts);
+                    shadow_result(occluded, d4, s_c, j, rad);
                 }
             }
         }

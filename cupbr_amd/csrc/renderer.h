@@ -14,7 +14,7 @@ constexpr int kNumImages = 8;  // cupbr_image
 
 // Device counters of one render call, one 128-byte line each so that atomics on
 // different counters never serialise on the same L2 line. The trace kernel's work
-// counters hand out 64-ray chunks to persistent waves; each counter is reset by
+// counters hand out pieces of an XCD's rays to its persistent waves; each counter is reset by
 // the kernel that runs after its last user.
 struct alignas(128) CounterLine {
     uint32_t v;
@@ -23,8 +23,8 @@ struct alignas(128) CounterLine {
 struct Counters {
     CounterLine queue_count[2];  // extension queues (ping-pong by bounce parity)
     CounterLine shadow_count[2]; // shadow queues (bounce parity)
-    CounterLine work[8];         // trace kernel: extension rays handed out, per XCD group
-    CounterLine swork[8];        // trace kernel: shadow rays handed out, per XCD group
+    CounterLine work[8];         // trace kernel: extension rays handed out beyond the dealt pieces, per XCD
+    CounterLine swork[8];        // trace kernel: shadow rays handed out beyond the dealt pieces, per XCD
     CounterLine query_count;  // radiance-cache queries of the batch
     CounterLine query_early;  // queries that existed after the second bounce's shade
     CounterLine row_count;    // radiance-cache training rows of the batch
