@@ -20,10 +20,9 @@ from . import Camera, CupbrError, GridMedium, GridRenderer, Scene
 class _GridRenderFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, density, albedo, renderer: GridRenderer, proposal):
-        prop = proposal if proposal is not None else density.detach().clone()
-        image = renderer.render(density, albedo, proposal=prop)
+        image = renderer.render(density, albedo, proposal=proposal)  # None: the density itself
         ctx.renderer = renderer
-        ctx.save_for_backward(density, albedo, prop)
+        ctx.save_for_backward(density, albedo, proposal)
         return image
 
     @staticmethod

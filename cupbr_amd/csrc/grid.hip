@@ -45,7 +45,7 @@
 namespace cupbr {
 
 constexpr int kGridBlock = 256;
-constexpr int kGridLds = 32;
+constexpr int kGridLds = 24;  // 3 blocks of the adjoint per CU (46 KB each; at 32 entries only 2 fit: 19.7 against 17.7 ms)
 constexpr float kSurfaceOffset = 1e-4f;
 constexpr int kAlbLds = 3 * 1024;  // surfaces whose albedo gradients a block accumulates in LDS
 constexpr size_t kMaxGridSamples = (size_t)1 << 24;  // samples per forward chunk (192 MB buffer)
@@ -53,16 +53,24 @@ constexpr size_t kMaxGridSamples = (size_t)1 << 24;  // samples per forward chun
 // so the expected count per segment is below 1e5 and the bound is never reached in practice;
 // reaching it ends the path (or zeroes the shadow ray's transmittance), so every loop terminates.
 constexpr uint32_t kMaxTrackSteps = 1u << 22;
-// The adjoint's density-gradient atomics go to one private copy of the gradient per group of
-// blocks, block b -> copy b % kGradCopies. Workgroups are dispatched to the 8 XCDs round-robin,
-// so each copy is written by one XCD and its lines stay in that XCD's L2 instead of moving
-// between L2s on every atomic; a reduction adds the copies to the caller's gradient in copy
-// order. The mapping only affects speed: any assignment of blocks to copies sums the same terms.
-#ifndef CUPBR_GRID_GRAD_COPIES
-#define CUPBR_GRID_GRAD_COPIES 8
-#endif
-constexpr uint32_t kGradCopies = CUPBR_GRID_GRAD_COPIES;
-constexpr size_t kMaxGradCopyBytes = (size_t)1 << 30;  // larger grids scatter into the output directly
+// The adjoint's density-gradient adds. What bounds them is requests to L2: 21 G/s, each of up to 16
+// consecutive words of one instruction. A stencil's 8 voxels lie on four lines, and one lane adding to
+// them is 8 requests; so the adjoint adds into cells instead, (nx + 1)(ny + 1)(nz + 1) of 8 consecutive
+// words, one per corner, and 8 lanes add one stencil's 8 words together in one request (scatter_cell).
+// k_grid_fold and k_grid_gather then add the cells' corners to the caller's gradient.
+// There is one copy of the cells per group of blocks, block b -> copy b % copies. Workgroups are
+// dispatched to the 8 XCDs round-robin, so with 8 copies each is written by one XCD and its lines stay in
+// that XCD's L2 instead of moving between L2s on every atomic. The mapping only affects speed: any
+// assignment of blocks to copies sums the same terms.
+// 64^3 voxels, 256x256, 64 spp (101 M stencils a launch): 39.0 ms adding voxel by voxel to copies of the
+// gradient (20.5 G adds/s, the request rate), 11.8 ms in cells (68 G adds/s, 8.5 G requests: the
+// divergence of the paths bounds it now); clearing, folding and gathering the 140 MB take 35 us. 256^3, 512x512, 16 spp: 39.4 -> 19.2 ms.
+constexpr uint32_t kGradCopies = 8;
+constexpr size_t kMaxGradCopyBytes = (size_t)8 << 30;  // fewer copies above; grids of one such copy add to the output
+// Cells per path above which clearing and folding the cells (64 bytes each, per copy) cost more than the
+// requests they save: those add to the output too. 64^3 cells, 32 k paths (8 cells a path): 474 us in cells,
+// 485 voxel by voxel; 16 k paths (17): 487 and 473; 128^3 cells, 32 k paths (65): 801 and 511.
+constexpr size_t kCellsPerPath = 16;
 
 struct GridDev {
     const float* rho;   // density parameters
@@ -77,13 +85,15 @@ struct GridDev {
 struct Stencil {
     uint32_t idx[8];
     float w[8];
+    float f[3];     // position inside the cell
+    uint32_t cell;  // the cell between voxels lo and lo + 1 of each axis, lo from -1 to n - 1
 };
 
 // trilinear stencil of x: corner k = (dx, dy, dz) = (k & 1, (k >> 1) & 1, k >> 2)
 __device__ __forceinline__ void stencil(const GridDev& G, v3 x, Stencil& s) {
     const float p[3] = {x.x, x.y, x.z};
-    uint32_t i0[3], i1[3];
-    float f[3];
+    uint32_t i0[3], i1[3], c[3];
+    float* f = s.f;
     for (int a = 0; a < 3; ++a) {
         const float u = (p[a] - G.bmin[a]) / G.ext[a] * (float)G.n[a] - 0.5f;
         const float fl = floorf(u);
@@ -92,7 +102,9 @@ __device__ __forceinline__ void stencil(const GridDev& G, v3 x, Stencil& s) {
         const int hi_max = (int)G.n[a] - 1;
         i0[a] = (uint32_t)min(max(lo, 0), hi_max);
         i1[a] = (uint32_t)min(max(lo + 1, 0), hi_max);
+        c[a] = (uint32_t)min(max(lo + 1, 0), hi_max + 1);
     }
+    s.cell = (c[2] * (G.n[1] + 1u) + c[1]) * (G.n[0] + 1u) + c[0];
     for (int k = 0; k < 8; ++k) {
         const int dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
         const uint32_t ix = dx ? i1[0] : i0[0], iy = dy ? i1[1] : i0[1], iz = dz ? i1[2] : i0[2];
@@ -107,15 +119,55 @@ __device__ __forceinline__ float sample_grid(const float* g, const Stencil& s) {
     return v;
 }
 
-__device__ __forceinline__ uint32_t scatter_grad(float* grad, const Stencil& s, float c) {
+// A wave's scratch for scatter_cell: one entry per lane that has a stencil to add.
+struct CellScratch {
+    float add[64][8];  // one value per corner
+    uint32_t cell[64];
+};
+
+// Where a path's density gradient goes: cells (scatter_cell) or, with none, the gradient itself.
+struct GradOut {
+    float* rho;    // the gradient, or a copy of the cells
+    CellScratch* cells;  // nullptr: rho is the gradient
+};
+
+// Adds c * w_k to corner k of the stencil's cell, for the lanes that call it together (any of a wave):
+// word j of the n calling lanes' 8 n words is corner j % 8 of the (j / 8)-th lane's stencil, and each
+// instruction adds n consecutive ones.
+__device__ __forceinline__ void scatter_cell(const GradOut& out, const Stencil& s, float c) {
+    const unsigned long long m = __ballot(true);
+    const uint32_t n = (uint32_t)__popcll(m), rank = (uint32_t)__popcll(m & ((1ull << __lane_id()) - 1ull));
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) out.cells->add[rank][k] = c * s.w[k];
+    out.cells->cell[rank] = s.cell;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const float* add = &out.cells->add[0][0];
+    float v[8];
+    uint32_t at[8];
+#pragma unroll
+    for (uint32_t q = 0; q < 8; ++q) {
+        const uint32_t j = q * n + rank;
+        v[q] = add[j];
+        at[q] = out.cells->cell[j >> 3];
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < 8; ++q) atomicAdd(out.rho + (size_t)at[q] * 8u + ((q * n + rank) & 7u), v[q]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // the next call's entries come after these reads
+}
+
+__device__ __forceinline__ uint32_t scatter_grad(const GradOut& out, const Stencil& s, float c) {
     if (c == 0.0f || !(fabsf(c) < __builtin_inff())) return 0;
-    uint32_t n = 0;
-    for (int k = 0; k < 8; ++k)
-        if (s.w[k] != 0.0f) {
-            atomicAdd(grad + s.idx[k], c * s.w[k]);
-            ++n;
-        }
-    return n;
+    if (out.cells) {
+        scatter_cell(out, s, c);
+    } else {
+        for (int k = 0; k < 8; ++k)
+            if (s.w[k] != 0.0f) atomicAdd(out.rho + s.idx[k], c * s.w[k]);
+    }
+    // voxels with a weight (1 - f is never 0)
+    return (s.f[0] != 0.0f ? 2u : 1u) * (s.f[1] != 0.0f ? 2u : 1u) * (s.f[2] != 0.0f ? 2u : 1u);
 }
 
 // parametric range [t0, t1] of o + t d inside the medium box, clipped to [0, tmax]
@@ -145,7 +197,7 @@ __device__ __forceinline__ bool clip_box(const GridDev& G, v3 o, v3 d, float tma
 struct Adj {
     v3 delta;     // dLoss/dI of the pixel, divided by spp
     v3 rem;       // radiance of the path not yet collected
-    float* grad_rho;
+    GradOut grad_rho;
     float* grad_alb;
 };
 
@@ -187,7 +239,7 @@ __device__ __forceinline__ float ratio_track(const GridDev& G, GridTracer& Tr, v
 
 // the same tentative points again, adding coef * dlog(1 - sigma/m)/dsigma * scale to the voxels
 __device__ __forceinline__ void ratio_track_grad(const GridDev& G, GridTracer& Tr, v3 o, v3 d, float dist,
-                                                 uint32_t seed, float coef, float* grad) {
+                                                 uint32_t seed, float coef, const GradOut& grad) {
     float t0, t1;
     if (!clip_box(G, o, d, dist, t0, t1)) return;
     const float len = t1 - t0;
@@ -249,8 +301,13 @@ __device__ v3 grid_path(const DevScene& S, const GridDev& G, GridTracer& T, cons
                 Stencil s;
                 stencil(G, x, s);
                 const float sigma = G.scale * sample_grid(G.rho, s);
-                const float P = clampf(G.scale * sample_grid(G.prop, s) / G.maj, G.eps, 1.0f - G.eps);
-                T.n_reads += 2;
+                float prop = sigma;  // the proposal's: read once when it is the density (17.7 -> 17.2 ms)
+                ++T.n_reads;
+                if (G.prop != G.rho) {
+                    prop = G.scale * sample_grid(G.prop, s);
+                    ++T.n_reads;
+                }
+                const float P = clampf(prop / G.maj, G.eps, 1.0f - G.eps);
                 float f, dlog;
                 const bool real = rnd(seed) < P;
                 if (real) {
@@ -347,13 +404,14 @@ __global__ __launch_bounds__(kGridBlock) void k_grid(DevScene S, GridDev G, cupb
                                                      uint32_t spp, uint32_t frame0, uint32_t s_begin, uint32_t s_count,
                                                      uint32_t max_depth, float* __restrict__ samples,
                                                      const float* __restrict__ d_image, float* grad_rho,
-                                                     float* grad_alb, uint32_t n_alb, size_t copy_stride,
+                                                     float* grad_alb, uint32_t n_alb, uint32_t copies, size_t copy_stride,
                                                      uint32_t* spill, unsigned long long* counts,
                                                      const float* __restrict__ fwd_samples) {
     __shared__ uint32_t lds[kGridLds * kGridBlock];
     // per-block albedo gradients (few surfaces, hit by every path): LDS atomics, one global
     // atomic per entry at the end
     __shared__ float alb_lds[kAlbLds];
+    __shared__ CellScratch cell_lds[kAdj ? kGridBlock / 64 : 1];
     const bool alb_local = kAdj && n_alb <= (uint32_t)kAlbLds;
     if (alb_local) {
         for (uint32_t k = threadIdx.x; k < n_alb; k += blockDim.x) alb_lds[k] = 0.0f;
@@ -361,8 +419,8 @@ __global__ __launch_bounds__(kGridBlock) void k_grid(DevScene S, GridDev G, cupb
     }
     const size_t gtid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
-    // private gradient copies (copy_stride floats apart; 0: scatter into grad_rho itself)
-    if (kAdj && copy_stride) grad_rho += (size_t)(blockIdx.x % kGradCopies) * copy_stride;
+    // copies of the cells, copy_stride floats apart (0: grad_rho is the gradient itself)
+    if (kAdj && copy_stride) grad_rho += (size_t)(blockIdx.x % copies) * copy_stride;
     LaneStack<kGridLds> st{lds + threadIdx.x, kGridBlock, spill ? spill + gtid : nullptr, (uint32_t)stride};
     GridTracer T{S, st};
     const uint32_t npix = w * h;
@@ -381,7 +439,7 @@ __global__ __launch_bounds__(kGridBlock) void k_grid(DevScene S, GridDev G, cupb
             Adj A;
             A.delta = ld3(d_image + 3 * (size_t)p) / (float)spp;
             A.rem = L;
-            A.grad_rho = grad_rho;
+            A.grad_rho = GradOut{grad_rho, copy_stride ? &cell_lds[threadIdx.x >> 6] : nullptr};
             A.grad_alb = alb_local ? alb_lds : grad_alb;
             if (A.delta.x != 0.0f || A.delta.y != 0.0f || A.delta.z != 0.0f)
                 grid_path<true>(S, G, T, cam, px, py, w, h, frame0 + s, max_depth, &A);
@@ -406,12 +464,45 @@ __global__ void k_grid_zero(float4* __restrict__ p, size_t n4) {
         p[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
-// grad[v] += sum over copies c (in order) of copies[c * stride + v], v < n_vox <= stride
-__global__ void k_grid_reduce(float* __restrict__ grad, const float* __restrict__ copies, size_t n_vox,
-                              size_t stride) {
+// copy 0 <- the sum of the copies, in copy order (n4 float4 per copy, stride4 apart)
+__global__ void k_grid_fold(float4* __restrict__ cells, size_t n4, size_t stride4, uint32_t copies) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) {
+        float4 sum = cells[i];
+        for (uint32_t c = 1; c < copies; ++c) {
+            const float4 v = cells[(size_t)c * stride4 + i];
+            sum.x += v.x;
+            sum.y += v.y;
+            sum.z += v.z;
+            sum.w += v.w;
+        }
+        cells[i] = sum;
+    }
+}
+
+// grad[v] += the cell corners that are voxel v. Along an axis of n voxels, voxel i is corner 1 of cell i
+// and corner 0 of cell i + 1, and at the faces (where the lookup clamps) also corner 0 of cell 0 (i = 0)
+// and corner 1 of cell n (i = n - 1).
+__global__ __launch_bounds__(256) void k_grid_gather(float* __restrict__ grad, const float* __restrict__ cells,
+                                                     uint32_t nx, uint32_t ny, uint32_t nz) {
+    const size_t n_vox = (size_t)nx * ny * nz;
     for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < n_vox; v += (size_t)gridDim.x * blockDim.x) {
+        const uint32_t i[3] = {(uint32_t)(v % nx), (uint32_t)(v / nx % ny), (uint32_t)(v / nx / ny)};
+        const uint32_t n[3] = {nx, ny, nz};
+        uint32_t cell[3][4], corner[3][4], count[3];
+        for (int a = 0; a < 3; ++a) {
+            cell[a][0] = i[a], corner[a][0] = 1u;
+            cell[a][1] = i[a] + 1u, corner[a][1] = 0u;
+            count[a] = 2;
+            if (i[a] == 0u) cell[a][count[a]] = 0u, corner[a][count[a]++] = 0u;
+            if (i[a] == n[a] - 1u) cell[a][count[a]] = n[a], corner[a][count[a]++] = 1u;
+        }
         float sum = 0.0f;
-        for (uint32_t c = 0; c < kGradCopies; ++c) sum += copies[(size_t)c * stride + v];
+        for (uint32_t z = 0; z < count[2]; ++z)
+            for (uint32_t y = 0; y < count[1]; ++y)
+                for (uint32_t x = 0; x < count[0]; ++x) {
+                    const size_t c = ((size_t)cell[2][z] * (ny + 1u) + cell[1][y]) * (nx + 1u) + cell[0][x];
+                    sum += cells[c * 8u + corner[2][z] * 4u + corner[1][y] * 2u + corner[0][x]];
+                }
         if (sum != 0.0f) grad[v] += sum;
     }
 }
@@ -523,7 +614,7 @@ int grid_render_device(const cupbr_scene* cs, const cupbr_camera* cam, const cup
         uint32_t* spill;
         if (grid_launch_shape(s, (size_t)n_px * cnt, &blocks, &spill)) return CUPBR_ERR_OUT_OF_MEMORY;
         hipLaunchKernelGGL(k_grid<false>, dim3(blocks), dim3(kGridBlock), 0, stream, s->dev, G, *cam, w, h, spp, frame0,
-                           s0, cnt, max_depth, s->grid_samples.as<float>(), nullptr, nullptr, nullptr, 0u, (size_t)0,
+                           s0, cnt, max_depth, s->grid_samples.as<float>(), nullptr, nullptr, nullptr, 0u, 1u, (size_t)0,
                            spill, counts, nullptr);
         CUPBR_HIP_CHECK(hipGetLastError());
         hipLaunchKernelGGL(k_grid_accumulate, dim3((n_px + 255) / 256), dim3(256), 0, stream, image,
@@ -573,27 +664,35 @@ int grid_adjoint_device(const cupbr_scene* cs, const cupbr_camera* cam, const cu
     uint32_t* spill;
     if (grid_launch_shape(s, (size_t)w * h * spp, &blocks, &spill)) return CUPBR_ERR_OUT_OF_MEMORY;
     if (int rc = scene_stream_acquire(s, stream)) return rc;
-    // private gradient copies (cleared by a kernel, not a memset, so that a captured graph replays it)
-    const size_t n_vox = (size_t)m->nx * m->ny * m->nz;
-    const size_t copy_floats = (n_vox + 3) & ~(size_t)3;  // 16-byte aligned copies
-    const bool private_copies = kGradCopies > 1 && copy_floats * kGradCopies * sizeof(float) <= kMaxGradCopyBytes;
+    // copies of the gradient's cells (cleared by a kernel, not a memset, so that a captured graph replays it)
+    const size_t n_cells = ((size_t)m->nx + 1) * (m->ny + 1) * (m->nz + 1), cell_floats = n_cells * 8;
+    uint32_t copies = kGradCopies;
+    while (copies > 0 && cell_floats * copies * sizeof(float) > kMaxGradCopyBytes) copies >>= 1;
+    bool in_cells = copies > 0 && (size_t)w * h * spp * kCellsPerPath >= n_cells;
+    if (in_cells && s->grid_grad.ensure(cell_floats * copies * sizeof(float))) {
+        (void)hipGetLastError();  // no memory for them
+        in_cells = false;
+    }
     float* target = grad_rho;
-    if (private_copies) {
-        if (s->grid_grad.ensure(copy_floats * kGradCopies * sizeof(float))) return CUPBR_ERR_OUT_OF_MEMORY;
+    if (in_cells) {
         target = s->grid_grad.as<float>();
-        const size_t n4 = copy_floats * kGradCopies / 4;
+        const size_t n4 = cell_floats * copies / 4;
         hipLaunchKernelGGL(k_grid_zero, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096)), dim3(256), 0, stream,
                            reinterpret_cast<float4*>(target), n4);
         CUPBR_HIP_CHECK(hipGetLastError());
     }
     hipLaunchKernelGGL(k_grid<true>, dim3(blocks), dim3(kGridBlock), 0, stream, s->dev, G, *cam, w, h, spp, frame0, 0u,
                        spp, max_depth, nullptr, d_image, target, grad_alb,
-                       (uint32_t)(3 * (s->objects.size() + s->triangles.size() / 9)),
-                       private_copies ? copy_floats : (size_t)0, spill, counts, fwd_samples);
+                       (uint32_t)(3 * (s->objects.size() + s->triangles.size() / 9)), copies,
+                       in_cells ? cell_floats : (size_t)0, spill, counts, fwd_samples);
     CUPBR_HIP_CHECK(hipGetLastError());
-    if (private_copies) {
-        hipLaunchKernelGGL(k_grid_reduce, dim3((unsigned)std::min<size_t>((n_vox + 255) / 256, 4096)), dim3(256), 0,
-                           stream, grad_rho, target, n_vox, copy_floats);
+    if (in_cells) {
+        const size_t n4 = cell_floats / 4, n_vox = (size_t)m->nx * m->ny * m->nz;
+        hipLaunchKernelGGL(k_grid_fold, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096)), dim3(256), 0, stream,
+                           reinterpret_cast<float4*>(target), n4, n4, copies);
+        CUPBR_HIP_CHECK(hipGetLastError());
+        hipLaunchKernelGGL(k_grid_gather, dim3((unsigned)std::min<size_t>((n_vox + 255) / 256, 8192)), dim3(256), 0,
+                           stream, grad_rho, target, m->nx, m->ny, m->nz);
         CUPBR_HIP_CHECK(hipGetLastError());
     }
     return scene_stream_release(s, stream);

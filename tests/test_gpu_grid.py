@@ -210,3 +210,31 @@ def test_grid_full_size_workload():
     gr3, ga3 = R.adjoint(rho, alb, -0.5 * d_img)
     torch.testing.assert_close(gr3, -0.5 * gr, rtol=1e-4, atol=1e-5 * float(gr.abs().max()))
     torch.testing.assert_close(ga3, -0.5 * ga, rtol=1e-4, atol=1e-5 * float(ga.abs().max()))
+
+
+@pytest.mark.parametrize("shape,size,spp", [
+    ((1, 1, 1), 24, 8),      # every lookup clamped on all axes
+    ((1, 5, 2), 24, 8),
+    ((3, 1, 7), 24, 8),
+    ((17, 9, 33), 24, 8),    # gradient in cells
+    ((64, 64, 64), 16, 4),   # few paths for the grid: added to the output directly
+    ((64, 64, 64), 48, 8),   # the same grid in cells
+])
+def test_grid_adjoint_shapes_against_fp64_oracle(shape, size, spp):
+    G = scenes.grid_medium_scene(res=64)
+    rho, tgt = (np.ascontiguousarray(G[k][:shape[0], :shape[1], :shape[2]]) + np.float32(0.05)
+                for k in ("density", "target_density"))
+    ca = G["camera"]
+    cam = cb.Camera.look_at(ca["eye"], ca["target"], ca["up"], ca["vfov"], size, size)
+    R = cb.GridRenderer(cb.Scene.from_desc(G["desc"]), cam, cb.GridMedium.from_dict(shape, G["medium"]), size, size,
+                        spp=spp, max_depth=6)
+    S = oracle.OracleScene(G["desc"])
+    args = (cam.as_dict(), G["medium"])
+    target = S.grid(*args, tgt, G["albedo"], size, size, spp=spp, depth=6)
+    d_img = (2 * (R.render(rho, G["albedo"]) - target)).astype(np.float32)
+    gr, ga = R.adjoint(rho, G["albedo"], d_img)
+    rr, ra = S.grid(*args, rho, G["albedo"], size, size, spp=spp, depth=6, d_image=d_img, precision=64)
+    assert gr.shape == rho.shape and np.isfinite(gr).all()
+    # the bars of the other oracle comparisons here
+    assert np.linalg.norm(gr - rr) <= 1e-3 * np.linalg.norm(rr)
+    assert np.linalg.norm(ga - ra) <= 1e-3 * np.linalg.norm(ra)
