@@ -82,7 +82,7 @@ int trace_visibility_device(const cupbr_scene* s, const float* rays, const float
                             hipStream_t stream);
 // the closest-hit kernel of trace_closest_device on a given grid of 256-lane blocks, with a spill
 // stack of (stack_entries - 32) words per lane at a stride of blocks * 256 (nullptr when
-// stack_entries <= 32)
+// stack_entries <= 32); small batches are traced by several lanes per ray, with neither
 constexpr int kTraceBlock = 256;
 constexpr int kTraceLds = 32;
 int trace_closest_launch(const cupbr_scene* s, const float* rays, size_t n, int32_t* obj, int32_t* tri, float* t,

@@ -381,6 +381,126 @@ __device__ __forceinline__ bool ray_step(const DevScene& S, RayState& r, LaneSta
     return true;
 }
 
+// One ray per group of kGroup lanes of a wave: each step takes the kGroup / 4 entries on top of the ray's
+// stack, four lanes to an entry, a lane testing one child of an inner node or every fourth primitive of a
+// leaf. What bounds a batch too small to fill the chip is the longest ray's chain of dependent steps, each
+// a round trip to memory; this shortens the chain by up to kGroup / 4 at the price of visits that the
+// sequential order would have culled. The tests are those of traverse, and the result, a minimum of
+// (t, rank) over all primitives of overlapping boxes (any-hit: whether there is one), is the same for any
+// order of visits.
+// stack: kGroup * (depth + 1) words of LDS of the group's own. The levels of the entries never decrease from
+// bottom to top, as children replace their parents in the parents' order. An entry of level d - 1 is taken
+// only together with all entries of levels d and more above it, fewer than kGroup / 4, so the entries of a
+// level that are on the stack at one time come from one step: at most kGroup of them, on depth levels.
+// Called by whole waves; a group with valid = false only takes part in the wave's votes.
+template <bool kAny, uint32_t kGroup>
+__device__ __forceinline__ bool traverse_group(const DevScene& S, v3 o, v3 d, float dist, bool valid, uint32_t* stack,
+                                               TraceResult& best) {
+    constexpr uint32_t kEntries = kGroup / 4;
+    constexpr int kCulled = 0x7FFFFFFF;
+    const uint32_t lane = __lane_id(), sub = lane % kGroup, entry = sub >> 2, c = sub & 3u;
+    const auto group_bits = [&](bool b) {  // the group's votes, lane sub in bit sub
+        return (__ballot(b) >> (lane - sub)) & (~0ull >> (64u - kGroup));
+    };
+    const auto reduce = [&](TraceResult& r) {  // the group's minimum of (t, rank), in every lane
+#pragma unroll
+        for (uint32_t off = 1; off < kGroup; off <<= 1) {
+            const float t = __shfl_xor(r.t, off);
+            const uint32_t prim = __shfl_xor(r.prim, off), rank = __shfl_xor(r.rank, off);
+            if (t < r.t || (t == r.t && rank < r.rank)) r = TraceResult{t, prim, rank};
+        }
+    };
+    best = TraceResult{__builtin_inff(), kNoHit, 0xFFFFFFFFu};
+    bool any = false;
+    if (valid)
+        for (uint32_t i = sub; i < S.n_unb; i += kGroup) {
+            const UnbRec u = S.unb[i];
+            float t;
+            if (!plane_quad_test(u, o, d, t)) continue;
+            const uint32_t rank = __float_as_uint(u.n.w);
+            any = any || t <= dist;
+            if (t < best.t || (t == best.t && rank < best.rank)) best = TraceResult{t, kUnbBit | i, rank};
+        }
+    if (kAny)
+        any = group_bits(any) != 0ull;
+    else if (S.n_unb)
+        reduce(best);
+    const float ix = 1.0f / d.x, iy = 1.0f / d.y, iz = 1.0f / d.z;
+    const float tlo = -1e-5f;
+    uint32_t sp = valid && !(kAny && any) && S.n_nodes ? 1u : 0u;
+    if (sub == 0u) stack[0] = 0u;
+    while (__ballot(sp != 0u)) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();  // the entries pushed by other lanes
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const bool mine = entry < sp;
+        const uint32_t word = mine ? stack[sp - 1u - entry] : kLeafBit;
+        sp -= min(sp, kEntries);
+        int key = kCulled;
+        uint32_t child = 0u;
+        TraceResult found = best;
+        bool hit = false;
+        if (!(word & kLeafBit)) {
+            const float lim = (kAny ? dist : best.t) * 1.0001f + 1e-6f;
+            const char* base = reinterpret_cast<const char*>(S.hnodes) + (size_t)word * 128u;
+            const float4 co = *reinterpret_cast<const float4*>(base);
+            const uint4 px = *reinterpret_cast<const uint4*>(base + (ix >= 0.0f ? 16u : 32u));
+            const uint4 py = *reinterpret_cast<const uint4*>(base + (iy >= 0.0f ? 48u : 64u));
+            const uint4 pz = *reinterpret_cast<const uint4*>(base + (iz >= 0.0f ? 80u : 96u));
+            child = *reinterpret_cast<const uint32_t*>(base + 112u + 4u * c);
+            const uint32_t ex = __float_as_uint(co.w);
+            const float ax = __builtin_ldexpf(ix, (int)(int8_t)(ex & 0xFFu));
+            const float ay = __builtin_ldexpf(iy, (int)(int8_t)((ex >> 8) & 0xFFu));
+            const float az = __builtin_ldexpf(iz, (int)(int8_t)((ex >> 16) & 0xFFu));
+            const float bx = (co.x - o.x) * ix, by = (co.y - o.y) * iy, bz = (co.z - o.z) * iz;
+            const auto half = [&](uint32_t w01, uint32_t w23) {  // half c of the four
+                const uint32_t w = (c & 2u ? w23 : w01) >> (c & 1u ? 16 : 0);
+                return __low2float(*reinterpret_cast<const __half2*>(&w));
+            };
+            const float tn = fmaxf(fmaxf(fmaf(half(px.x, px.y), ax, bx), fmaf(half(py.x, py.y), ay, by)),
+                                   fmaxf(fmaf(half(pz.x, pz.y), az, bz), tlo));
+            const float tf = fminf(fminf(fmaf(half(px.z, px.w), ax, bx), fmaf(half(py.z, py.w), ay, by)),
+                                   fminf(fmaf(half(pz.z, pz.w), az, bz), lim));
+            if (tn <= tf * 1.000002f) key = __float_as_int(tn);
+        } else if (mine) {
+            const uint32_t first = leaf_first(word), n_leaf = leaf_count(word);
+            for (uint32_t k = c; k < n_leaf; k += 4u) {
+                const PrimRec pr = S.prims[first + k];
+                if (kAny) {
+                    float t;
+                    hit = hit || (prim_test(pr, o, d, t) && t <= dist && object_box_ok(S, pr, o, d));
+                } else {
+                    closest_prim(S, pr, first + k, o, d, found);
+                }
+            }
+            if (!kAny) hit = found.prim != best.prim;
+        }
+        // the hit children go on top, the first entry's topmost and each entry's nearest first
+        uint32_t nearer = 0;
+#pragma unroll
+        for (uint32_t x = 1; x < 4; ++x) {
+            constexpr int kPerm[4] = {0, 0xB1, 0x4E, 0x1B};  // quad lanes c ^ 1, c ^ 2, c ^ 3
+            const int k = x == 1 ? __builtin_amdgcn_mov_dpp(key, kPerm[1], 0xF, 0xF, true)
+                        : x == 2 ? __builtin_amdgcn_mov_dpp(key, kPerm[2], 0xF, 0xF, true)
+                                 : __builtin_amdgcn_mov_dpp(key, kPerm[3], 0xF, 0xF, true);
+            nearer += k < key || (k == key && (c ^ x) < c) ? 1u : 0u;
+        }
+        const unsigned long long pushed = group_bits(key != kCulled);
+        const uint32_t siblings = (uint32_t)__popcll((pushed >> (4u * entry)) & 15u);
+        const uint32_t below = (uint32_t)__popcll(pushed >> (4u * entry) >> 4);
+        if (key != kCulled) stack[sp + below + siblings - 1u - nearer] = child;
+        sp += (uint32_t)__popcll(pushed);
+        if (kAny) {
+            any = any || group_bits(hit) != 0ull;
+            if (any) sp = 0u;
+        } else if (__ballot(hit)) {
+            reduce(found);
+            best = found;
+        }
+    }
+    return any;
+}
+
 // a load whose address is the same in every lane, issued as a scalar load (records of the
 // BVH and primitive arrays, which no kernel writes while it traverses them)
 __device__ __forceinline__ float4 uniform_load4(const void* p) {
