@@ -24,19 +24,6 @@
 #include "shading.h"
 #include "traverse.h"
 
-// Lanes of the refill loop that must be at a leaf before a wave runs a leaf step (inner-node steps
-// otherwise), at most: a wave runs its leaf step once half of its rays wait at a leaf, capped at
-// this many lanes. 32 (always half) measured best with the half rule (1080p, 1M triangles: cap 12
-// / 16 / 20 / 24 / 28 / 32 -> 1143 / 1155-1159 / 1163 / 1164-1168 / 1168 / 1168 Msamples/s). With
-// a fixed count instead (an earlier build): 8 / 16 / 24 / 32 -> 901 / 932 / 920 / 843; leaf and
-// inner steps taken together every iteration: 889.
-#ifndef CUPBR_LEAF_BATCH
-#define CUPBR_LEAF_BATCH 32
-#endif
-// idle lanes of a wave that trigger a refill from the ray queue
-#ifndef CUPBR_REFILL_IDLE
-#define CUPBR_REFILL_IDLE 32
-#endif
 // Rays per lane of the persistent grid from which a trace launch refills its lanes; below, every wave
 // traces one 64-ray chunk, whose end waits for one tail, not for two (extension rays, then shadow
 // rays). 1080p / 1M triangles at 1 spp with 1, 2 and 4 rays: 4.00, 4.09 and 4.27 ms (the volume renderer,
@@ -432,59 +419,13 @@ struct RayShare {
     __device__ __forceinline__ uint32_t index(uint32_t r) const { return (r / kGranule * 8u + g) * kGranule + r % kGranule; }
 };
 
-// One queue of the trace kernel, n rays, with per-lane refill: a wave gives fresh rays of its share
-// (RayShare) to its idle lanes whenever at least CUPBR_REFILL_IDLE (32) of them are idle (or all are), so
-// that a lane whose ray ended does not wait for the slowest ray of a 64-ray chunk. finish(i, hit, r)
-// consumes the result of ray i.
+// One queue of the trace kernel, n rays, dealt out by RayShare; finish(i, hit, r) consumes the result of ray i.
 template <bool kAny, class Load, class Finish>
 __device__ __forceinline__ void trace_queue(const DevScene& S, uint32_t n, CounterLine* counter,
                                             LaneStack<kPtLds>& st, Load load, Finish finish) {
-    const uint32_t lane = __lane_id();
-    bool active = false, pool = true, hit = false;
-    uint32_t my = 0;
     RayShare share;
     share.begin(counter, n);
-    RayState rs;
-    for (;;) {
-        const unsigned long long idle = __ballot(!active);
-        if (pool && (__popcll(idle) >= CUPBR_REFILL_IDLE || idle == ~0ull)) {
-            if (share.at >= share.end) pool = share.refill();
-            if (!active) {
-                const uint32_t idx = share.at + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                if (idx < share.end) {
-                    my = share.index(idx);
-                    v3 o, d;
-                    float dist;
-                    load(my, o, d, dist);
-                    active = ray_begin<kAny>(S, rs, o, d, dist, hit);
-                    if (!active) finish(my, hit, rs.best);
-                }
-            }
-            share.at = min(share.at + (uint32_t)__popcll(idle), share.end);
-        }
-        const unsigned long long am = __ballot(active);
-        if (am == 0ull) {
-            if (!pool) break;
-            continue;
-        }
-        // Wave-uniform phases: a primitive step for the lanes at a leaf once half of the wave's rays
-        // are there (at most CUPBR_LEAF_BATCH lanes), or all of them (no lane has an inner node
-        // left); an inner-node step for the others otherwise. A lane whose ray reached a leaf waits
-        // during inner phases, so that the primitive test runs for many lanes at once instead of a
-        // few in every iteration (before: leaf code in 97% of iterations for 9 of 64 lanes). Counted
-        // against the wave's own rays, the rule also keeps a nearly empty wave (the last rays of a
-        // launch) from holding its leaf lanes back until every other ray reaches a leaf (1080p, 1M
-        // triangles: a fixed 16 lanes 1147, half capped at 16 1155-1159, half 1168 Msamples/s).
-        const bool at_leaf = active && (rs.cur & kLeafBit);
-        const uint32_t n_leaf = (uint32_t)__popcll(__ballot(at_leaf));
-        const uint32_t n_act = (uint32_t)__popcll(am);
-        const bool leaf_phase = n_leaf >= min((uint32_t)CUPBR_LEAF_BATCH, (n_act + 1u) / 2u) || n_leaf == n_act;
-        const bool go = leaf_phase ? at_leaf : (active && !at_leaf);
-        if (go && !ray_step<kAny>(S, rs, st, hit)) {
-            finish(my, hit, rs.best);
-            active = false;
-        }
-    }
+    trace_pool<kAny, true>(S, share, st, load, finish);
 }
 
 // One bounce's extension rays (queue cur), then the previous bounce's shadow rays (parity cur ^ 1),

@@ -128,6 +128,7 @@ int scene_upload(const cupbr_scene* cs) {
     d.n_nodes = (uint32_t)s->h_nodes.size();
     d.n_prims = (uint32_t)s->h_prims.size();
     d.n_unb = (uint32_t)s->h_unb.size();
+    d.stack_reserve = s->stack_entries - 1u;
     d.n_objs = (uint32_t)s->objects.size();
     d.n_lights = (uint32_t)s->lights.size();
     d.env_w = s->env.empty() ? 0 : s->env_w;

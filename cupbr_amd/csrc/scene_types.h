@@ -102,6 +102,7 @@ struct DevScene {
     const float* env;  // env_w * env_h * 3
     const uint32_t* rank_prim;  // reference rank -> prim index, kUnbBit|unbounded index, or 0xFFFFFFFF
     uint32_t n_nodes, n_prims, n_unb, n_objs, n_lights;
+    uint32_t stack_reserve;  // three per BVH4 level: entries one ray's depth-first walk keeps at most
     uint32_t env_w, env_h;
     int32_t use_env;
     cupbr_volume volume;

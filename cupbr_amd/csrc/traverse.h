@@ -381,6 +381,18 @@ __device__ __forceinline__ bool ray_step(const DevScene& S, RayState& r, LaneSta
     return true;
 }
 
+// the minimum of (t, rank) over a group of kGroup lanes, in every lane of it
+template <uint32_t kGroup>
+__device__ __forceinline__ TraceResult group_min(TraceResult r) {
+#pragma unroll
+    for (uint32_t off = 1; off < kGroup; off <<= 1) {
+        const float t = __shfl_xor(r.t, off);
+        const uint32_t prim = __shfl_xor(r.prim, off), rank = __shfl_xor(r.rank, off);
+        if (t < r.t || (t == r.t && rank < r.rank)) r = TraceResult{t, prim, rank};
+    }
+    return r;
+}
+
 // One ray per group of kGroup lanes of a wave: each step takes the kGroup / 4 entries on top of the ray's
 // stack, four lanes to an entry, a lane testing one child of an inner node or every fourth primitive of a
 // leaf. What bounds a batch too small to fill the chip is the longest ray's chain of dependent steps, each
@@ -388,54 +400,33 @@ __device__ __forceinline__ bool ray_step(const DevScene& S, RayState& r, LaneSta
 // sequential order would have culled. The tests are those of traverse, and the result, a minimum of
 // (t, rank) over all primitives of overlapping boxes (any-hit: whether there is one), is the same for any
 // order of visits.
-// stack: kGroup * (depth + 1) words of LDS of the group's own. The levels of the entries never decrease from
-// bottom to top, as children replace their parents in the parents' order. An entry of level d - 1 is taken
-// only together with all entries of levels d and more above it, fewer than kGroup / 4, so the entries of a
-// level that are on the stack at one time come from one step: at most kGroup of them, on depth levels.
-// Called by whole waves; a group with valid = false only takes part in the wave's votes.
-template <bool kAny, uint32_t kGroup>
-__device__ __forceinline__ bool traverse_group(const DevScene& S, v3 o, v3 d, float dist, bool valid, uint32_t* stack,
-                                               TraceResult& best) {
+// stack(k): entry k of kCapacity words of LDS of the group's own. reserve, three words per level of the
+// tree, is what walking one entry at a time can add; a step takes one entry only while its pushes could
+// leave less than that, so reserve < kCapacity is all the stack needs.
+// In: best, a closest hit found already (none: t = inf, rank = 0xFFFFFFFF). Called by whole waves; a group
+// with valid = false only takes part in the wave's votes. Returns (any-hit) whether there is a hit.
+template <bool kAny, uint32_t kGroup, uint32_t kCapacity, class Stack>
+__device__ __forceinline__ bool traverse_group(const DevScene& S, v3 o, v3 d, float dist, bool valid, uint32_t reserve,
+                                               Stack stack, TraceResult& best) {
     constexpr uint32_t kEntries = kGroup / 4;
     constexpr int kCulled = 0x7FFFFFFF;
     const uint32_t lane = __lane_id(), sub = lane % kGroup, entry = sub >> 2, c = sub & 3u;
     const auto group_bits = [&](bool b) {  // the group's votes, lane sub in bit sub
         return (__ballot(b) >> (lane - sub)) & (~0ull >> (64u - kGroup));
     };
-    const auto reduce = [&](TraceResult& r) {  // the group's minimum of (t, rank), in every lane
-#pragma unroll
-        for (uint32_t off = 1; off < kGroup; off <<= 1) {
-            const float t = __shfl_xor(r.t, off);
-            const uint32_t prim = __shfl_xor(r.prim, off), rank = __shfl_xor(r.rank, off);
-            if (t < r.t || (t == r.t && rank < r.rank)) r = TraceResult{t, prim, rank};
-        }
-    };
-    best = TraceResult{__builtin_inff(), kNoHit, 0xFFFFFFFFu};
     bool any = false;
-    if (valid)
-        for (uint32_t i = sub; i < S.n_unb; i += kGroup) {
-            const UnbRec u = S.unb[i];
-            float t;
-            if (!plane_quad_test(u, o, d, t)) continue;
-            const uint32_t rank = __float_as_uint(u.n.w);
-            any = any || t <= dist;
-            if (t < best.t || (t == best.t && rank < best.rank)) best = TraceResult{t, kUnbBit | i, rank};
-        }
-    if (kAny)
-        any = group_bits(any) != 0ull;
-    else if (S.n_unb)
-        reduce(best);
     const float ix = 1.0f / d.x, iy = 1.0f / d.y, iz = 1.0f / d.z;
     const float tlo = -1e-5f;
-    uint32_t sp = valid && !(kAny && any) && S.n_nodes ? 1u : 0u;
-    if (sub == 0u) stack[0] = 0u;
+    uint32_t sp = valid && S.n_nodes ? 1u : 0u;
+    if (sub == 0u) stack(0u) = 0u;
     while (__ballot(sp != 0u)) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();  // the entries pushed by other lanes
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const bool mine = entry < sp;
-        const uint32_t word = mine ? stack[sp - 1u - entry] : kLeafBit;
-        sp -= min(sp, kEntries);
+        const uint32_t take = min(sp, sp + 3u * kEntries + reserve <= kCapacity ? kEntries : 1u);
+        const bool mine = entry < take;
+        const uint32_t word = mine ? stack(sp - 1u - entry) : kLeafBit;
+        sp -= take;
         int key = kCulled;
         uint32_t child = 0u;
         TraceResult found = best;
@@ -488,17 +479,131 @@ __device__ __forceinline__ bool traverse_group(const DevScene& S, v3 o, v3 d, fl
         const unsigned long long pushed = group_bits(key != kCulled);
         const uint32_t siblings = (uint32_t)__popcll((pushed >> (4u * entry)) & 15u);
         const uint32_t below = (uint32_t)__popcll(pushed >> (4u * entry) >> 4);
-        if (key != kCulled) stack[sp + below + siblings - 1u - nearer] = child;
+        if (key != kCulled) stack(sp + below + siblings - 1u - nearer) = child;
         sp += (uint32_t)__popcll(pushed);
         if (kAny) {
             any = any || group_bits(hit) != 0ull;
             if (any) sp = 0u;
         } else if (__ballot(hit)) {
-            reduce(found);
-            best = found;
+            best = group_min<kGroup>(found);
         }
     }
     return any;
+}
+
+// traverse with a group of kGroup lanes per ray
+template <bool kAny, uint32_t kGroup, uint32_t kCapacity, class Stack>
+__device__ __forceinline__ bool trace_group(const DevScene& S, v3 o, v3 d, float dist, bool valid, uint32_t reserve,
+                                            Stack stack, TraceResult& best) {
+    best = TraceResult{__builtin_inff(), kNoHit, 0xFFFFFFFFu};
+    bool any = false;
+    if (valid)  // planes and quads first, as in traverse
+        for (uint32_t i = __lane_id() % kGroup; i < S.n_unb; i += kGroup) {
+            const UnbRec u = S.unb[i];
+            float t;
+            if (!plane_quad_test(u, o, d, t)) continue;
+            const uint32_t rank = __float_as_uint(u.n.w);
+            any = any || t <= dist;
+            if (t < best.t || (t == best.t && rank < best.rank)) best = TraceResult{t, kUnbBit | i, rank};
+        }
+    if (kAny) {
+        const uint32_t first = __lane_id() / kGroup * kGroup;
+        any = ((__ballot(any) >> first) & (~0ull >> (64u - kGroup))) != 0ull;
+    } else if (S.n_unb) {
+        best = group_min<kGroup>(best);
+    }
+    return traverse_group<kAny, kGroup, kCapacity>(S, o, d, dist, valid && !(kAny && any), reserve, stack, best) || (kAny && any);
+}
+
+// Lanes of the refill loop that must be at a leaf before a wave runs a leaf step (inner-node steps
+// otherwise), at most: a wave runs its leaf step once half of its rays wait at a leaf, capped at
+// this many lanes. 32 (always half) measured best with the half rule (1080p, 1M triangles: cap 12
+// / 16 / 20 / 24 / 28 / 32 -> 1143 / 1155-1159 / 1163 / 1164-1168 / 1168 / 1168 Msamples/s). With
+// a fixed count instead (an earlier build): 8 / 16 / 24 / 32 -> 901 / 932 / 920 / 843; leaf and
+// inner steps taken together every iteration: 889.
+constexpr uint32_t kLeafBatch = 32;
+// lanes per ray for a wave's last rays
+constexpr uint32_t kTailGroup = 16;
+
+// The rays of a wave's share, with per-lane refill: the wave gives fresh rays to its idle lanes whenever at
+// least kIdle of them are idle (or all are), so that a lane whose ray ended does not wait for the slowest
+// ray of a 64-ray chunk. The share has a current piece [at, end); refill() makes a new one (false when
+// there is none), index(k) names its ray k. load(i, o, d, dist) reads ray i, finish(i, hit, r) consumes
+// its result. Two ways of stepping:
+//   kPhased   leaf steps and inner-node steps of the wave apart (below): most rays per second where a
+//             wave refills many times
+//   otherwise every lane its own step, and the last rays of the share by kTailGroup lanes each
+//             (traverse_group), which start them over with the hit found so far: shortest where a wave
+//             has only a few rays per lane and its longest ray bounds it. The path tracer's trace kernel
+//             does not take it: the second walk costs it 14 spilled registers (109.6 -> 114.4 ms a frame
+//             of 1080p, 1M triangles, 64 spp) and saves 1% of a 1-spp frame.
+template <bool kAny, bool kPhased, class Share, int kLds, class Load, class Finish>
+__device__ __forceinline__ void trace_pool(const DevScene& S, Share& share, LaneStack<kLds>& st, Load load,
+                                           Finish finish) {
+    constexpr uint32_t kTailWords = kLds * kTailGroup;
+    constexpr int kIdle = kPhased ? 32 : 16;
+    const uint32_t lane = __lane_id();
+    bool active = false, pool = true, hit = false;
+    decltype(share.index(0u)) my = 0;
+    RayState rs;
+    for (;;) {
+        const unsigned long long idle = __ballot(!active);
+        if (pool && (__popcll(idle) >= kIdle || idle == ~0ull)) {
+            if (share.at >= share.end) pool = share.refill();
+            if (!active) {
+                const uint32_t idx = share.at + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+                if (idx < share.end) {
+                    my = share.index(idx);
+                    v3 o, d;
+                    float dist;
+                    load(my, o, d, dist);
+                    active = ray_begin<kAny>(S, rs, o, d, dist, hit);
+                    if (!active) finish(my, hit, rs.best);
+                }
+            }
+            share.at = min(share.at + (uint32_t)__popcll(idle), share.end);
+        }
+        const unsigned long long am = __ballot(active);
+        if (am == 0ull) {
+            if (!pool) break;
+            continue;
+        }
+        if (!kPhased && !pool && (uint32_t)__popcll(am) <= 64u / kTailGroup && S.stack_reserve < kTailWords) {
+            unsigned long long m = am;
+            for (uint32_t k = lane / kTailGroup; k != 0u; --k) m &= m - 1ull;  // 0 from the last ray on
+            const bool valid = m != 0ull;
+            const int src = valid ? __builtin_ctzll(m) : 0;
+            const auto from = [&](float x) { return __shfl(x, src); };
+            const v3 o = mk(from(rs.o.x), from(rs.o.y), from(rs.o.z)), d = mk(from(rs.d.x), from(rs.d.y), from(rs.d.z));
+            TraceResult best{from(rs.best.t), (uint32_t)__shfl((int)rs.best.prim, src), (uint32_t)__shfl((int)rs.best.rank, src)};
+            my = __shfl(my, src);
+            const uint32_t first = lane / kTailGroup * kTailWords;  // the wave's stacks end here: row by row, 64 words each
+            uint32_t* words = st.lds - lane;
+            const uint32_t row = st.lds_stride;
+            const bool any = traverse_group<kAny, kTailGroup, kTailWords>(
+                S, o, d, best.t, valid, S.stack_reserve,
+                [&](uint32_t k) -> uint32_t& { return words[((first + k) >> 6) * row + ((first + k) & 63u)]; }, best);
+            if (valid && lane % kTailGroup == 0u) finish(my, any, best);
+            break;
+        }
+        // Wave-uniform phases: a primitive step for the lanes at a leaf once half of the wave's rays
+        // are there (at most kLeafBatch lanes), or all of them (no lane has an inner node
+        // left); an inner-node step for the others otherwise. A lane whose ray reached a leaf waits
+        // during inner phases, so that the primitive test runs for many lanes at once instead of a
+        // few in every iteration (before: leaf code in 97% of iterations for 9 of 64 lanes). Counted
+        // against the wave's own rays, the rule also keeps a nearly empty wave (the last rays of a
+        // launch) from holding its leaf lanes back until every other ray reaches a leaf (1080p, 1M
+        // triangles: a fixed 16 lanes 1147, half capped at 16 1155-1159, half 1168 Msamples/s).
+        const bool at_leaf = active && (rs.cur & kLeafBit);
+        const uint32_t n_leaf = (uint32_t)__popcll(__ballot(at_leaf));
+        const uint32_t n_act = (uint32_t)__popcll(am);
+        const bool leaf_phase = n_leaf >= min(kLeafBatch, (n_act + 1u) / 2u) || n_leaf == n_act;
+        const bool go = !kPhased ? active : leaf_phase ? at_leaf : active && !at_leaf;
+        if (go && !ray_step<kAny>(S, rs, st, hit)) {
+            finish(my, hit, rs.best);
+            active = false;
+        }
+    }
 }
 
 // a load whose address is the same in every lane, issued as a scalar load (records of the

@@ -75,3 +75,20 @@ def test_scene_without_a_tree():
             assert np.array_equal(a, c)
         vis = S.trace_visibility(torch.from_numpy(rays[:n]).cuda(), torch.from_numpy(dist[:n]).cuda()).cpu().numpy()
         assert np.array_equal(ref.visibility(rays[:n], dist[:n], precision=32, mode=0), vis)
+
+
+@pytest.mark.parametrize("name", ["meshes", "mixed"])
+def test_large_batches_agree(name):
+    """One lane per ray: pieces of 64 rays (one refill) to 512, whole and ragged, with the wave's last rays
+    walked by groups; the results of a batch are the slice of a larger one's."""
+    make, lo, hi = SCENES[name]
+    S = cb.Scene.from_desc(make())
+    n = 2_200_001
+    rays, dist = (torch.from_numpy(x).cuda() for x in _rays(n, lo, hi, 23))
+    whole = list(S.trace_closest(rays)) + [S.trace_visibility(rays, dist)]
+    for first, count in ((0, 64), (3, 100_000), (n - 163_841, 163_841), (1, 262_144), (17, 700_003)):
+        print(f"{name}: {count} rays", flush=True)
+        part = slice(first, first + count)
+        r, d = rays[part].contiguous(), dist[part].contiguous()
+        for a, b in zip(whole, list(S.trace_closest(r)) + [S.trace_visibility(r, d)]):
+            assert torch.equal(a[part].view(torch.uint8), b.view(torch.uint8))
