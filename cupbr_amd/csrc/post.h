@@ -11,7 +11,7 @@ struct cupbr_post {
     cupbr::DevBuf output;        // getPostProcessBuffer()
     hipStream_t stream = nullptr;
     int32_t pyramid = CUPBR_BLOOM_REFERENCE;
-    cupbr::DevBuf levels;        // Gaussian pyramid: the thresholded image and five levels
+    cupbr::DevBuf levels;        // Gaussian pyramid: its five levels
 };
 
 struct cupbr_tonemapper {
