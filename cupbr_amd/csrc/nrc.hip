@@ -152,16 +152,16 @@ __global__ __launch_bounds__(kNrcBlock, 2) void k_nrc_infer(const bf16x8* __rest
                                                             const uint32_t* __restrict__ n_dev, uint32_t stride,
                                                             float* __restrict__ out,
                                                             const uint32_t* __restrict__ begin_dev) {
+    const int lane = threadIdx.x & 63, g = lane >> 4;
+    bf16x8 w[kFwdSize / 512];  // loaded while the counts are
+#pragma unroll
+    for (int i = 0; i < kFwdSize / 512; ++i) w[i] = packed[i * 64 + lane];
     if (n_dev) n = min(n, *n_dev);  // count written by an earlier kernel on the stream
     const uint32_t begin = begin_dev ? min(*begin_dev, n) : 0u;
-    const int lane = threadIdx.x & 63, g = lane >> 4;
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const uint32_t n_waves = (gridDim.x * blockDim.x) >> 6;
     const uint32_t pairs = (n - begin + 31) / 32;  // two tiles of 16 queries per wave and step
     if (wave >= pairs) return;
-    bf16x8 w[kFwdSize / 512];
-#pragma unroll
-    for (int i = 0; i < kFwdSize / 512; ++i) w[i] = packed[i * 64 + lane];
     for (uint32_t t = wave; t < pairs; t += n_waves) {
         uint32_t q[2];
         bf16x8 a[2][2], b[2][2];
@@ -185,6 +185,20 @@ __global__ __launch_bounds__(kNrcBlock, 2) void k_nrc_infer(const bf16x8* __rest
             }
             encode(box, raw, g, a[h]);
         }
+        // the path's throughput and radiance while the layers run
+        f32x4 thr[2];
+        float* px[2];
+        float rgb[2][3];
+        if (kAccumulate && g == 0) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (q[h] >= n) continue;
+                const float* r = rec + (size_t)q[h] * stride;
+                thr[h] = f32x4{r[16], r[17], r[18], r[19]};
+                px[h] = out + 4 * (size_t)__float_as_uint(thr[h][3]);
+                for (int k = 0; k < 3; ++k) rgb[h][k] = px[h][k];
+            }
+        }
         hidden_layer2(w, a[0], a[1], b[0], b[1]);
         hidden_layer2(w + 8, b[0], b[1], a[0], a[1]);
         hidden_layer2(w + 16, a[0], a[1], b[0], b[1]);
@@ -195,12 +209,7 @@ __global__ __launch_bounds__(kNrcBlock, 2) void k_nrc_infer(const bf16x8* __rest
             for (int kc = 0; kc < 2; ++kc) o = mfma(w[32 + kc], a[h][kc], o);
             if (g == 0 && q[h] < n) {
                 if (kAccumulate) {
-                    const float* r = rec + (size_t)q[h] * stride;
-                    const uint32_t path = __float_as_uint(r[19]);
-                    float* px = out + 4 * (size_t)path;
-                    px[0] += r[16] * fmaxf(o[0], 0.0f);
-                    px[1] += r[17] * fmaxf(o[1], 0.0f);
-                    px[2] += r[18] * fmaxf(o[2], 0.0f);
+                    for (int k = 0; k < 3; ++k) px[h][k] = rgb[h][k] + thr[h][k] * fmaxf(o[k], 0.0f);
                 } else {
                     out[3 * (size_t)q[h] + 0] = o[0];
                     out[3 * (size_t)q[h] + 1] = o[1];
@@ -267,9 +276,9 @@ __global__ __launch_bounds__(kNrcBlock, 1) void k_nrc_train(const bf16x8* __rest
                                                             float* __restrict__ losses) {
     __shared__ bf16x8 wf[kFwdSize / 8];
     __shared__ bf16x8 wb[kBwdSize / 8];
-    // [layer][feature][row]: X of the 5 layers, then G of the 4 hidden ones
-    __shared__ __attribute__((aligned(16))) __bf16 xg[9][64 * kTrainStride];
-    __shared__ __attribute__((aligned(16))) __bf16 g5[16 * kTrainStride];
+    // [feature][row], 16 features per operand: X of the 5 layers, G of the 4 hidden ones, G of the output layer
+    __shared__ __attribute__((aligned(16))) __bf16 xg[kOperands * 16 * kTrainStride];
+    __bf16* const g5 = xg + 36 * 16 * kTrainStride;
     __shared__ float loss_s[kNrcBlock / 64];
     const int lane = threadIdx.x & 63, g = lane >> 4, wave = threadIdx.x >> 6;
     const int col = wave * 16 + (lane & 15);
@@ -296,6 +305,8 @@ __global__ __launch_bounds__(kNrcBlock, 1) void k_nrc_train(const bf16x8* __rest
         for (int k = 0; k < 19; ++k) raw[k] = r[k];
     };
     load_row(tile_at(blockIdx.x));
+    bf16x8 x[5][2];
+    encode(box, raw, g, x[0]);  // while the weights arrive
 #pragma unroll
     for (int k = 0; k < nf; ++k)
         if ((int)threadIdx.x + k * kNrcBlock < kFwdSize / 8) wf[threadIdx.x + k * kNrcBlock] = f[k];
@@ -306,10 +317,11 @@ __global__ __launch_bounds__(kNrcBlock, 1) void k_nrc_train(const bf16x8* __rest
     float loss_acc = 0.0f;
     for (uint32_t u = blockIdx.x; tile_at(u) < B / kTrainRows; u += gridDim.x) {  // gridDim.x: a multiple of 64
         const uint32_t t = tile_at(u);
-        if (u != blockIdx.x) load_row(t);
-        bf16x8 x[5][2];
+        if (u != blockIdx.x) {
+            load_row(t);
+            encode(box, raw, g, x[0]);
+        }
         f32x4 pre[4][4];
-        encode(box, raw, g, x[0]);
 #pragma unroll
         for (int L = 0; L < 4; ++L) hidden_layer(wf + L * (kFwdLayer / 8), lane, x[L], x[L + 1], pre[L]);
         const f32x4 o = output_layer(wf + 4 * (kFwdLayer / 8), lane, x[4]);
@@ -329,7 +341,7 @@ __global__ __launch_bounds__(kNrcBlock, 1) void k_nrc_train(const bf16x8* __rest
             }
         }
 #pragma unroll
-        for (int L = 0; L < 5; ++L) store_rows(xg[L], col, g, x[L]);
+        for (int L = 0; L < 5; ++L) store_rows(xg + L * 64 * kTrainStride, col, g, x[L]);
 #pragma unroll
         for (int j = 0; j < 4; ++j) g5[(g * 4 + j) * kTrainStride + col] = g == 0 ? cur[0][j] : to_bf16(0.0f);
         // backward through W5^T, then W4^T..W2^T, masking with the ReLU of each hidden layer
@@ -354,18 +366,24 @@ __global__ __launch_bounds__(kNrcBlock, 1) void k_nrc_train(const bf16x8* __rest
                     const int ot = 2 * kc + (j >> 2), v = j & 3;
                     cur[kc][j] = to_bf16(pre[L][ot][v] > 0.0f ? acc[ot][v] : 0.0f);
                 }
-            store_rows(xg[5 + L], col, g, cur);
+            store_rows(xg + (5 + L) * 64 * kTrainStride, col, g, cur);
         }
         __syncthreads();
-        // operand rows: lane l holds row l % 16 of its 16 features, batch rows 32 half + 8 (l / 16) .. + 7
-        const int at = (lane & 15) * kTrainStride + 8 * g;
-        bf16x8* to = acts + (size_t)(t / kSliceTiles) * kOperands * kSliceOperand +
-                     t % kSliceTiles * (kTrainRows / 32 * 64) + lane;
-        for (uint32_t k = wave; k < 2 * kOperands; k += kNrcBlock / 64) {
-            const uint32_t half = k & 1u, op = k >> 1;
-            const __bf16* from = op < 36u ? xg[op >> 2] + (op & 3u) * 16u * kTrainStride : g5;
-            to[op * kSliceOperand + half * 64u] = *reinterpret_cast<const bf16x8*>(from + at + 32 * half);
-        }
+        // operand rows: lane l holds row l % 16 of its 16 features, batch rows 32 half + 8 (l / 16) .. + 7.
+        // Wave w copies half w % 2 of operands w / 2, w / 2 + 2, .., all reads in flight together (a step of 4096
+        // rows 15.3 -> 13.9 us)
+        const uint32_t half = wave & 1u, op0 = wave >> 1;
+        const __bf16* from = xg + (op0 * 16u + (lane & 15u)) * kTrainStride + 32u * half + 8u * g;
+        bf16x8* to = acts + ((size_t)(t / kSliceTiles) * kOperands + op0) * kSliceOperand +
+                     t % kSliceTiles * (kTrainRows / 32 * 64) + half * 64u + lane;
+        constexpr uint32_t n_copies = (kOperands + 1) / 2;
+        bf16x8 v[n_copies];
+#pragma unroll
+        for (uint32_t j = 0; j < n_copies; ++j)
+            if (op0 + 2u * j < kOperands) v[j] = *reinterpret_cast<const bf16x8*>(from + j * 32u * kTrainStride);
+#pragma unroll
+        for (uint32_t j = 0; j < n_copies; ++j)
+            if (op0 + 2u * j < kOperands) to[j * 2u * kSliceOperand] = v[j];
         __syncthreads();
     }
     for (int off = 32; off > 0; off >>= 1) loss_acc += __shfl_xor(loss_acc, off);
