@@ -39,6 +39,18 @@ constexpr int kPtWaves = kPtBlock / 64;
 // traversal stack entries per lane kept in LDS (16 KB per 256-thread block: the trace kernel's 61
 // VGPRs, not LDS, then bound its occupancy at 8 waves per SIMD; deeper entries spill to memory)
 constexpr int kPtLds = 16;
+// Batches of up to this many paths per CU run whole paths in one launch (k_pt_paths): as many as are resident at
+// once, 4 waves per SIMD. What bounds a small batch is the longest path's chain of rays and, with a launch and a
+// queue per bounce, the launches; a resident batch needs neither queues nor the path state in memory. Frames of
+// 256x256, 1 spp, depth 5, queues / whole paths (us): Cornell box 189 / 156, mixed primitives 197 / 147, spheres and
+// boxes 819 / 277, 1M triangles 1503 / 761; 512x512: 279 / 241, 261 / 246, 994 / 590, 1623 / 1541. At 331x217,
+// 6 spp (1.6 times the limit) 299 / 300, 360 / 311, 1003 / 738, but 1786 / 2371.
+constexpr uint32_t kWholePaths = 1024;
+// Traversal stack entries (three per BVH4 level) above which a wave of such a batch holds only as many paths (8 to 32)
+// as 16 waves per CU need, so that 8 lanes walk the tree for each: 1M triangles, 64x64, 1 spp, 1310 -> 312 us, 256x256
+// 1318 -> 761. In a shallow tree that pays up to 64 paths per CU only (Cornell box, depth 5: 64x64 158 -> 100 us, but
+// 256x256 156 -> 225).
+constexpr uint32_t kDeepStack = 24;
 // consecutive rays of a trace queue that belong to one XCD
 constexpr uint32_t kGranule = 1024;
 
@@ -124,8 +136,7 @@ __device__ __forceinline__ void reset_batch_counters(Counters* c, uint32_t npath
     for (int g = 0; g < 8; ++g) c->work[g].v = c->swork[g].v = 0;
     c->shadow_count[0].v = 0;
     c->shadow_count[1].v = 0;
-    c->query_count.v = 0;
-    c->row_count.v = 0;
+    c->cache.both = 0;
     c->iqueue_count[0].v = 0;
     c->iqueue_count[1].v = 0;
 }
@@ -175,6 +186,87 @@ struct NrcShade {
     float camera_min_roughness;
 };
 
+// What a path's vertex adds and asks for.
+struct Vertex {
+    bool emits, next, shadow, query, row;
+    v3 emission;  // to the path's radiance (emits), before the light's contribution
+    v3 next_o, next_d;
+    v3 shadow_o, shadow_d, light;  // shadow ray, and what the light adds if it is visible
+    float dist;
+    float4 rec[6];  // cache query or pending row
+};
+
+// One vertex of path p, where its ray (o, d) hit prim at t, or left the scene: PathTracer.cu:20-160 in the
+// reference's order. w3: throughput. L: the path's radiance so far, for the cache's records only.
+template <bool kNrc, class Seed>
+__device__ __forceinline__ void path_vertex(const DevScene& S, uint32_t bounce, uint32_t max_depth, int rr,
+                                            const NrcShade& nrc, v3 o, v3 d, float t, uint32_t prim, uint32_t p,
+                                            bool training, v3 L, v3& w3, Seed& seed, Vertex& v) {
+    v.emits = v.next = v.shadow = v.query = v.row = false;
+    if (prim == kNoHit) {  // :127-135
+        if (S.use_env) {
+            v.emission = w3 * env_lookup(S, d);
+            v.emits = true;
+        }
+        return;
+    }
+    const float nl = (float)(S.n_lights + (S.use_env ? 1u : 0u));
+    const v3 P = o + t * d;  // geom.P = origin + t * direction
+    v3 N;
+    uint32_t obj;
+    hit_geometry(S, prim, P, N, obj);
+    const Mat m = load_mat(S.mats + obj);
+    const v3 inc = -1.0f * d;
+    // emissiveIllumintation :20-26; nothing for a black surface, unless the throughput is infinite or NaN
+    v.emission = w3 * m.albedo_e;
+    v.emits = !(v.emission.x == 0.0f && v.emission.y == 0.0f && v.emission.z == 0.0f);
+    const bool cache_vertex = bounce >= 1 ? (m.type == CUPBR_LAMBERT || m.type == CUPBR_PHONG || m.type == CUPBR_GGX)
+                                          : ((m.type == CUPBR_LAMBERT && nrc.camera_min_roughness <= 1.0f) ||
+                                             (m.type == CUPBR_GGX && m.roughness >= nrc.camera_min_roughness));
+    if (kNrc && cache_vertex && !(dot(N, inc) <= 0.0f)) {
+        v.rec[0] = make_float4(P.x, P.y, P.z, inc.x);
+        v.rec[1] = make_float4(inc.y, inc.z, N.x, N.y);
+        v.rec[2] = make_float4(N.z, m.roughness, m.albedo_d.x, m.albedo_d.y);
+        v.rec[3] = make_float4(m.albedo_d.z, m.albedo_s.x, m.albedo_s.y, m.albedo_s.z);
+        if (!training) {  // rendering path: ends here with throughput * cache
+            v.query = true;
+            v.rec[4] = make_float4(w3.x, w3.y, w3.z, __uint_as_float(p));
+            return;
+        }
+        v.row = true;  // training path: pending row, the path goes on
+        L += v.emission;
+        v.rec[4] = make_float4(L.x, L.y, L.z, w3.x);
+        v.rec[5] = make_float4(w3.y, w3.z, __uint_as_float(p), 0.0f);
+    }
+    if (m.type != CUPBR_GLASS && dot(N, inc) <= 0.0f) return;  // :36-41
+    // directIllumination :43-73
+    v3 ldir, le;
+    float dist = 0.0f;
+    if (nee_sample(S, m, seed, P, inc, N, ldir, le, dist)) {
+        v.light = (nl * fmaxf(0.0f, dot(N, ldir))) * brdf(m, inc, ldir, N) * le * w3;
+        if (!(v.light.x == 0.0f && v.light.y == 0.0f && v.light.z == 0.0f)) {
+            v.shadow = true;
+            v.shadow_o = P + 0.001f * ldir;
+            v.shadow_d = normalize(ldir);
+            v.dist = dist;
+        }
+    }
+    if (rr) {  // :141-152
+        const float alpha = clampf(fmaxf(w3.x, fmaxf(w3.y, w3.z)), 0.0f, 1.0f);
+        if (rnd(seed) > alpha || safe_float_equal(alpha, 0.0f)) return;
+        w3 = w3 / alpha;
+    }
+    // indirectIllumination :76-95
+    const DirPdf sp = sample_direction(m, seed, inc, N);
+    if (norm(sp.d) < kEpsilon) return;
+    w3 = w3 * fabsf(dot(sp.d, N)) * brdf(m, inc, sp.d, N) / sp.pdf;
+    if (bounce + 1 < max_depth) {  // :156-160
+        v.next = true;
+        v.next_o = P + 0.01f * sp.d;
+        v.next_d = normalize(sp.d);
+    }
+}
+
 template <bool kNrc, class Seed>
 __device__ __forceinline__ void pt_shade(const DevScene& S, int cur, uint32_t bounce, uint32_t max_depth, int rr,
                                          const float4* __restrict__ q_o, const float4* __restrict__ q_d,
@@ -187,121 +279,46 @@ __device__ __forceinline__ void pt_shade(const DevScene& S, int cur, uint32_t bo
     const uint32_t n = c->queue_count[cur].v;
     if (blockIdx.x == 0 && threadIdx.x < 8)  // the next trace starts at 0
         c->work[threadIdx.x].v = c->swork[threadIdx.x].v = 0;
-    const float nl = (float)(S.n_lights + (S.use_env ? 1u : 0u));
     for (uint32_t base = blockIdx.x * kPtBlock; base < n; base += gridDim.x * kPtBlock) {
         const uint32_t i = base + threadIdx.x;
-        bool want_next = false, want_shadow = false, want_query = false, want_row = false;
-        float4 no = {}, nd = {}, so = {}, sd = {}, sc = {};
-        float4 rec[6] = {};  // cache query or pending row
+        Vertex v;
+        v.next = v.shadow = v.query = v.row = false;
+        uint32_t p = 0;
         if (i < n) {
             const float4 o4 = q_o[i & omask], d4 = q_d[i];
             const float2 hh = q_hit[i];
-            const uint32_t p = __float_as_uint(d4.w);
-            const v3 o = mk(o4.x, o4.y, o4.z), d = mk(d4.x, d4.y, d4.z);
+            p = __float_as_uint(d4.w);
             const float4 W = weight[p];
-            const float4 R = rad[p];
+            float4 R = {};
+            if (kNrc) R = rad[p];
             v3 w3 = mk(W.x, W.y, W.z);
             Seed seed = seed_from_bits<Seed>(__float_as_uint(W.w));
-            v3 L = mk(R.x, R.y, R.z);
-            const uint32_t prim = __float_as_uint(hh.y);
-            if (prim == kNoHit) {  // :127-135
-                if (S.use_env) L += w3 * env_lookup(S, d);
-            } else {
-                const v3 P = o + hh.x * d;  // geom.P = origin + t * direction
-                v3 N;
-                uint32_t obj;
-                hit_geometry(S, prim, P, N, obj);
-                const Mat m = load_mat(S.mats + obj);
-                const v3 inc = -1.0f * d;
-                L += w3 * m.albedo_e;  // emissiveIllumintation :20-26
-                bool alive = true;
-                bool cached = false;
-                const bool cache_vertex =
-                    bounce >= 1 ? (m.type == CUPBR_LAMBERT || m.type == CUPBR_PHONG || m.type == CUPBR_GGX)
-                                : ((m.type == CUPBR_LAMBERT && nrc.camera_min_roughness <= 1.0f) ||
-                                   (m.type == CUPBR_GGX && m.roughness >= nrc.camera_min_roughness));
-                if (kNrc && cache_vertex && !(dot(N, inc) <= 0.0f)) {
-                    rec[0] = make_float4(P.x, P.y, P.z, inc.x);
-                    rec[1] = make_float4(inc.y, inc.z, N.x, N.y);
-                    rec[2] = make_float4(N.z, m.roughness, m.albedo_d.x, m.albedo_d.y);
-                    rec[3] = make_float4(m.albedo_d.z, m.albedo_s.x, m.albedo_s.y, m.albedo_s.z);
-                    if (__float_as_uint(R.w) & 1u) {  // training path: pending row, the path goes on
-                        want_row = true;
-                        rec[4] = make_float4(L.x, L.y, L.z, w3.x);
-                        rec[5] = make_float4(w3.y, w3.z, __uint_as_float(p), 0.0f);
-                    } else {  // rendering path: ends here with throughput * cache
-                        want_query = true;
-                        cached = true;
-                        rec[4] = make_float4(w3.x, w3.y, w3.z, __uint_as_float(p));
-                    }
-                }
-                if (cached) {
-                    alive = false;
-                } else if (m.type != CUPBR_GLASS && dot(N, inc) <= 0.0f) {  // :36-41
-                    w3 = splat(0.0f);
-                    alive = false;
-                } else {
-                    // directIllumination :43-73
-                    v3 ldir, le;
-                    float dist = 0.0f;
-                    if (nee_sample(S, m, seed, P, inc, N, ldir, le, dist)) {
-                        const v3 contrib = (nl * fmaxf(0.0f, dot(N, ldir))) * brdf(m, inc, ldir, N) * le * w3;
-                        if (!(contrib.x == 0.0f && contrib.y == 0.0f && contrib.z == 0.0f)) {
-                            const v3 sorg = P + 0.001f * ldir;
-                            const v3 sdir = normalize(ldir);
-                            want_shadow = true;
-                            so = make_float4(sorg.x, sorg.y, sorg.z, dist);
-                            sd = make_float4(sdir.x, sdir.y, sdir.z, __uint_as_float(p));
-                            sc = make_float4(contrib.x, contrib.y, contrib.z, 0.0f);
-                        }
-                    }
-                    if (rr) {  // :141-152
-                        const float alpha = clampf(fmaxf(w3.x, fmaxf(w3.y, w3.z)), 0.0f, 1.0f);
-                        if (rnd(seed) > alpha || safe_float_equal(alpha, 0.0f)) {
-                            alive = false;
-                            w3 = splat(0.0f);
-                        } else {
-                            w3 = w3 / alpha;
-                        }
-                    }
-                    if (alive) {  // indirectIllumination :76-95
-                        const DirPdf sp = sample_direction(m, seed, inc, N);
-                        if (norm(sp.d) < kEpsilon) {
-                            alive = false;
-                        } else {
-                            w3 = w3 * fabsf(dot(sp.d, N)) * brdf(m, inc, sp.d, N) / sp.pdf;
-                            if (bounce + 1 < max_depth) {  // :156-160
-                                const v3 norg = P + 0.01f * sp.d;
-                                const v3 ndir = normalize(sp.d);
-                                want_next = true;
-                                no = make_float4(norg.x, norg.y, norg.z, 0.0f);
-                                nd = make_float4(ndir.x, ndir.y, ndir.z, __uint_as_float(p));
-                            }
-                        }
-                    }
-                }
-                weight[p] = make_float4(w3.x, w3.y, w3.z, __uint_as_float(state_bits(seed)));
+            path_vertex<kNrc, Seed>(S, bounce, max_depth, rr, nrc, mk(o4.x, o4.y, o4.z), mk(d4.x, d4.y, d4.z), hh.x,
+                                    __float_as_uint(hh.y), p, __float_as_uint(R.w) & 1u, mk(R.x, R.y, R.z), w3, seed, v);
+            if (v.emits) {
+                if (!kNrc) R = rad[p];
+                rad[p] = make_float4(R.x + v.emission.x, R.y + v.emission.y, R.z + v.emission.z, R.w);
             }
-            rad[p] = make_float4(L.x, L.y, L.z, R.w);
+            if (v.next) weight[p] = make_float4(w3.x, w3.y, w3.z, __uint_as_float(state_bits(seed)));
         }
-        const uint32_t ns = block_append(want_next, &c->queue_count[cur ^ 1].v, s_append);
-        if (want_next) {
-            nq_o[ns] = no;
-            nq_d[ns] = nd;
+        const uint32_t ns = block_append(v.next, &c->queue_count[cur ^ 1].v, s_append);
+        if (v.next) {
+            nq_o[ns] = make_float4(v.next_o.x, v.next_o.y, v.next_o.z, 0.0f);
+            nq_d[ns] = make_float4(v.next_d.x, v.next_d.y, v.next_d.z, __uint_as_float(p));
         }
-        const uint32_t ss = block_append(want_shadow, &c->shadow_count[cur].v, s_append);
-        if (want_shadow) {
-            s_o[ss] = so;
-            s_d[ss] = sd;
-            s_c[ss] = sc;
+        const uint32_t ss = block_append(v.shadow, &c->shadow_count[cur].v, s_append);
+        if (v.shadow) {
+            s_o[ss] = make_float4(v.shadow_o.x, v.shadow_o.y, v.shadow_o.z, v.dist);
+            s_d[ss] = make_float4(v.shadow_d.x, v.shadow_d.y, v.shadow_d.z, __uint_as_float(p));
+            s_c[ss] = make_float4(v.light.x, v.light.y, v.light.z, 0.0f);
         }
         if (kNrc) {
-            const uint32_t qs = block_append(want_query, &c->query_count.v, s_append);
-            if (want_query)
-                for (int k = 0; k < 5; ++k) nrc.queries[(size_t)qs * 5 + k] = rec[k];
-            const uint32_t rs = block_append(want_row, &c->row_count.v, s_append);
-            if (want_row && rs < nrc.max_rows)
-                for (int k = 0; k < 6; ++k) nrc.pending[(size_t)rs * 6 + k] = rec[k];
+            const uint32_t qs = block_append(v.query, &c->cache.queries, s_append);
+            if (v.query)
+                for (int k = 0; k < 5; ++k) nrc.queries[(size_t)qs * 5 + k] = v.rec[k];
+            const uint32_t rs = block_append(v.row, &c->cache.rows, s_append);
+            if (v.row && rs < nrc.max_rows)
+                for (int k = 0; k < 6; ++k) nrc.pending[(size_t)rs * 6 + k] = v.rec[k];
         }
     }
 }
@@ -333,31 +350,30 @@ void k_pt_shade_nrc(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, in
 }
 
 // query count after the second bounce's shade: the queries inferred on the side stream
-__global__ void k_snapshot_queries(Counters* c) { c->query_early.v = c->query_count.v; }
+__global__ void k_snapshot_queries(Counters* c) { c->query_early.v = c->cache.queries; }
 
 // training rows from the pending rows of finished training paths: target = (final radiance -
 // radiance before the vertex's reflection) / throughput at the vertex (0 where the throughput is 0);
 // also counts the batch's queries and rows
-__global__ __launch_bounds__(kPtBlock) void k_nrc_rows(const float4* __restrict__ pending, Counters* c,
-                                                       uint32_t max_rows, const float4* __restrict__ rad,
-                                                       float4* __restrict__ rows) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t n = min(c->row_count.v, max_rows);
-    if (i == 0) {
-        c->cache_queries += c->query_count.v;
+__device__ __forceinline__ void nrc_rows(uint32_t first, uint32_t stride, const float4* __restrict__ pending, Counters* c,
+                                         uint32_t max_rows, const float4* __restrict__ rad, float4* __restrict__ rows) {
+    const uint32_t n = min(c->cache.rows, max_rows);
+    if (first == 0) {
+        c->cache_queries += c->cache.queries;
         c->cache_rows += n;
     }
-    if (i >= n) return;
-    const float4* r = pending + (size_t)i * 6;
-    const float4 a = r[4], b = r[5];
-    const uint32_t p = __float_as_uint(b.z);
-    const float4 R = rad[p];
-    const float beta[3] = {a.w, b.x, b.y}, snap[3] = {a.x, a.y, a.z}, fin[3] = {R.x, R.y, R.z};
-    float tgt[3];
-    for (int k = 0; k < 3; ++k) tgt[k] = beta[k] > 0.0f ? (fin[k] - snap[k]) / beta[k] : 0.0f;
-    float4* o = rows + (size_t)i * 5;
-    for (int k = 0; k < 4; ++k) o[k] = r[k];
-    o[4] = make_float4(tgt[0], tgt[1], tgt[2], 0.0f);
+    for (uint32_t i = first; i < n; i += stride) {
+        const float4* r = pending + (size_t)i * 6;
+        const float4 a = r[4], b = r[5];
+        const uint32_t p = __float_as_uint(b.z);
+        const float4 R = rad[p];
+        const float beta[3] = {a.w, b.x, b.y}, snap[3] = {a.x, a.y, a.z}, fin[3] = {R.x, R.y, R.z};
+        float tgt[3];
+        for (int k = 0; k < 3; ++k) tgt[k] = beta[k] > 0.0f ? (fin[k] - snap[k]) / beta[k] : 0.0f;
+        float4* o = rows + (size_t)i * 5;
+        for (int k = 0; k < 4; ++k) o[k] = r[k];
+        o[4] = make_float4(tgt[0], tgt[1], tgt[2], 0.0f);
+    }
 }
 
 // shadow ray i: visible -> radiance of its path += contribution (traceVisibility, :66-73)
@@ -559,13 +575,94 @@ void k_pt_camera(DevScene S, uint32_t n, cupbr_camera cam, uint32_t w, uint32_t 
     });
 }
 
+// Slots of two lists for the lanes of a wave that want one, whose counts are the halves of *counts: one add.
+__device__ __forceinline__ void wave_append2(bool want_lo, bool want_hi, unsigned long long* counts, uint32_t& lo,
+                                             uint32_t& hi) {
+    const unsigned long long ml = __ballot(want_lo), mh = __ballot(want_hi), below = (1ull << __lane_id()) - 1ull;
+    unsigned long long base = 0;
+    if ((ml | mh) != 0ull && __lane_id() == 0u)
+        base = atomicAdd(counts, (unsigned long long)__popcll(mh) << 32 | (unsigned long long)__popcll(ml));
+    lo = __builtin_amdgcn_readfirstlane((uint32_t)base) + (uint32_t)__popcll(ml & below);
+    hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) + (uint32_t)__popcll(mh & below);
+}
+
+// Whole paths of a small batch: the camera rays as packets (camera_packets), then vertex, shadow ray and next ray in
+// turn, in the order of the kernels above, so that a path's radiance is the same sum. per_wave paths a wave; with
+// kFew its last 16 and fewer rays by 8 lanes each (trace_lanes).
+template <bool kNrc, bool kFew, class Seed>
+__global__ __launch_bounds__(kPtBlock)
+void k_pt_paths(DevScene S, uint32_t n, uint32_t per_wave, cupbr_camera cam, uint32_t w, uint32_t h, uint32_t frame0,
+                SampleOrder order, uint32_t train_thresh, uint32_t max_depth, int rr, float4* __restrict__ rad,
+                Counters* c, NrcShade nrc, uint32_t* spill, uint32_t spill_stride) {
+    __shared__ uint32_t lds[kPtLds * kPtBlock];
+    const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
+    LaneStack<kPtLds> st{lds + threadIdx.x, kPtBlock, spill ? spill + gtid : nullptr, spill_stride};
+    const uint32_t blk = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const uint32_t wave_first = (blk * kPtWaves + (threadIdx.x >> 6)) * per_wave;
+    if (wave_first >= n) return;  // whole waves only: traverse_packet needs all 64 lanes
+    const uint32_t p = wave_first + __lane_id();
+    const bool mine = __lane_id() < per_wave && p < n;
+    bool alive = mine;
+    v3 o = splat(0.0f), d = mk(0.0f, 0.0f, 1.0f), w3 = splat(1.0f), L = splat(0.0f);
+    Seed seed{};
+    bool training = false;
+    if (alive) {
+        uint32_t pix, frame;
+        camera_path(cam, w, h, frame0, order, p, seed, pix, frame, o, d);
+        training = is_training_path(pix, frame, train_thresh);
+    }
+    TraceResult r;
+    traverse_packet(S, o, d, alive, r);
+    uint32_t n_ext = alive ? 1u : 0u, n_sh = 0;
+    for (uint32_t bounce = 0;; ++bounce) {
+        Vertex v;
+        v.next = v.shadow = v.query = v.row = false;
+        if (alive) {
+            path_vertex<kNrc, Seed>(S, bounce, max_depth, rr, nrc, o, d, r.t, r.prim, p, training, L, w3, seed, v);
+            if (v.emits) L += v.emission;
+        }
+        if (kNrc) {
+            uint32_t qs, rs;
+            wave_append2(v.query, v.row, &c->cache.both, qs, rs);
+            if (v.query)
+                for (int k = 0; k < 5; ++k) nrc.queries[(size_t)qs * 5 + k] = v.rec[k];
+            if (v.row && rs < nrc.max_rows)
+                for (int k = 0; k < 6; ++k) nrc.pending[(size_t)rs * 6 + k] = v.rec[k];
+        }
+        bool occluded = false;
+        n_sh += v.shadow ? 1u : 0u;
+        if (kFew)
+            occluded = trace_lanes<true>(S, v.shadow, v.shadow_o, v.shadow_d, v.dist, st, r);
+        else if (v.shadow)
+            occluded = traverse<true>(S, v.shadow_o, v.shadow_d, v.dist, st, r);
+        if (v.shadow && !occluded) L += v.light;
+        alive = v.next;
+        if (__ballot(alive) == 0ull) break;
+        n_ext += alive ? 1u : 0u;
+        o = v.next_o;
+        d = v.next_d;
+        if (kFew)
+            trace_lanes<false>(S, alive, o, d, 0.0f, st, r);
+        else if (alive)
+            traverse<false>(S, o, d, 0.0f, st, r);
+    }
+    if (mine) rad[p] = make_float4(L.x, L.y, L.z, __uint_as_float(training ? 1u : 0u));
+    for (int off = 32; off > 0; off >>= 1) {
+        n_ext += __shfl_xor(n_ext, off);
+        n_sh += __shfl_xor(n_sh, off);
+    }
+    if (__lane_id() == 0u) {
+        atomicAdd(&c->extension_rays, (unsigned long long)n_ext);
+        atomicAdd(&c->shadow_rays, (unsigned long long)n_sh);
+    }
+}
+
 // The running mean of PathTracer.cu:162-168 per pixel, frame by frame in order. A pixel's samples
 // are runs of consecutive slots (SampleOrder: up to f frames); a thread loads up to 8 of them at
 // once, so that the 128-byte line they share is fetched once.
-__global__ __launch_bounds__(kPtBlock) void k_accumulate(float* __restrict__ img, const float4* __restrict__ rad,
-                                                         uint32_t w, uint32_t h, SampleOrder order, uint32_t frame0,
-                                                         uint32_t nspp) {
-    const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void accumulate_pixel(uint32_t pix, float* __restrict__ img, const float4* __restrict__ rad,
+                                                 uint32_t w, uint32_t h, SampleOrder order, uint32_t frame0,
+                                                 uint32_t nspp) {
     if (pix >= w * h) return;
     const uint32_t py = pix / w, j = tile_slot(pix - py * w, py, w, h);
     v3 acc = ld3(img + 3 * (size_t)pix);
@@ -594,6 +691,25 @@ __global__ __launch_bounds__(kPtBlock) void k_accumulate(float* __restrict__ img
         s += run;
     }
     st3(img + 3 * (size_t)pix, acc);
+}
+
+__global__ __launch_bounds__(kPtBlock) void k_accumulate(float* __restrict__ img, const float4* __restrict__ rad,
+                                                         uint32_t w, uint32_t h, SampleOrder order, uint32_t frame0,
+                                                         uint32_t nspp) {
+    accumulate_pixel(blockIdx.x * blockDim.x + threadIdx.x, img, rad, w, h, order, frame0, nspp);
+}
+
+// the same with the radiance cache, and the batch's training rows (nrc_rows) in the blocks from pix_blocks on
+__global__ __launch_bounds__(kPtBlock) void k_accumulate_rows(float* __restrict__ img, const float4* __restrict__ rad,
+                                                              uint32_t w, uint32_t h, SampleOrder order, uint32_t frame0,
+                                                              uint32_t nspp, uint32_t pix_blocks,
+                                                              const float4* __restrict__ pending, Counters* c,
+                                                              uint32_t max_rows, float4* __restrict__ rows) {
+    if (blockIdx.x < pix_blocks)
+        accumulate_pixel(blockIdx.x * blockDim.x + threadIdx.x, img, rad, w, h, order, frame0, nspp);
+    else
+        nrc_rows((blockIdx.x - pix_blocks) * blockDim.x + threadIdx.x, (gridDim.x - pix_blocks) * blockDim.x, pending, c,
+                 max_rows, rad, rows);
 }
 
 // ------------------------------------------------------------------ gradient-domain paths
@@ -1092,6 +1208,16 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
                      : (pcg ? k_pt_shade<Pcg32> : k_pt_shade<uint32_t>);
     auto raygen = pcg ? k_pt_raygen<Pcg32> : k_pt_raygen<uint32_t>;
     auto camera = pcg ? k_pt_camera<Pcg32> : k_pt_camera<uint32_t>;
+    const auto packet_blocks = [](uint32_t n) { return ((n + kPtBlock - 1) / kPtBlock + 7u) / 8u * 8u; };
+    // a small batch in one launch (not when the stages of a frame are timed)
+    const uint32_t cus = (uint32_t)device_cu_count();
+    const bool whole = packet && !r->profiling && (size_t)batch * npix <= (size_t)cus * kWholePaths;
+    const bool deep = r->scene->stack_entries > kDeepStack;
+    uint32_t per_wave = 8;
+    while (per_wave < 64u && (size_t)per_wave * cus * (deep ? 16u : 8u) < (size_t)batch * npix) per_wave *= deep ? 2u : 8u;
+    auto paths = nrc ? (pcg ? k_pt_paths<true, true, Pcg32> : k_pt_paths<true, true, uint32_t>)
+                 : per_wave < 64u ? (pcg ? k_pt_paths<false, true, Pcg32> : k_pt_paths<false, true, uint32_t>)
+                                  : (pcg ? k_pt_paths<false, false, Pcg32> : k_pt_paths<false, false, uint32_t>);
     NrcShade ns{nullptr, nullptr, 0, __builtin_inff()};
     uint32_t train_thresh = 0;
     if (nrc) {
@@ -1123,13 +1249,17 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
                                wf.weight.as<float4>(), wf.radiance.as<float4>(), c, train_thresh);
             if ((rc = stage_mark(r, 3))) return rc;
         }
+        if (whole)
+            hipLaunchKernelGGL(paths, dim3(packet_blocks((npath + per_wave - 1) / per_wave * 64u)), dim3(kPtBlock), 0,
+                               r->stream, S, npath, per_wave, cam, w, h,
+                               frame0 + s0, order, train_thresh, r->max_trace_depth, (int)r->russian_roulette,
+                               wf.radiance.as<float4>(), c, ns, spill, grid_threads);
         // per bounce: trace (this bounce's extension rays + the previous bounce's shadow rays), then
         // shade (appends the next extension rays and this bounce's shadow rays, by bounce parity)
-        for (uint32_t b = 0; b <= bounces; ++b) {
+        for (uint32_t b = 0; b <= bounces && !whole; ++b) {
             const int cur = (int)(b & 1);
             if (b == 0 && packet) {
-                const uint32_t nblk = (npath + kPtBlock - 1) / kPtBlock;
-                hipLaunchKernelGGL(camera, dim3((nblk + 7u) / 8u * 8u), dim3(kPtBlock), 0, r->stream, S, npath, cam, w,
+                hipLaunchKernelGGL(camera, dim3(packet_blocks(npath)), dim3(kPtBlock), 0, r->stream, S, npath, cam, w,
                                    h, frame0 + s0, order, train_thresh, wf.q_o[0].as<float4>(), wf.q_d[0].as<float4>(),
                                    wf.weight.as<float4>(), wf.radiance.as<float4>(), wf.q_hit.as<float2>(), c);
             } else {
@@ -1166,7 +1296,7 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
         if (nrc) {
             // throughput * cache for the paths that ended at a cache vertex (those not already
             // inferred on the side stream), then the training rows
-            if ((rc = nrc_infer(r->nrc, r->nrc_queries.as<float>(), npath, &c->query_count.v, 20,
+            if ((rc = nrc_infer(r->nrc, r->nrc_queries.as<float>(), npath, &c->cache.queries, 20,
                                 wf.radiance.as<float>(), true, r->stream,
                                 side_pending ? &c->query_early.v : nullptr)))
                 return rc;
@@ -1174,19 +1304,21 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
                 CUPBR_HIP_CHECK(hipStreamWaitEvent(r->stream, r->ev_side_done, 0));
                 side_pending = false;
             }
-            hipLaunchKernelGGL(k_nrc_rows, dim3((r->nrc_max_rows + kPtBlock - 1) / kPtBlock), dim3(kPtBlock), 0,
-                               r->stream, r->nrc_pending.as<float4>(), c, r->nrc_max_rows, wf.radiance.as<float4>(),
-                               r->nrc_rows.as<float4>());
             if ((rc = stage_mark(r, 3))) return rc;
+            const uint32_t pix_blocks = (npix + kPtBlock - 1) / kPtBlock;
+            hipLaunchKernelGGL(k_accumulate_rows, dim3(pix_blocks + (uint32_t)device_cu_count()), dim3(kPtBlock), 0,
+                               r->stream, img, wf.radiance.as<float4>(), w, h, order, frame0 + s0, nb, pix_blocks,
+                               r->nrc_pending.as<float4>(), c, r->nrc_max_rows, r->nrc_rows.as<float4>());
+        } else {
+            hipLaunchKernelGGL(k_accumulate, dim3((npix + kPtBlock - 1) / kPtBlock), dim3(kPtBlock), 0, r->stream, img,
+                               wf.radiance.as<float4>(), w, h, order, frame0 + s0, nb);
         }
-        hipLaunchKernelGGL(k_accumulate, dim3((npix + kPtBlock - 1) / kPtBlock), dim3(kPtBlock), 0, r->stream, img,
-                           wf.radiance.as<float4>(), w, h, order, frame0 + s0, nb);
         if ((rc = stage_mark(r, 3))) return rc;
         // the row count stays on the device: a batch without training rows takes no steps (Cornell box,
         // 256x256, 1 spp and 4 steps: 0.83 -> 0.80 ms without the copy to the host and the wait for it)
         if (nrc && train_thresh != 0u && r->nrc_steps > 0) {
             if ((rc = nrc_train(r->nrc, r->nrc_rows.as<float>(), r->nrc_max_rows, r->nrc_batch, r->nrc_steps, r->nrc_lr,
-                                nullptr, r->stream, &c->row_count.v)))
+                                nullptr, r->stream, &c->cache.rows)))
                 return rc;
         }
         if (nrc && (rc = stage_mark(r, 3))) return rc;

@@ -25,9 +25,13 @@ struct Counters {
     CounterLine shadow_count[2]; // shadow queues (bounce parity)
     CounterLine work[8];         // trace kernel: extension rays handed out beyond the dealt pieces, per XCD
     CounterLine swork[8];        // trace kernel: shadow rays handed out beyond the dealt pieces, per XCD
-    CounterLine query_count;  // radiance-cache queries of the batch
+    union alignas(128) {
+        struct {
+            uint32_t queries, rows;  // radiance-cache queries and training rows of the batch
+        };
+        unsigned long long both;
+    } cache;
     CounterLine query_early;  // queries that existed after the second bounce's shade
-    CounterLine row_count;    // radiance-cache training rows of the batch
     CounterLine iqueue_count[2];  // volume renderer: rays inside an object (bounce parity)
     unsigned long long extension_rays;
     unsigned long long shadow_rays;

@@ -515,6 +515,47 @@ __device__ __forceinline__ bool trace_group(const DevScene& S, v3 o, v3 d, float
     return traverse_group<kAny, kGroup, kCapacity>(S, o, d, dist, valid && !(kAny && any), reserve, stack, best) || (kAny && any);
 }
 
+// traverse for the active lanes of a wave (all of which call it), each with its own ray: one lane per ray, or 8 lanes
+// each for the last rays (up to 16) of a wave whose other paths have ended.
+template <bool kAny, int kLds>
+__device__ __forceinline__ bool trace_lanes(const DevScene& S, bool active, v3 o, v3 d, float dist, LaneStack<kLds>& st,
+                                            TraceResult& r) {
+    constexpr uint32_t kGroup = 8, kRays = 64 / kGroup, kWords = kLds * kGroup;
+    const unsigned long long m = __ballot(active);
+    const uint32_t n = (uint32_t)__popcll(m), lane = __lane_id();
+    bool any = false;
+    if (n > 16u || S.stack_reserve >= kWords) {
+        if (active) any = traverse<kAny>(S, o, d, dist, st, r);
+        return any;
+    }
+    // lane k gets the number of the k-th active lane
+    const uint32_t rank = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+    const int ids = __builtin_amdgcn_ds_permute((int)(active ? rank : n + lane - rank) * 4, (int)lane);
+    for (uint32_t first = 0; first < n; first += kRays) {
+        const uint32_t k = first + lane / kGroup;
+        const int src = __shfl(ids, (int)min(k, 63u));
+        const auto from = [&](float x) { return __shfl(x, src); };
+        const v3 go = mk(from(o.x), from(o.y), from(o.z)), gd = mk(from(d.x), from(d.y), from(d.z));
+        const float gdist = from(dist);
+        uint32_t* words = st.lds - lane;  // the wave's stack words: row by row, 64 each
+        const uint32_t row = st.lds_stride, base = lane / kGroup * kWords;
+        TraceResult best;
+        const bool hit = trace_group<kAny, kGroup, kWords>(
+            S, go, gd, gdist, k < n, S.stack_reserve,
+            [&](uint32_t e) -> uint32_t& { return words[((base + e) >> 6) * row + ((base + e) & 63u)]; }, best);
+        const int back = (int)((rank % kRays) * kGroup);
+        const bool mine = active && rank / kRays * kRays == first;
+        if (kAny) {
+            const bool h = __shfl((int)hit, back) != 0;
+            any = mine ? h : any;
+        } else {
+            const TraceResult b{__shfl(best.t, back), (uint32_t)__shfl((int)best.prim, back), (uint32_t)__shfl((int)best.rank, back)};
+            if (mine) r = b;
+        }
+    }
+    return any;
+}
+
 // Lanes of the refill loop that must be at a leaf before a wave runs a leaf step (inner-node steps
 // otherwise), at most: a wave runs its leaf step once half of its rays wait at a leaf, capped at
 // this many lanes. 32 (always half) measured best with the half rule (1080p, 1M triangles: cap 12

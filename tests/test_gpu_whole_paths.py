@@ -1,0 +1,65 @@
+"""Small path-tracer batches, traced in one launch, equal the wavefront queues bit for bit.
+
+A batch of up to 1024 paths per CU (262,144 on 256 CUs) runs each path in registers, 64 paths a wave or, in small
+batches and deep trees, 8 to 32 with several lanes per ray. Timing a frame's stages keeps the queues; both add the
+same terms to a path in the same order.
+"""
+import numpy as np
+import pytest
+
+import cupbr_amd as cb
+from cupbr_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+SCENES = {
+    "cornell": lambda: scenes.cornell_box(),
+    "mixed": lambda: scenes.mixed_primitives(env=True),
+    "boxes": lambda: scenes.million_triangles(n_spheres=2, subdiv=4, n_boxes=300),  # a deep tree
+}
+
+
+def _frame(scene, ca, w, h, spp, depth, queues, rr=False, rng=0, cache=None):
+    r = cb.PBRenderer(cb.RenderingMethod.PATHTRACER)
+    r.set_output_size(w, h)
+    r.register_scene(scene)
+    r.set_max_trace_depth(depth)
+    r.set_russian_roulette(rr)
+    r.set_rng(rng)
+    if cache is not None:
+        r.set_radiance_cache(cache, training_paths=w * h // 4, train_steps=0)
+    r.set_profiling(queues)
+    r.render(cb.Camera.look_at(ca["eye"], ca["target"], ca["up"], ca["vfov"], w, h), spp)
+    st = r.stats()
+    return r.get_output_image(), {k: st[k] for k in ("extension_rays", "shadow_rays", "cache_queries", "cache_training_rows")}
+
+
+@pytest.mark.parametrize("name", list(SCENES))
+@pytest.mark.parametrize("w,h,spp,depth,rr,rng", [
+    (1, 1, 1, 5, False, 0), (7, 5, 1, 1, False, 0), (13, 11, 3, 9, True, 0),
+    (128, 128, 1, 4, False, 1),   # the last batch of 8 paths a wave in a shallow tree
+    (113, 145, 1, 6, True, 0),    # the first of 64
+    (256, 257, 1, 5, False, 0), (512, 512, 1, 3, True, 1),  # the largest batch
+    (512, 513, 1, 3, False, 0),   # queues
+])
+def test_whole_paths_equal_queues(name, w, h, spp, depth, rr, rng):
+    desc, ca = SCENES[name]()
+    scene = cb.Scene.from_desc(desc)
+    got, n_got = _frame(scene, ca, w, h, spp, depth, False, rr, rng)
+    want, n_want = _frame(scene, ca, w, h, spp, depth, True, rr, rng)
+    print(f"{name} {w}x{h} {spp} spp depth {depth}: {n_got}", flush=True)
+    assert n_got == n_want and n_got["extension_rays"] >= w * h * spp
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("name", list(SCENES))
+@pytest.mark.parametrize("w,h", [(37, 29), (256, 256), (300, 299)])
+def test_cached_whole_paths_equal_queues(name, w, h):
+    """The same with a radiance cache (without training steps, so that both frames ask the same weights)."""
+    desc, ca = SCENES[name]()
+    scene = cb.Scene.from_desc(desc)
+    cache = cb.RadianceCache((-3, -3, -3), (3, 3, 3), seed=3)
+    got, n_got = _frame(scene, ca, w, h, 2, 6, False, cache=cache)
+    want, n_want = _frame(scene, ca, w, h, 2, 6, True, cache=cache)
+    assert n_got == n_want and n_got["cache_queries"] > 0 and n_got["cache_training_rows"] > 0
+    assert np.array_equal(got, want)
