@@ -39,6 +39,21 @@ int device_cu_count() {
     return cache[dev];
 }
 
+// asked once per device: the call takes 10 us, a twentieth of a small frame
+size_t device_memory() {
+    static std::mutex mu;
+    static std::vector<size_t> cache;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    std::lock_guard<std::mutex> lock(mu);
+    if ((int)cache.size() <= dev) cache.resize(dev + 1, 0);
+    if (cache[dev] == 0) {
+        size_t free_b = 0, total_b = 0;
+        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess) cache[dev] = total_b;
+    }
+    return cache[dev];
+}
+
 int renderer_clear_images(cupbr_renderer* r) {
     // setMethod clears eight of the nine images (PBRenderer.cu:125-134); base is cleared at allocation
     for (int i = 0; i < kNumImages; ++i) {

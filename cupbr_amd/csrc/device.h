@@ -20,6 +20,8 @@ int set_error(int code, const std::string& msg, bool print = false);
 
 // number of compute units of the current device (cached per device)
 int device_cu_count();
+// bytes of memory of the current device, 0 when unknown
+size_t device_memory();
 
 // RAII device buffer that only grows
 struct DevBuf {

@@ -1180,11 +1180,7 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
     // each batch.
     const uint32_t target = 1u << 27;
     uint32_t cap = 1u << 27;
-    {
-        size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && total_b > 0)
-            cap = (uint32_t)std::min<size_t>(cap, std::max<size_t>(total_b / 8 / 200, 1u << 20));
-    }
+    if (const size_t total = device_memory()) cap = (uint32_t)std::min<size_t>(cap, std::max<size_t>(total / 8 / 200, 1u << 20));
     uint32_t batch = std::max<uint32_t>(1, (target + npix - 1) / npix);
     batch = std::min(batch, std::max<uint32_t>(1, cap / npix));
     batch = std::min(batch, spp);
@@ -1332,11 +1328,7 @@ int volume_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t 
     if (npix == 0 || spp == 0) return CUPBR_OK;
     const uint32_t target = 1u << 27;
     uint32_t cap = 1u << 27;
-    {
-        size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && total_b > 0)
-            cap = (uint32_t)std::min<size_t>(cap, std::max<size_t>(total_b / 8 / 264, 1u << 20));
-    }
+    if (const size_t total = device_memory()) cap = (uint32_t)std::min<size_t>(cap, std::max<size_t>(total / 8 / 264, 1u << 20));
     uint32_t batch = std::max<uint32_t>(1, (target + npix - 1) / npix);
     batch = std::min(batch, std::max<uint32_t>(1, cap / npix));
     batch = std::min(batch, spp);
@@ -1415,11 +1407,7 @@ int gdpt_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t fr
     // paths in flight, in whole frames (5 per interior pixel), bounded as in the path tracer
     const uint32_t target = 1u << 27;
     uint32_t cap = 1u << 27;
-    {
-        size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && total_b > 0)
-            cap = (uint32_t)std::min<size_t>(cap, std::max<size_t>(total_b / 8 / 200, 1u << 20));
-    }
+    if (const size_t total = device_memory()) cap = (uint32_t)std::min<size_t>(cap, std::max<size_t>(total / 8 / 200, 1u << 20));
     const uint32_t per_frame = 5u * n_int;
     uint32_t batch = std::max<uint32_t>(1, target / per_frame);
     batch = std::min(batch, std::max<uint32_t>(1, cap / per_frame));
