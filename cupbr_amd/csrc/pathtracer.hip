@@ -42,17 +42,18 @@ constexpr int kPtLds = 16;
 // Batches of up to this many paths per CU run whole paths in one launch (k_pt_paths): as many as are resident at
 // once, 4 waves per SIMD. What bounds a small batch is the longest path's chain of rays and, with a launch and a
 // queue per bounce, the launches; a resident batch needs neither queues nor the path state in memory. Frames of
-// 256x256, 1 spp, depth 5, queues / whole paths (us): Cornell box 189 / 156, mixed primitives 197 / 147, spheres and
-// boxes 819 / 277, 1M triangles 1503 / 761; 512x512: 279 / 241, 261 / 246, 994 / 590, 1623 / 1541. At 331x217,
-// 6 spp (1.6 times the limit) 299 / 300, 360 / 311, 1003 / 738, but 1786 / 2371.
+// 256x256, 1 spp, depth 5, queues / whole paths (us): spheres and boxes 819 / 277, 1M triangles 1503 / 761; 512x512:
+// 994 / 590, 1623 / 1541. At 331x217, 6 spp (1.6 times the limit) 1003 / 738, but 1786 / 2371.
 constexpr uint32_t kWholePaths = 1024;
 // Traversal stack entries (three per BVH4 level) above which a wave of such a batch holds only as many paths (8 to 32)
 // as 16 waves per CU need, so that 8 lanes walk the tree for each: 1M triangles, 64x64, 1 spp, 1310 -> 312 us, 256x256
 // 1318 -> 761. In a shallow tree that pays up to 64 paths per CU only (Cornell box, depth 5: 64x64 158 -> 100 us, but
-// 256x256 156 -> 225).
+// 256x256 156 -> 225); cached frames take 64 paths a wave beyond it, plain ones the queues (kWholeShallow).
 constexpr uint32_t kDeepStack = 24;
-// consecutive rays of a trace queue that belong to one XCD
-constexpr uint32_t kGranule = 1024;
+// The limit of plain frames in a shallow tree. Larger ones would still gain a little (Cornell box, 256x256, 152 -> 139
+// us a frame; mixed primitives 331x217, 6 spp, none), but a cached frame (190 us) would then cost 1.4 plain ones
+// instead of 1.25, and what the cache is for, less error in equal time, needs that to stay well below 1.5.
+constexpr uint32_t kWholeShallow = 64;
 
 // Block-wide append: every thread of the block calls it; lanes with `want` get consecutive
 // slots of the queue whose length is *count (one atomic per block).
@@ -74,6 +75,36 @@ __device__ __forceinline__ uint32_t block_append(bool want, uint32_t* count, uin
     const uint32_t slot = s[kPtWaves] + s[wave] + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
     __syncthreads();
     return slot;
+}
+
+// block_append to two queues together: one 64-bit add for both counts (the low and the high word of
+// *count). s: 2 (kPtWaves + 1) words.
+__device__ __forceinline__ void block_append2(bool want_lo, bool want_hi, unsigned long long* count, uint32_t* s,
+                                              uint32_t& lo, uint32_t& hi) {
+    const unsigned long long me = __ballot(want_lo), ms = __ballot(want_hi);
+    const uint32_t wave = threadIdx.x >> 6, lane = __lane_id();
+    if (lane == 0) {
+        s[2 * wave] = (uint32_t)__popcll(me);
+        s[2 * wave + 1] = (uint32_t)__popcll(ms);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long tot = 0;
+        for (int w = 0; w < kPtWaves; ++w) {
+            const uint32_t e = s[2 * w], h = s[2 * w + 1];
+            s[2 * w] = (uint32_t)tot;
+            s[2 * w + 1] = (uint32_t)(tot >> 32);
+            tot += (unsigned long long)h << 32 | e;
+        }
+        const unsigned long long base = tot ? atomicAdd(count, tot) : 0ull;
+        s[2 * kPtWaves] = (uint32_t)base;
+        s[2 * kPtWaves + 1] = (uint32_t)(base >> 32);
+    }
+    __syncthreads();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    lo = s[2 * kPtWaves] + s[2 * wave] + (uint32_t)__popcll(me & below);
+    hi = s[2 * kPtWaves + 1] + s[2 * wave + 1] + (uint32_t)__popcll(ms & below);
+    __syncthreads();
 }
 
 // adds a wave's traversal counts to two device counters
@@ -130,15 +161,15 @@ __device__ __forceinline__ void camera_path(const cupbr_camera& cam, uint32_t w,
     launch_ray(px, py, w, h, cam, seed, o, d);
 }
 
-// the per-batch counter reset that precedes bounce 0
-__device__ __forceinline__ void reset_batch_counters(Counters* c, uint32_t npath) {
-    c->queue_count[0].v = npath;
-    for (int g = 0; g < 8; ++g) c->work[g].v = c->swork[g].v = 0;
-    c->shadow_count[0].v = 0;
-    c->shadow_count[1].v = 0;
-    c->cache.both = 0;
-    c->iqueue_count[0].v = 0;
-    c->iqueue_count[1].v = 0;
+// the per-batch counter reset that precedes bounce 0 (whose rays are those of parity 1), by threads 0..7
+// of the calling kernel's first block: thread x for XCD x
+__device__ __forceinline__ void reset_batch_counters(Counters* c, XcdQueue order, uint32_t npath, uint32_t x) {
+    c->rays[1][x].ext = order.length(npath, x);
+    c->rays[1][x].shadow = 0;
+    c->rays[0][x].both = 0;
+    c->work[x].v = c->swork[x].v = 0;
+    c->inside[0][x].v = c->inside[1][x].v = 0;
+    if (x == 0) c->cache.both = 0;
 }
 
 // A camera path's state as bounce 0 leaves it: direction and path id (queue 0), throughput 1 and
@@ -158,9 +189,10 @@ template <class Seed>
 __global__ __launch_bounds__(kPtBlock) void k_pt_raygen(cupbr_camera cam, uint32_t w, uint32_t h, uint32_t frame0,
                                                         uint32_t npath, SampleOrder order, float4* __restrict__ q_o,
                                                         float4* __restrict__ q_d, float4* __restrict__ weight,
-                                                        float4* __restrict__ rad, Counters* c, uint32_t train_thresh) {
+                                                        float4* __restrict__ rad, Counters* c, XcdQueue queue,
+                                                        uint32_t train_thresh) {
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p == 0) reset_batch_counters(c, npath);
+    if (p < 8) reset_batch_counters(c, queue, npath, p);
     if (p >= npath) return;  // p: queue slot and path id
     Seed seed;
     uint32_t pix, frame;
@@ -273,18 +305,18 @@ __device__ __forceinline__ void pt_shade(const DevScene& S, int cur, uint32_t bo
                                          const float2* __restrict__ q_hit, float4* __restrict__ nq_o,
                                          float4* __restrict__ nq_d, float4* __restrict__ s_o, float4* __restrict__ s_d,
                                          float4* __restrict__ s_c, float4* __restrict__ weight,
-                                         float4* __restrict__ rad, Counters* c, const NrcShade& nrc,
+                                         float4* __restrict__ rad, Counters* c, XcdQueue queue, const NrcShade& nrc,
                                          uint32_t omask) {
-    __shared__ uint32_t s_append[kPtWaves + 1];
-    const uint32_t n = c->queue_count[cur].v;
+    __shared__ uint32_t s_append[2 * (kPtWaves + 1)];
+    const uint32_t xcd = blockIdx.x & 7u, n = c->rays[cur ^ 1][xcd].ext;
     if (blockIdx.x == 0 && threadIdx.x < 8)  // the next trace starts at 0
         c->work[threadIdx.x].v = c->swork[threadIdx.x].v = 0;
-    for (uint32_t base = blockIdx.x * kPtBlock; base < n; base += gridDim.x * kPtBlock) {
-        const uint32_t i = base + threadIdx.x;
+    for (uint32_t base = (blockIdx.x >> 3) * kPtBlock; base < n; base += (gridDim.x >> 3) * kPtBlock) {
+        const uint32_t i = queue.slot(xcd, base + threadIdx.x);
         Vertex v;
         v.next = v.shadow = v.query = v.row = false;
         uint32_t p = 0;
-        if (i < n) {
+        if (base + threadIdx.x < n) {
             const float4 o4 = q_o[i & omask], d4 = q_d[i];
             const float2 hh = q_hit[i];
             p = __float_as_uint(d4.w);
@@ -301,22 +333,24 @@ __device__ __forceinline__ void pt_shade(const DevScene& S, int cur, uint32_t bo
             }
             if (v.next) weight[p] = make_float4(w3.x, w3.y, w3.z, __uint_as_float(state_bits(seed)));
         }
-        const uint32_t ns = block_append(v.next, &c->queue_count[cur ^ 1].v, s_append);
+        uint32_t ns, ss;
+        block_append2(v.next, v.shadow, &c->rays[cur][xcd].both, s_append, ns, ss);
         if (v.next) {
+            ns = queue.slot(xcd, ns);
             nq_o[ns] = make_float4(v.next_o.x, v.next_o.y, v.next_o.z, 0.0f);
             nq_d[ns] = make_float4(v.next_d.x, v.next_d.y, v.next_d.z, __uint_as_float(p));
         }
-        const uint32_t ss = block_append(v.shadow, &c->shadow_count[cur].v, s_append);
         if (v.shadow) {
+            ss = queue.slot(xcd, ss);
             s_o[ss] = make_float4(v.shadow_o.x, v.shadow_o.y, v.shadow_o.z, v.dist);
             s_d[ss] = make_float4(v.shadow_d.x, v.shadow_d.y, v.shadow_d.z, __uint_as_float(p));
             s_c[ss] = make_float4(v.light.x, v.light.y, v.light.z, 0.0f);
         }
         if (kNrc) {
-            const uint32_t qs = block_append(v.query, &c->cache.queries, s_append);
+            uint32_t qs, rs;
+            block_append2(v.query, v.row, &c->cache.both, s_append, qs, rs);
             if (v.query)
                 for (int k = 0; k < 5; ++k) nrc.queries[(size_t)qs * 5 + k] = v.rec[k];
-            const uint32_t rs = block_append(v.row, &c->cache.rows, s_append);
             if (v.row && rs < nrc.max_rows)
                 for (int k = 0; k < 6; ++k) nrc.pending[(size_t)rs * 6 + k] = v.rec[k];
         }
@@ -332,9 +366,9 @@ void k_pt_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, int rr
                 const float4* __restrict__ q_d, const float2* __restrict__ q_hit, float4* __restrict__ nq_o,
                 float4* __restrict__ nq_d, float4* __restrict__ s_o, float4* __restrict__ s_d,
                 float4* __restrict__ s_c, float4* __restrict__ weight, float4* __restrict__ rad, Counters* c,
-                NrcShade nrc, uint32_t omask) {
+                XcdQueue queue, NrcShade nrc, uint32_t omask) {
     pt_shade<false, Seed>(S, cur, bounce, max_depth, rr, q_o, q_d, q_hit, nq_o, nq_d, s_o, s_d, s_c, weight, rad, c,
-                          nrc, omask);
+                          queue, nrc, omask);
 }
 
 // Shade with the radiance cache: queries and training rows (NrcShade)
@@ -344,9 +378,9 @@ void k_pt_shade_nrc(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, in
                     const float4* __restrict__ q_d, const float2* __restrict__ q_hit, float4* __restrict__ nq_o,
                     float4* __restrict__ nq_d, float4* __restrict__ s_o, float4* __restrict__ s_d,
                     float4* __restrict__ s_c, float4* __restrict__ weight, float4* __restrict__ rad, Counters* c,
-                    NrcShade nrc, uint32_t omask) {
+                    XcdQueue queue, NrcShade nrc, uint32_t omask) {
     pt_shade<true, Seed>(S, cur, bounce, max_depth, rr, q_o, q_d, q_hit, nq_o, nq_d, s_o, s_d, s_c, weight, rad, c,
-                         nrc, omask);
+                         queue, nrc, omask);
 }
 
 // query count after the second bounce's shade: the queries inferred on the side stream
@@ -388,34 +422,31 @@ __device__ __forceinline__ void shadow_result(bool occluded, const float4 d4, co
     rad[p] = make_float4(L.x, L.y, L.z, R.w);
 }
 
-// A wave's share of one queue of n rays. The queue is cut into granules of kGranule rays, granule k
-// belonging to XCD k % 8 (the blocks b with b % 8 = k % 8), so that the XCDs have equal work without
-// taking rays from each other. An XCD's rays, numbered through its granules, go to its waves in
-// pieces: a wave's first piece is dealt by its index, the next ones come from the XCD's counter.
+// A wave's share of its XCD's len rays of one queue. They go to the XCD's waves in pieces: a wave's first
+// piece is dealt by its index, the next ones come from the XCD's counter.
 // What bounds the handing out is the counters: one 128-byte line serves an add with a return value
 // every 13 ns when only its own XCD uses it, and other XCDs' reads in between hold every add up. With
 // one add per refill of some 40 rays, the 20 M rays of a Cornell box bounce were 0.85 ms of counting
 // in a launch of 1.76 ms; with waves that tried all 8 counters before they ended, a launch took at
 // least 115 us however few rays it had, and one that refilled some 300 us. Hence the XCD's own counter
-// only, and pieces of 64 to 256 rays: as many as leave each of the XCD's waves two more, so that they
-// shrink towards the end. Gradient domain (Cornell box, 512x512, 16 spp) 9.5 -> 7.4 ms, volume
-// renderer (512x512, 16 spp) 3.85 -> 2.63 ms, 1080p / 1M triangles / 64 spp 113.5 -> 109.8 ms. Granules
-// of 256, 4096, 16384 and 65536 rays: 110.0, 109.6, 109.9, 110.6 ms; pieces of up to 64, 512 and 1024
-// rays 3% slower, the same, the same.
+// only (the XCDs' shares of a queue are equal enough), and pieces of 64 to 256 rays: as many as leave
+// each of the XCD's waves two more, so that they shrink towards the end. Gradient domain (Cornell box,
+// 512x512, 16 spp) 9.5 -> 7.4 ms, volume renderer (512x512, 16 spp) 3.85 -> 2.63 ms, 1080p / 1M triangles /
+// 64 spp 113.5 -> 109.8 ms. Pieces of up to 64, 512 and 1024 rays: 3% slower, the same, the same.
 struct RayShare {
+    XcdQueue queue;
     CounterLine* counter;    // the XCD's
-    uint32_t g, waves;       // the XCD and its number of waves
+    uint32_t waves;          // its number of waves
     uint32_t len, dealt;     // its rays, and those of the first pieces
     uint32_t at, end;        // the wave's piece
     __device__ __forceinline__ uint32_t piece(uint32_t left) const {
         return min(max(left / (2u * waves) & ~63u, 64u), 256u);
     }
-    __device__ __forceinline__ void begin(CounterLine* c, uint32_t n) {
-        g = blockIdx.x & 7u;
-        counter = c + g;
+    __device__ __forceinline__ void begin(XcdQueue q, CounterLine* c, uint32_t n) {
+        queue = q;
+        counter = c;
         waves = (gridDim.x >> 3) * kPtWaves;
-        const uint32_t rest = n % (8u * kGranule), mine = rest - min(rest, g * kGranule);
-        len = n / (8u * kGranule) * kGranule + min(mine, kGranule);
+        len = n;
         const uint32_t size = piece(len);
         dealt = min(size * waves, len);
         at = __builtin_amdgcn_readfirstlane(min(((blockIdx.x >> 3) * kPtWaves + (threadIdx.x >> 6)) * size, len));
@@ -431,16 +462,15 @@ struct RayShare {
         end = min(at + size, len);
         return at < len;
     }
-    // the queue index of the XCD's ray r < len
-    __device__ __forceinline__ uint32_t index(uint32_t r) const { return (r / kGranule * 8u + g) * kGranule + r % kGranule; }
+    __device__ __forceinline__ uint32_t index(uint32_t k) const { return queue.slot(blockIdx.x & 7u, k); }
 };
 
-// One queue of the trace kernel, n rays, dealt out by RayShare; finish(i, hit, r) consumes the result of ray i.
+// An XCD's n rays of one queue, dealt out by RayShare; finish(i, hit, r) consumes the result of the ray in slot i.
 template <bool kAny, class Load, class Finish>
-__device__ __forceinline__ void trace_queue(const DevScene& S, uint32_t n, CounterLine* counter,
+__device__ __forceinline__ void trace_queue(const DevScene& S, XcdQueue queue, uint32_t n, CounterLine* counter,
                                             LaneStack<kPtLds>& st, Load load, Finish finish) {
     RayShare share;
-    share.begin(counter, n);
+    share.begin(queue, counter, n);
     trace_pool<kAny, true>(S, share, st, load, finish);
 }
 
@@ -454,30 +484,28 @@ template <bool kCount>
 __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(8, 8)))
 void k_pt_trace(DevScene S, int cur, const float4* __restrict__ q_o, const float4* __restrict__ q_d,
                 float2* __restrict__ q_hit, const float4* __restrict__ s_o, const float4* __restrict__ s_d,
-                const float4* __restrict__ s_c, float4* __restrict__ rad, Counters* c, uint32_t* spill,
+                const float4* __restrict__ s_c, float4* __restrict__ rad, Counters* c, XcdQueue queue, uint32_t* spill,
                 uint32_t spill_stride) {
     __shared__ uint32_t lds[kPtLds * kPtBlock];
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t n_ext = c->queue_count[cur].v;
-    const uint32_t n_sh = c->shadow_count[cur ^ 1].v;
-    if (gtid == 0) {
-        c->queue_count[cur ^ 1].v = 0;
-        c->iqueue_count[cur ^ 1].v = 0;
-        c->shadow_count[cur].v = 0;
-        c->extension_rays += n_ext;
-        c->shadow_rays += n_sh;
+    // Workgroups are dispatched to the 8 XCDs round-robin: block b runs on XCD b % 8 (only the speed
+    // depends on it) and traces that XCD's share of the queues
+    const uint32_t xcd = blockIdx.x & 7u;
+    const uint32_t n_ext = c->rays[cur ^ 1][xcd].ext, n_sh = c->rays[cur ^ 1][xcd].shadow;
+    if (gtid < 8) {
+        c->rays[cur][gtid].both = 0;
+        c->inside[cur][gtid].v = 0;
+        atomicAdd(&c->extension_rays, (unsigned long long)c->rays[cur ^ 1][gtid].ext);
+        atomicAdd(&c->shadow_rays, (unsigned long long)c->rays[cur ^ 1][gtid].shadow);
     }
     LaneStack<kPtLds> st{lds + threadIdx.x, kPtBlock, spill ? spill + gtid : nullptr, spill_stride};
     TravCount te, ts;
-    // Workgroups are dispatched to the 8 XCDs round-robin: block b runs on XCD b % 8 (only the speed
-    // depends on it)
-    const uint32_t g0 = blockIdx.x & 7u;
-    // the same decision for every wave (n_ext and n_sh are read at the start)
-    const bool refill = !kCount && n_ext + n_sh >= CUPBR_REFILL_MIN * gridDim.x * kPtBlock;
+    // the same decision for every wave of the XCD (n_ext and n_sh are read at the start)
+    const bool refill = !kCount && n_ext + n_sh >= CUPBR_REFILL_MIN * (gridDim.x >> 3) * kPtBlock;
     if (refill && gtid == 0) c->refill_launches += 1;
     if (refill) {
         trace_queue<false>(
-            S, n_ext, c->work, st,
+            S, queue, n_ext, &c->work[xcd], st,
             [&](uint32_t i, v3& o, v3& d, float& dist) {
                 const float4 o4 = q_o[i], d4 = q_d[i];
                 o = mk(o4.x, o4.y, o4.z);
@@ -486,7 +514,7 @@ void k_pt_trace(DevScene S, int cur, const float4* __restrict__ q_o, const float
             },
             [&](uint32_t i, bool, const TraceResult& r) { q_hit[i] = make_float2(r.t, __uint_as_float(r.prim)); });
         trace_queue<true>(
-            S, n_sh, c->swork, st,
+            S, queue, n_sh, &c->swork[xcd], st,
             [&](uint32_t j, v3& o, v3& d, float& dist) {
                 const float4 o4 = s_o[j], d4 = s_d[j];
                 o = mk(o4.x, o4.y, o4.z);
@@ -496,29 +524,27 @@ void k_pt_trace(DevScene S, int cur, const float4* __restrict__ q_o, const float
             [&](uint32_t j, bool occluded, const TraceResult&) { shadow_result(occluded, s_d[j], s_c, j, rad); });
     } else {
         // 64-ray chunks, one ray per lane until the chunk is done (and the visit-counting pass). The
-        // chunks, extension then shadow, are dealt out by wave: XCD x (blocks b % 8 = x) takes the
-        // x-th eighth of them, its waves one after the other. No counters: a wave has one chunk (in the
-        // visit-counting pass as many as it takes). Cornell box, 256x256, 1 spp: 730 -> 238 us a frame.
-        // Chunks of 32, 16 or 8 rays on more waves gave 247, 249 and 256 us.
+        // XCD's chunks, extension then shadow, go to its waves one after the other. No counters: a wave
+        // has one chunk (in the visit-counting pass as many as it takes). Cornell box, 256x256, 1 spp:
+        // 730 -> 238 us a frame. Chunks of 32, 16 or 8 rays on more waves gave 247, 249 and 256 us.
         const uint32_t e_chunks = (n_ext + 63u) >> 6, chunks = e_chunks + ((n_sh + 63u) >> 6);
-        const uint32_t first = g0 * chunks / 8u, last = (g0 + 1u) * chunks / 8u;
-        const uint32_t waves = (gridDim.x >> 3) * kPtWaves;  // per XCD; gridDim.x is a multiple of 8
-        for (uint32_t q = first + (blockIdx.x >> 3) * kPtWaves + (threadIdx.x >> 6); q < last; q += waves) {
+        const uint32_t waves = (gridDim.x >> 3) * kPtWaves;
+        for (uint32_t q = (blockIdx.x >> 3) * kPtWaves + (threadIdx.x >> 6); q < chunks; q += waves) {
             if (q < e_chunks) {
-                const uint32_t i = (q << 6) + __lane_id();
-                if (i < n_ext) {
+                const uint32_t r = (q << 6) + __lane_id(), i = queue.slot(xcd, r);
+                if (r < n_ext) {
                     const float4 o4 = q_o[i], d4 = q_d[i];
-                    TraceResult r;
-                    traverse<false, kPtLds, kCount>(S, mk(o4.x, o4.y, o4.z), mk(d4.x, d4.y, d4.z), 0.0f, st, r, &te);
-                    q_hit[i] = make_float2(r.t, __uint_as_float(r.prim));
+                    TraceResult hit;
+                    traverse<false, kPtLds, kCount>(S, mk(o4.x, o4.y, o4.z), mk(d4.x, d4.y, d4.z), 0.0f, st, hit, &te);
+                    q_hit[i] = make_float2(hit.t, __uint_as_float(hit.prim));
                 }
             } else {
-                const uint32_t j = ((q - e_chunks) << 6) + __lane_id();
-                if (j < n_sh) {
+                const uint32_t r = ((q - e_chunks) << 6) + __lane_id(), j = queue.slot(xcd, r);
+                if (r < n_sh) {
                     const float4 o4 = s_o[j], d4 = s_d[j];
-                    TraceResult r;
+                    TraceResult hit;
                     const bool occluded = traverse<true, kPtLds, kCount>(S, mk(o4.x, o4.y, o4.z),
-                                                                          mk(d4.x, d4.y, d4.z), o4.w, st, r, &ts);
+                                                                          mk(d4.x, d4.y, d4.z), o4.w, st, hit, &ts);
                     shadow_result(occluded, d4, s_c, j, rad);
                 }
             }
@@ -561,12 +587,10 @@ template <class Seed>
 __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(8, 8)))
 void k_pt_camera(DevScene S, uint32_t n, cupbr_camera cam, uint32_t w, uint32_t h, uint32_t frame0, SampleOrder order,
                  uint32_t train_thresh, float4* __restrict__ q_o, float4* __restrict__ q_d,
-                 float4* __restrict__ weight, float4* __restrict__ rad, float2* __restrict__ q_hit, Counters* c) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        reset_batch_counters(c, n);
-        c->queue_count[1].v = 0;
-        c->extension_rays += n;
-    }
+                 float4* __restrict__ weight, float4* __restrict__ rad, float2* __restrict__ q_hit, Counters* c,
+                 XcdQueue queue) {
+    if (blockIdx.x == 0 && threadIdx.x < 8) reset_batch_counters(c, queue, n, threadIdx.x);
+    if (blockIdx.x == 0 && threadIdx.x == 0) c->extension_rays += n;
     camera_packets(S, n, q_o, q_hit, [&](uint32_t i, v3& o, v3& d) {
         Seed seed;
         uint32_t pix, frame;
@@ -743,22 +767,14 @@ __device__ __forceinline__ void gdpt_camera_path(const cupbr_camera& cam, uint32
     launch_ray(nx, ny, w, h, cam, chain, o, d);
 }
 
-// the GDPT batch's counter reset that precedes bounce 0
-__device__ __forceinline__ void reset_gdpt_counters(Counters* c, uint32_t npath) {
-    c->queue_count[0].v = npath;
-    for (int k = 0; k < 8; ++k) c->work[k].v = c->swork[k].v = 0;
-    c->shadow_count[0].v = 0;
-    c->shadow_count[1].v = 0;
-}
-
 __global__ __launch_bounds__(kPtBlock) void k_gdpt_raygen(cupbr_camera cam, uint32_t w, uint32_t h, uint32_t frame0,
                                                           uint32_t n_int, uint32_t n_groups, float4* __restrict__ q_o,
                                                           float4* __restrict__ q_d, float4* __restrict__ weight,
                                                           float4* __restrict__ rad, uint32_t* __restrict__ slot0,
-                                                          Counters* c) {
+                                                          Counters* c, XcdQueue queue) {
     // one thread per path, so that the queue and state writes of a wave are contiguous
     const uint32_t pid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (pid == 0) reset_gdpt_counters(c, 5u * n_groups);
+    if (pid < 8) reset_batch_counters(c, queue, 5u * n_groups, pid);
     if (pid >= 5u * n_groups) return;
     uint32_t chain;
     v3 o, d;
@@ -775,13 +791,10 @@ __global__ __launch_bounds__(kPtBlock) void k_gdpt_raygen(cupbr_camera cam, uint
 __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(8, 8)))
 void k_gdpt_camera(DevScene S, uint32_t n, cupbr_camera cam, uint32_t w, uint32_t h, uint32_t frame0, uint32_t n_int,
                    float4* __restrict__ q_o, float4* __restrict__ q_d, float4* __restrict__ weight,
-                   float4* __restrict__ rad, uint32_t* __restrict__ slot0, float2* __restrict__ q_hit, Counters* c) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        reset_gdpt_counters(c, n);
-        c->queue_count[1].v = 0;
-        c->iqueue_count[1].v = 0;
-        c->extension_rays += n;
-    }
+                   float4* __restrict__ rad, uint32_t* __restrict__ slot0, float2* __restrict__ q_hit, Counters* c,
+                   XcdQueue queue) {
+    if (blockIdx.x == 0 && threadIdx.x < 8) reset_batch_counters(c, queue, n, threadIdx.x);
+    if (blockIdx.x == 0 && threadIdx.x == 0) c->extension_rays += n;
     camera_packets(S, n, q_o, q_hit, [&](uint32_t i, v3& o, v3& d) {
         uint32_t chain;
         gdpt_camera_path(cam, w, h, frame0, n_int, i, chain, o, d);
@@ -800,16 +813,17 @@ void k_gdpt_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, cons
                   const float4* __restrict__ q_d, const float2* __restrict__ q_hit, float4* __restrict__ nq_o,
                   float4* __restrict__ nq_d, float4* __restrict__ s_o, float4* __restrict__ s_d,
                   float4* __restrict__ s_c, float4* __restrict__ weight, float4* __restrict__ rad, Counters* c,
-                  const uint32_t* __restrict__ slot_now, uint32_t* __restrict__ slot_next, uint32_t omask) {
-    __shared__ uint32_t s_append[kPtWaves + 1];
-    const uint32_t n = c->queue_count[cur].v;
+                  XcdQueue queue, const uint32_t* __restrict__ slot_now, uint32_t* __restrict__ slot_next,
+                  uint32_t omask) {
+    __shared__ uint32_t s_append[2 * (kPtWaves + 1)];
+    const uint32_t xcd = blockIdx.x & 7u, n = c->rays[cur ^ 1][xcd].ext;
     if (blockIdx.x == 0 && threadIdx.x < 8) c->work[threadIdx.x].v = c->swork[threadIdx.x].v = 0;
     const float nl = (float)(S.n_lights + (S.use_env ? 1u : 0u));
-    for (uint32_t base = blockIdx.x * kPtBlock; base < n; base += gridDim.x * kPtBlock) {
-        const uint32_t i = base + threadIdx.x;
+    for (uint32_t base = (blockIdx.x >> 3) * kPtBlock; base < n; base += (gridDim.x >> 3) * kPtBlock) {
+        const uint32_t i = queue.slot(xcd, base + threadIdx.x);
         bool want_next = false, want_shadow = false;
         float4 no = {}, nd = {}, so = {}, sd = {}, sc = {};
-        if (i < n) {
+        if (base + threadIdx.x < n) {
             const float4 o4 = q_o[i & omask], d4 = q_d[i];
             const float2 hh = q_hit[i];
             const uint32_t p = __float_as_uint(d4.w);
@@ -873,16 +887,18 @@ void k_gdpt_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, cons
             }
             if (k == 0) slot_next[g] = kNoSlot;  // overwritten below when the base path goes on
         }
-        const uint32_t ns = block_append(want_next, &c->queue_count[cur ^ 1].v, s_append);
+        uint32_t ns, ss;
+        block_append2(want_next, want_shadow, &c->rays[cur][xcd].both, s_append, ns, ss);
         if (want_next) {
+            ns = queue.slot(xcd, ns);
             nq_o[ns] = no;
             nq_d[ns] = nd;
             const uint32_t p = __float_as_uint(nd.w);
             const uint32_t g = p / 5u;
             if (p == 5u * g) slot_next[g] = ns;
         }
-        const uint32_t ss = block_append(want_shadow, &c->shadow_count[cur].v, s_append);
         if (want_shadow) {
+            ss = queue.slot(xcd, ss);
             s_o[ss] = so;
             s_d[ss] = sd;
             s_c[ss] = sc;
@@ -944,20 +960,22 @@ void k_vol_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, int r
                  const float4* __restrict__ iq_d, float4* __restrict__ nq_o, float4* __restrict__ nq_d,
                  float4* __restrict__ niq_o, float4* __restrict__ niq_d, float4* __restrict__ s_o,
                  float4* __restrict__ s_d, float4* __restrict__ s_c, float4* __restrict__ weight,
-                 float4* __restrict__ rad, Counters* c, uint32_t omask) {
-    __shared__ uint32_t s_append[kPtWaves + 1];
-    const uint32_t n_out = c->queue_count[cur].v, n_in = c->iqueue_count[cur].v, n = n_out + n_in;
+                 float4* __restrict__ rad, Counters* c, XcdQueue queue, uint32_t omask) {
+    __shared__ uint32_t s_append[2 * (kPtWaves + 1)];
+    const uint32_t xcd = blockIdx.x & 7u;
+    const uint32_t n_out = c->rays[cur ^ 1][xcd].ext, n_in = c->inside[cur ^ 1][xcd].v, n = n_out + n_in;
     if (blockIdx.x == 0 && threadIdx.x < 8) c->work[threadIdx.x].v = c->swork[threadIdx.x].v = 0;
     const float nl = (float)(S.n_lights + (S.use_env ? 1u : 0u));
     unsigned long long inside_traces = 0;
-    for (uint32_t base = blockIdx.x * kPtBlock; base < n; base += gridDim.x * kPtBlock) {
-        const uint32_t i = base + threadIdx.x;
+    for (uint32_t base = (blockIdx.x >> 3) * kPtBlock; base < n; base += (gridDim.x >> 3) * kPtBlock) {
+        const uint32_t r = base + threadIdx.x;
+        const bool from_inside = r >= n_out;
+        const uint32_t i = queue.slot(xcd, from_inside ? r - n_out : r);
         bool want_next = false, want_shadow = false, next_inside = false;
         float4 no = {}, nd = {}, so = {}, sd = {}, sc = {};
-        if (i < n) {
-            const bool from_inside = i >= n_out;
-            const float4 o4 = from_inside ? iq_o[i - n_out] : q_o[i & omask];
-            const float4 d4 = from_inside ? iq_d[i - n_out] : q_d[i];
+        if (r < n) {
+            const float4 o4 = from_inside ? iq_o[i] : q_o[i & omask];
+            const float4 d4 = from_inside ? iq_d[i] : q_d[i];
             const uint32_t p = __float_as_uint(d4.w);
             const float4 W = weight[p];
             const float4 R = rad[p];
@@ -1110,18 +1128,21 @@ void k_vol_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, int r
             rad[p] = make_float4(L.x, L.y, L.z, __uint_as_float(vstate));
         }
         const bool app_out = want_next && !next_inside, app_in = want_next && next_inside;
-        const uint32_t ns = block_append(app_out, &c->queue_count[cur ^ 1].v, s_append);
+        uint32_t ns, ss;
+        block_append2(app_out, want_shadow, &c->rays[cur][xcd].both, s_append, ns, ss);
         if (app_out) {
+            ns = queue.slot(xcd, ns);
             nq_o[ns] = no;
             nq_d[ns] = nd;
         }
-        const uint32_t ni = block_append(app_in, &c->iqueue_count[cur ^ 1].v, s_append);
+        uint32_t ni = block_append(app_in, &c->inside[cur][xcd].v, s_append);
         if (app_in) {
+            ni = queue.slot(xcd, ni);
             niq_o[ni] = no;
             niq_d[ni] = nd;
         }
-        const uint32_t ss = block_append(want_shadow, &c->shadow_count[cur].v, s_append);
         if (want_shadow) {
+            ss = queue.slot(xcd, ss);
             s_o[ss] = so;
             s_d[ss] = sd;
             s_c[ss] = sc;
@@ -1159,6 +1180,14 @@ static int ensure_wavefront(cupbr_renderer* r, uint32_t paths, uint32_t grid_thr
     return CUPBR_OK;
 }
 
+// The queues' granules for batches of up to npath paths: 1024 rays, fewer where that would leave an XCD
+// less than 8 of them (small images keep all XCDs busy)
+static XcdQueue xcd_queue(uint32_t npath) {
+    uint32_t lg = 10;
+    while (lg > 6u && (npath >> lg) < 64u) --lg;
+    return XcdQueue{lg};
+}
+
 // SampleOrder of a batch of nb frames of npix pixels: as many frames per wave as divide nb (a power
 // of two up to 64) while 64 / frames still divides the pixel count
 SampleOrder sample_order(uint32_t npix, uint32_t nb) {
@@ -1186,7 +1215,8 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
     batch = std::min(batch, spp);
     const int blocks = device_cu_count() * 8;
     const uint32_t grid_threads = (uint32_t)blocks * kPtBlock;
-    int rc = ensure_wavefront(r, batch * npix, grid_threads);
+    const XcdQueue queue = xcd_queue(batch * npix);
+    int rc = ensure_wavefront(r, queue.capacity(batch * npix), grid_threads);
     if (rc) return rc;
     Wavefront& wf = r->wf;
     Counters* c = wf.counters.as<Counters>();
@@ -1207,8 +1237,9 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
     const auto packet_blocks = [](uint32_t n) { return ((n + kPtBlock - 1) / kPtBlock + 7u) / 8u * 8u; };
     // a small batch in one launch (not when the stages of a frame are timed)
     const uint32_t cus = (uint32_t)device_cu_count();
-    const bool whole = packet && !r->profiling && (size_t)batch * npix <= (size_t)cus * kWholePaths;
     const bool deep = r->scene->stack_entries > kDeepStack;
+    const bool whole = packet && !r->profiling &&
+                       (size_t)batch * npix <= (size_t)cus * (deep || nrc ? kWholePaths : kWholeShallow);
     uint32_t per_wave = 8;
     while (per_wave < 64u && (size_t)per_wave * cus * (deep ? 16u : 8u) < (size_t)batch * npix) per_wave *= deep ? 2u : 8u;
     auto paths = nrc ? (pcg ? k_pt_paths<true, true, Pcg32> : k_pt_paths<true, true, uint32_t>)
@@ -1242,7 +1273,7 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
         if (!packet) {
             hipLaunchKernelGGL(raygen, dim3((npath + kPtBlock - 1) / kPtBlock), dim3(kPtBlock), 0, r->stream, cam, w,
                                h, frame0 + s0, npath, order, wf.q_o[0].as<float4>(), wf.q_d[0].as<float4>(),
-                               wf.weight.as<float4>(), wf.radiance.as<float4>(), c, train_thresh);
+                               wf.weight.as<float4>(), wf.radiance.as<float4>(), c, queue, train_thresh);
             if ((rc = stage_mark(r, 3))) return rc;
         }
         if (whole)
@@ -1257,12 +1288,12 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
             if (b == 0 && packet) {
                 hipLaunchKernelGGL(camera, dim3(packet_blocks(npath)), dim3(kPtBlock), 0, r->stream, S, npath, cam, w,
                                    h, frame0 + s0, order, train_thresh, wf.q_o[0].as<float4>(), wf.q_d[0].as<float4>(),
-                                   wf.weight.as<float4>(), wf.radiance.as<float4>(), wf.q_hit.as<float2>(), c);
+                                   wf.weight.as<float4>(), wf.radiance.as<float4>(), wf.q_hit.as<float2>(), c, queue);
             } else {
                 hipLaunchKernelGGL(trace, dim3(blocks), dim3(kPtBlock), 0, r->stream, S, cur, wf.q_o[cur].as<float4>(),
                                    wf.q_d[cur].as<float4>(), wf.q_hit.as<float2>(), wf.s_o[cur ^ 1].as<float4>(),
                                    wf.s_d[cur ^ 1].as<float4>(), wf.s_c[cur ^ 1].as<float4>(),
-                                   wf.radiance.as<float4>(), c, spill, grid_threads);
+                                   wf.radiance.as<float4>(), c, queue, spill, grid_threads);
             }
             if ((rc = stage_mark(r, 0))) return rc;
             if (b == bounces) break;  // the last trace only had the last bounce's shadow rays
@@ -1270,8 +1301,8 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
                                (int)r->russian_roulette, wf.q_o[cur].as<float4>(),
                                wf.q_d[cur].as<float4>(), wf.q_hit.as<float2>(), wf.q_o[cur ^ 1].as<float4>(),
                                wf.q_d[cur ^ 1].as<float4>(), wf.s_o[cur].as<float4>(), wf.s_d[cur].as<float4>(),
-                               wf.s_c[cur].as<float4>(), wf.weight.as<float4>(), wf.radiance.as<float4>(), c, ns,
-                               b == 0 && packet ? 0u : ~0u);
+                               wf.s_c[cur].as<float4>(), wf.weight.as<float4>(), wf.radiance.as<float4>(), c, queue,
+                               ns, b == 0 && packet ? 0u : ~0u);
             if ((rc = stage_mark(r, 1))) return rc;
             if (nrc && b == 1 && bounces > 2 && npath >= kSidePaths) {
                 // The paths that queried the cache so far have no shadow ray left in flight (the
@@ -1282,7 +1313,8 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
                 hipLaunchKernelGGL(k_snapshot_queries, dim3(1), dim3(1), 0, r->stream, c);
                 CUPBR_HIP_CHECK(hipEventRecord(r->ev_queries, r->stream));
                 CUPBR_HIP_CHECK(hipStreamWaitEvent(r->side_stream, r->ev_queries, 0));
-                if ((rc = nrc_infer(r->nrc, r->nrc_queries.as<float>(), npath, &c->query_early.v, 20,
+                if ((rc = nrc_infer(r->nrc, r->nrc_queries.as<float>(), npath,
+                                    &c->query_early.v, 20,
                                     wf.radiance.as<float>(), true, r->side_stream)))
                     return rc;
                 CUPBR_HIP_CHECK(hipEventRecord(r->ev_side_done, r->side_stream));
@@ -1334,15 +1366,16 @@ int volume_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t 
     batch = std::min(batch, spp);
     const int blocks = device_cu_count() * 8;
     const uint32_t grid_threads = (uint32_t)blocks * kPtBlock;
-    int rc = ensure_wavefront(r, batch * npix, grid_threads);
+    const XcdQueue queue = xcd_queue(batch * npix);
+    int rc = ensure_wavefront(r, queue.capacity(batch * npix), grid_threads);
     if (rc) return rc;
     Wavefront& wf = r->wf;
-    if (wf.iq_capacity < batch * npix) {
+    const uint32_t slots = queue.capacity(batch * npix);
+    if (wf.iq_capacity < slots) {
         for (int k = 0; k < 2; ++k) {
-            if ((rc = wf.iq_o[k].ensure((size_t)batch * npix * 16)) || (rc = wf.iq_d[k].ensure((size_t)batch * npix * 16)))
-                return rc;
+            if ((rc = wf.iq_o[k].ensure((size_t)slots * 16)) || (rc = wf.iq_d[k].ensure((size_t)slots * 16))) return rc;
         }
-        wf.iq_capacity = batch * npix;
+        wf.iq_capacity = slots;
     }
     Counters* c = wf.counters.as<Counters>();
     CUPBR_HIP_CHECK(hipMemsetAsync(c, 0, sizeof(Counters), r->stream));
@@ -1363,7 +1396,7 @@ int volume_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t 
         if (!packet) {
             hipLaunchKernelGGL(k_pt_raygen<uint32_t>, dim3((npath + kPtBlock - 1) / kPtBlock), dim3(kPtBlock), 0,
                                r->stream, cam, w, h, frame0 + s0, npath, order, wf.q_o[0].as<float4>(),
-                               wf.q_d[0].as<float4>(), wf.weight.as<float4>(), wf.radiance.as<float4>(), c, 0u);
+                               wf.q_d[0].as<float4>(), wf.weight.as<float4>(), wf.radiance.as<float4>(), c, queue, 0u);
             if ((rc = stage_mark(r, 3))) return rc;
         }
         for (uint32_t b = 0; b <= bounces; ++b) {
@@ -1373,12 +1406,12 @@ int volume_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t 
                 hipLaunchKernelGGL(k_pt_camera<uint32_t>, dim3((nblk + 7u) / 8u * 8u), dim3(kPtBlock), 0, r->stream, S,
                                    npath, cam, w, h, frame0 + s0, order, 0u, wf.q_o[0].as<float4>(),
                                    wf.q_d[0].as<float4>(), wf.weight.as<float4>(), wf.radiance.as<float4>(),
-                                   wf.q_hit.as<float2>(), c);
+                                   wf.q_hit.as<float2>(), c, queue);
             } else {
                 hipLaunchKernelGGL(trace, dim3(blocks), dim3(kPtBlock), 0, r->stream, S, cur, wf.q_o[cur].as<float4>(),
                                    wf.q_d[cur].as<float4>(), wf.q_hit.as<float2>(), wf.s_o[cur ^ 1].as<float4>(),
                                    wf.s_d[cur ^ 1].as<float4>(), wf.s_c[cur ^ 1].as<float4>(),
-                                   wf.radiance.as<float4>(), c, spill, grid_threads);
+                                   wf.radiance.as<float4>(), c, queue, spill, grid_threads);
             }
             if ((rc = stage_mark(r, 0))) return rc;
             if (b == bounces) break;
@@ -1389,7 +1422,7 @@ int volume_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t 
                                wf.q_o[cur ^ 1].as<float4>(), wf.q_d[cur ^ 1].as<float4>(),
                                wf.iq_o[cur ^ 1].as<float4>(), wf.iq_d[cur ^ 1].as<float4>(), wf.s_o[cur].as<float4>(),
                                wf.s_d[cur].as<float4>(), wf.s_c[cur].as<float4>(), wf.weight.as<float4>(),
-                               wf.radiance.as<float4>(), c, b == 0 && packet ? 0u : ~0u);
+                               wf.radiance.as<float4>(), c, queue, b == 0 && packet ? 0u : ~0u);
             if ((rc = stage_mark(r, 1))) return rc;
         }
         hipLaunchKernelGGL(k_accumulate, dim3((npix + kPtBlock - 1) / kPtBlock), dim3(kPtBlock), 0, r->stream, img,
@@ -1414,7 +1447,8 @@ int gdpt_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t fr
     batch = std::min(batch, spp);
     const int blocks = device_cu_count() * 8;
     const uint32_t grid_threads = (uint32_t)blocks * kPtBlock;
-    int rc = ensure_wavefront(r, batch * per_frame, grid_threads);
+    const XcdQueue queue = xcd_queue(batch * per_frame);
+    int rc = ensure_wavefront(r, queue.capacity(batch * per_frame), grid_threads);
     if (rc) return rc;
     Wavefront& wf = r->wf;
     if ((rc = wf.gdpt_slot.ensure((size_t)2 * batch * n_int * sizeof(uint32_t)))) return rc;
@@ -1435,7 +1469,7 @@ int gdpt_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t fr
         if (!packet) {  // with camera packets the camera trace makes the rays (k_gdpt_camera)
             hipLaunchKernelGGL(k_gdpt_raygen, dim3((npath + kPtBlock - 1) / kPtBlock), dim3(kPtBlock), 0, r->stream,
                                cam, w, h, frame0 + s0, n_int, groups, wf.q_o[0].as<float4>(), wf.q_d[0].as<float4>(),
-                               wf.weight.as<float4>(), wf.radiance.as<float4>(), slots[0], c);
+                               wf.weight.as<float4>(), wf.radiance.as<float4>(), slots[0], c, queue);
             if ((rc = stage_mark(r, 3))) return rc;
         }
         for (uint32_t b = 0; b <= bounces; ++b) {
@@ -1445,12 +1479,12 @@ int gdpt_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t fr
                 hipLaunchKernelGGL(k_gdpt_camera, dim3((nblk + 7u) / 8u * 8u), dim3(kPtBlock), 0, r->stream, S, npath,
                                    cam, w, h, frame0 + s0, n_int, wf.q_o[0].as<float4>(), wf.q_d[0].as<float4>(),
                                    wf.weight.as<float4>(),
-                                   wf.radiance.as<float4>(), slots[0], wf.q_hit.as<float2>(), c);
+                                   wf.radiance.as<float4>(), slots[0], wf.q_hit.as<float2>(), c, queue);
             } else {
                 hipLaunchKernelGGL(trace, dim3(blocks), dim3(kPtBlock), 0, r->stream, S, cur, wf.q_o[cur].as<float4>(),
                                    wf.q_d[cur].as<float4>(), wf.q_hit.as<float2>(), wf.s_o[cur ^ 1].as<float4>(),
                                    wf.s_d[cur ^ 1].as<float4>(), wf.s_c[cur ^ 1].as<float4>(),
-                                   wf.radiance.as<float4>(), c, spill, grid_threads);
+                                   wf.radiance.as<float4>(), c, queue, spill, grid_threads);
             }
             if ((rc = stage_mark(r, 0))) return rc;
             if (b == bounces) break;
@@ -1458,7 +1492,7 @@ int gdpt_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t fr
                                wf.q_o[cur].as<float4>(), wf.q_d[cur].as<float4>(),
                                wf.q_hit.as<float2>(), wf.q_o[cur ^ 1].as<float4>(), wf.q_d[cur ^ 1].as<float4>(),
                                wf.s_o[cur].as<float4>(), wf.s_d[cur].as<float4>(), wf.s_c[cur].as<float4>(),
-                               wf.weight.as<float4>(), wf.radiance.as<float4>(), c, slots[b & 1],
+                               wf.weight.as<float4>(), wf.radiance.as<float4>(), c, queue, slots[b & 1],
                                slots[(b + 1) & 1], b == 0 && packet ? 0u : ~0u);
             if ((rc = stage_mark(r, 1))) return rc;
         }
