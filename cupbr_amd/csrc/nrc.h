@@ -21,12 +21,12 @@ struct NrcBox {
 
 struct cupbr_nrc {
     cupbr::NrcBox box{};
-    cupbr::DevBuf w, m, v;                   // FP32 weights and Adam moments
+    cupbr::DevBuf w, moments;                // FP32 weights; Adam's two moments, then the step numbers (TrainState)
     cupbr::DevBuf packed_fwd, packed_bwd;    // BF16 matrix-core fragments of W and W^T
     cupbr::DevBuf acts, losses, sums;        // training scratch: activations and gradients, per-block losses,
                                              // weight-gradient sums per slice of the batch
-    cupbr::DevBuf state, bias;               // step numbers; Adam's bias corrections by step
-    float beta1 = 0.9f, beta2 = 0.99f, eps = 1e-10f;
+    cupbr::DevBuf bias;                      // Adam's bias corrections by step
+    static constexpr float beta1 = 0.9f, beta2 = 0.99f, eps = 1e-10f;
 };
 
 namespace cupbr {

@@ -565,9 +565,7 @@ int nrc_init_weights(cupbr_nrc* c, uint32_t seed) {
 
 int nrc_set_weights(cupbr_nrc* c, const float* host) {
     CUPBR_HIP_CHECK(hipMemcpy(c->w.ptr, host, kNrcParams * 4, hipMemcpyHostToDevice));
-    CUPBR_HIP_CHECK(hipMemset(c->m.ptr, 0, kNrcParams * 4));
-    CUPBR_HIP_CHECK(hipMemset(c->v.ptr, 0, kNrcParams * 4));
-    CUPBR_HIP_CHECK(hipMemset(c->state.ptr, 0, sizeof(TrainState)));
+    CUPBR_HIP_CHECK(hipMemset(c->moments.ptr, 0, 2 * kNrcParams * 4 + sizeof(TrainState)));
     return nrc_pack(c, nullptr);
 }
 
@@ -586,9 +584,9 @@ int nrc_create(const float lo[3], const float hi[3], uint32_t seed, cupbr_nrc** 
         c->box.inv_ext[a] = e > 0.0f ? 1.0f / e : 1.0f;
     }
     int rc;
-    if ((rc = c->w.ensure(kNrcParams * 4)) || (rc = c->m.ensure(kNrcParams * 4)) || (rc = c->v.ensure(kNrcParams * 4)) ||
+    if ((rc = c->w.ensure(kNrcParams * 4)) || (rc = c->moments.ensure(2 * kNrcParams * 4 + sizeof(TrainState))) ||
         (rc = c->packed_fwd.ensure(kFwdSize * 2)) || (rc = c->packed_bwd.ensure(kBwdSize * 2)) ||
-        (rc = c->state.ensure(sizeof(TrainState))) || (rc = c->bias.ensure(kBiasSteps * sizeof(float2)))) {
+        (rc = c->bias.ensure(kBiasSteps * sizeof(float2)))) {
         delete c;
         return rc;
     }
@@ -598,10 +596,13 @@ int nrc_create(const float lo[3], const float hi[3], uint32_t seed, cupbr_nrc** 
         delete c;
         return set_error(CUPBR_ERR_HIP, "hipMemset failed");
     }
-    // Adam's bias corrections, one pair per step number
-    std::vector<float2> bias(kBiasSteps);
-    for (uint32_t k = 0; k < kBiasSteps; ++k)
-        bias[k] = make_float2(1.0f - std::pow(c->beta1, (float)k), 1.0f - std::pow(c->beta2, (float)k));
+    // Adam's bias corrections, one pair per step number (every cache has the same betas)
+    static const std::vector<float2> bias = [](float b1, float b2) {
+        std::vector<float2> t(kBiasSteps);
+        for (uint32_t k = 0; k < kBiasSteps; ++k)
+            t[k] = make_float2(1.0f - std::pow(b1, (float)k), 1.0f - std::pow(b2, (float)k));
+        return t;
+    }(c->beta1, c->beta2);
     if (hipMemcpy(c->bias.ptr, bias.data(), kBiasSteps * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess) {
         delete c;
         return set_error(CUPBR_ERR_HIP, "hipMemcpy failed");
@@ -641,7 +642,8 @@ int nrc_train(cupbr_nrc* c, const float* rows, uint32_t n_rows, uint32_t batch, 
         (rc = c->sums.ensure((size_t)kWeightTiles * (batch / kSlice) * 1024)))
         return rc;
     const uint32_t sum_blocks = groups * 8 * (kWeightTiles / 4);
-    TrainState* state = c->state.as<TrainState>();
+    float *m = c->moments.as<float>(), *v = m + kNrcParams;
+    TrainState* state = reinterpret_cast<TrainState*>(v + kNrcParams);
     for (uint32_t s = 0; s < steps; ++s) {
         hipLaunchKernelGGL(k_nrc_train, dim3(blocks), dim3(kNrcBlock), 0, stream, c->packed_fwd.as<bf16x8>(),
                            c->packed_bwd.as<bf16x8>(), c->box, rows, n_rows, n_rows_dev, batch, state, s,
@@ -651,8 +653,7 @@ int nrc_train(cupbr_nrc* c, const float* rows, uint32_t n_rows, uint32_t batch, 
                            c->sums.as<f32x4>(), n_rows, n_rows_dev);
         CUPBR_HIP_CHECK(hipGetLastError());
         hipLaunchKernelGGL(k_nrc_adam, dim3(kWeightTiles + 1), dim3(kNrcBlock), 0, stream, c->sums.as<f32x4>(), n_slices,
-                           c->losses.as<float>(), blocks, 1.0f / (float)batch, c->w.as<float>(), c->m.as<float>(),
-                           c->v.as<float>(), lr, c->beta1, c->beta2, c->eps, c->bias.as<float2>(), n_rows, n_rows_dev,
+                           c->losses.as<float>(), blocks, 1.0f / (float)batch, c->w.as<float>(), m, v, lr, c->beta1, c->beta2, c->eps, c->bias.as<float2>(), n_rows, n_rows_dev,
                            state, s + 1 == steps ? steps : 0u, loss_dev ? loss_dev + s : nullptr,
                            c->packed_fwd.as<__bf16>(), c->packed_bwd.as<__bf16>());
         CUPBR_HIP_CHECK(hipGetLastError());
