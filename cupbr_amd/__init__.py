@@ -297,7 +297,7 @@ def measure_valu_peak(iterations: int = 20000) -> dict:
 
 def measure_atomic_peak(iterations: int = 256, words_per_copy: int = 64 ** 3) -> dict:
     """cupbr_measure_atomic_peak: time and count of FP32 atomic adds (no return) to pseudo-random
-    words of 8 per-XCD copies of words_per_copy floats (the grid adjoint's gradient layout)."""
+    words of 8 per-XCD copies of words_per_copy floats: the rate of atomic requests."""
     ms = C.c_double()
     n = C.c_uint64()
     _check(lib().cupbr_measure_atomic_peak(iterations, words_per_copy, C.byref(ms), C.byref(n)))

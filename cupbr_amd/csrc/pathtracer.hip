@@ -835,14 +835,15 @@ void k_gdpt_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, cons
             }
             if (go) {
                 const float4 W = weight[p];
-                const float4 R = rad[p];
                 v3 w3 = mk(W.x, W.y, W.z);
                 uint32_t seed = __float_as_uint(W.w);
-                v3 L = mk(R.x, R.y, R.z);
+                // most vertices add none, and their radiance is neither read nor written; a throughput is written for
+                // paths that go on (512x512, 16 spp: 6.95 -> 6.67 ms; volume renderer 2.58 -> 2.53)
+                v3 emission = splat(0.0f);
                 const v3 o = mk(o4.x, o4.y, o4.z), d = mk(d4.x, d4.y, d4.z);
                 const uint32_t prim = __float_as_uint(hh.y);
                 if (prim == kNoHit) {  // :128-137
-                    if (S.use_env) L += w3 * env_lookup(S, d);
+                    if (S.use_env) emission = w3 * env_lookup(S, d);
                 } else {
                     const v3 P = o + hh.x * d;
                     v3 N;
@@ -850,7 +851,7 @@ void k_gdpt_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, cons
                     hit_geometry(S, prim, P, N, obj);
                     const Mat m = load_mat(S.mats + obj);
                     const v3 inc = -1.0f * d;
-                    L += w3 * m.albedo_e;  // emissiveIllumintationGDPT :39-44
+                    emission = w3 * m.albedo_e;  // emissiveIllumintationGDPT :39-44
                     if (m.type != CUPBR_GLASS && dot(N, inc) <= 0.0f) {  // directIlluminationGDPT :46-88
                         w3 = splat(0.0f);
                     } else {
@@ -881,9 +882,12 @@ void k_gdpt_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, cons
                             nd = make_float4(ndir.x, ndir.y, ndir.z, __uint_as_float(p));
                         }
                     }
-                    weight[p] = make_float4(w3.x, w3.y, w3.z, __uint_as_float(seed));
+                    if (want_next) weight[p] = make_float4(w3.x, w3.y, w3.z, __uint_as_float(seed));
                 }
-                rad[p] = make_float4(L.x, L.y, L.z, R.w);
+                if (!(emission.x == 0.0f && emission.y == 0.0f && emission.z == 0.0f)) {
+                    const float4 R = rad[p];
+                    rad[p] = make_float4(R.x + emission.x, R.y + emission.y, R.z + emission.z, R.w);
+                }
             }
             if (k == 0) slot_next[g] = kNoSlot;  // overwritten below when the base path goes on
         }
@@ -981,8 +985,8 @@ void k_vol_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, int r
             const float4 R = rad[p];
             v3 w3 = mk(W.x, W.y, W.z);
             uint32_t seed = __float_as_uint(W.w);
-            v3 L = mk(R.x, R.y, R.z);
-            uint32_t vstate = __float_as_uint(R.w);
+            v3 emission = splat(0.0f);
+            const uint32_t vstate = __float_as_uint(R.w);
             bool inside = (vstate & kInsideBit) != 0u;
             uint32_t obj_index = vstate & ~kInsideBit;
             const v3 o = mk(o4.x, o4.y, o4.z), d = mk(d4.x, d4.y, d4.z);
@@ -997,7 +1001,7 @@ void k_vol_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, int r
             }
             const v3 inc = -1.0f * d;
             if (hr.prim == kNoHit) {  // :253-260
-                if (S.use_env) L += w3 * env_lookup(S, d);
+                if (S.use_env) emission = w3 * env_lookup(S, d);
             } else {
                 const v3 P = o + hr.t * d;
                 v3 N;
@@ -1122,10 +1126,11 @@ void k_vol_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, int r
                     no = make_float4(norg.x, norg.y, norg.z, 0.0f);
                     nd = make_float4(ndir.x, ndir.y, ndir.z, __uint_as_float(p));
                 }
-                weight[p] = make_float4(w3.x, w3.y, w3.z, __uint_as_float(seed));
+                if (want_next) weight[p] = make_float4(w3.x, w3.y, w3.z, __uint_as_float(seed));
             }
-            vstate = (inside ? kInsideBit : 0u) | obj_index;
-            rad[p] = make_float4(L.x, L.y, L.z, __uint_as_float(vstate));
+            const uint32_t state_now = (inside ? kInsideBit : 0u) | obj_index;
+            if (state_now != vstate || !(emission.x == 0.0f && emission.y == 0.0f && emission.z == 0.0f))
+                rad[p] = make_float4(R.x + emission.x, R.y + emission.y, R.z + emission.z, __uint_as_float(state_now));
         }
         const bool app_out = want_next && !next_inside, app_in = want_next && next_inside;
         uint32_t ns, ss;
