@@ -1,8 +1,8 @@
 """Small path-tracer batches, traced in one launch, equal the wavefront queues bit for bit.
 
-A batch of up to 1024 paths per CU (262,144 on 256 CUs) runs each path in registers, 64 paths a wave or, in small
-batches and deep trees, 8 to 32 with several lanes per ray. Timing a frame's stages keeps the queues; both add the
-same terms to a path in the same order.
+A batch of up to 1024 paths per CU (262,144 on 256 CUs; 16,384 for plain frames in a shallow tree) runs each path in
+registers, 64 paths a wave or, in small batches and deep trees, 8 to 32 with several lanes per ray. Timing a frame's
+stages keeps the queues; both add the same terms to a path in the same order.
 """
 import numpy as np
 import pytest
@@ -38,7 +38,7 @@ def _frame(scene, ca, w, h, spp, depth, queues, rr=False, rng=0, cache=None):
 @pytest.mark.parametrize("w,h,spp,depth,rr,rng", [
     (1, 1, 1, 5, False, 0), (7, 5, 1, 1, False, 0), (13, 11, 3, 9, True, 0),
     (128, 128, 1, 4, False, 1),   # the last batch of 8 paths a wave in a shallow tree
-    (113, 145, 1, 6, True, 0),    # the first of 64
+    (113, 145, 1, 6, True, 0),    # one more: queues in a shallow tree
     (256, 257, 1, 5, False, 0), (512, 512, 1, 3, True, 1),  # the largest batch
     (512, 513, 1, 3, False, 0),   # queues
 ])
