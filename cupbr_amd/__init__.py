@@ -252,6 +252,7 @@ def lib():
             "cupbr_pick": (C.c_int, [P, P, U32, U32, U32, U32, P, P]),
             "cupbr_scene_update_material": (C.c_int, [P, I32, P]),
             "cupbr_renderer_resume": (C.c_int, [P, P, SZ, U32]),
+            "cupbr_grid_forward_id": (C.c_int, [P, P]),
             "cupbr_grid_set_counting": (C.c_int, [P, I32]),
             "cupbr_grid_get_counts": (C.c_int, [P, P]),
             "cupbr_grid_render_device": (C.c_int, [P, P, P, P, P, P, U32, U32, U32, U32, U32, P, P]),
@@ -663,6 +664,12 @@ class GridRenderer:
         c = (C.c_uint64 * 4)()
         _check(lib().cupbr_grid_get_counts(self.scene.handle, c))
         return dict(closest_rays=c[0], shadow_rays=c[1], grid_reads=c[2], atomics=c[3])
+
+    def forward_id(self) -> int:
+        """cupbr_grid_forward_id: number of the render whose paths' radiance the scene keeps, 0: none."""
+        n = C.c_uint64()
+        _check(lib().cupbr_grid_forward_id(self.scene.handle, C.byref(n)))
+        return n.value
 
     def surface_count(self) -> int:
         n = C.c_uint32()

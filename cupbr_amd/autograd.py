@@ -17,24 +17,40 @@ import torch
 from . import Camera, CupbrError, GridMedium, GridRenderer, Scene
 
 
+def _dense(t):
+    """The contiguous float32 tensor that the kernels read for t, None when that is t itself."""
+    if t is None or (t.is_contiguous() and t.dtype == torch.float32):
+        return None
+    return t.detach().contiguous().float()
+
+
 class _GridRenderFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, density, albedo, renderer: GridRenderer, proposal):
-        image = renderer.render(density, albedo, proposal=proposal)  # None: the density itself
-        ctx.renderer = renderer
-        ctx.save_for_backward(density, albedo, proposal)
+        given = (density, albedo, proposal)  # proposal None: the density itself
+        dense = tuple(_dense(t) for t in given)
+        rho, alb, prop = (t if c is None else c for t, c in zip(given, dense))
+        image = renderer.render(rho, alb, proposal=prop)
+        ctx.renderer, ctx.forward_id = renderer, renderer.forward_id()
+        # the given tensors for autograd's version check, the converted ones for the adjoint
+        ctx.save_for_backward(*given, *dense)
         return image
 
     @staticmethod
     def backward(ctx, grad_image):
-        density, albedo, prop = ctx.saved_tensors
+        saved = ctx.saved_tensors
+        rho, alb, prop = (t if c is None else c for t, c in zip(saved[:3], saved[3:]))
         # The saved tensors cannot have changed since the forward (autograd checks their versions),
         # so the adjoint may reuse the forward pass's per-path radiance when that render was the
-        # last one on the scene; otherwise every path is replayed once more.
-        try:
-            gd, ga = ctx.renderer.adjoint(density, albedo, grad_image, proposal=prop, from_forward=True)
-        except CupbrError:
-            gd, ga = ctx.renderer.adjoint(density, albedo, grad_image, proposal=prop)
+        # last one on the scene (its number says so: equal addresses do not, they may have passed on
+        # to another tensor); otherwise every path is replayed once more.
+        if ctx.forward_id != 0 and ctx.renderer.forward_id() == ctx.forward_id:
+            try:
+                gd, ga = ctx.renderer.adjoint(rho, alb, grad_image, proposal=prop, from_forward=True)
+                return gd, ga, None, None
+            except CupbrError:  # a saved-tensor hook has moved them
+                pass
+        gd, ga = ctx.renderer.adjoint(rho, alb, grad_image, proposal=prop)
         return gd, ga, None, None
 
 

@@ -888,6 +888,12 @@ int cupbr_grid_adjoint_from_forward_device(const cupbr_scene* s, const cupbr_cam
                                grad_density, grad_albedo, (hipStream_t)stream, true);
 }
 
+int cupbr_grid_forward_id(const cupbr_scene* s, uint64_t* id) {
+    CHECK_ARG(s && id, "null argument");
+    *id = grid_forward_id(s);
+    return CUPBR_OK;
+}
+
 namespace {
 struct GridHostBufs {
     DevBuf rho, prop, alb;

@@ -597,6 +597,8 @@ int grid_get_counts(const cupbr_scene* s, uint64_t out[4]) {
     return CUPBR_OK;
 }
 
+uint64_t grid_forward_id(const cupbr_scene* s) { return s->grid_forward.valid ? s->grid_forward.id : 0; }
+
 int grid_render_device(const cupbr_scene* cs, const cupbr_camera* cam, const cupbr_grid_medium* m, const float* rho,
                        const float* prop, const float* alb, uint32_t w, uint32_t h, uint32_t frame0, uint32_t spp,
                        uint32_t max_depth, float* image, hipStream_t stream) {
@@ -606,6 +608,9 @@ int grid_render_device(const cupbr_scene* cs, const cupbr_camera* cam, const cup
     unsigned long long* counts = s->grid_counting ? s->grid_counts.as<unsigned long long>() : nullptr;
     const uint32_t n_px = w * h;
     const uint32_t chunk = (uint32_t)std::max<size_t>(1, std::min<size_t>(spp, kMaxGridSamples / n_px));
+    auto& f = s->grid_forward;
+    f.valid = false;  // the samples of the render before go
+    ++f.id;
     if (s->grid_samples.ensure((size_t)n_px * chunk * 12)) return CUPBR_ERR_OUT_OF_MEMORY;
     if (int rc = scene_stream_acquire(s, stream)) return rc;
     for (uint32_t s0 = 0; s0 < spp; s0 += chunk) {
@@ -624,7 +629,6 @@ int grid_render_device(const cupbr_scene* cs, const cupbr_camera* cam, const cup
     if (int rc = scene_stream_release(s, stream)) return rc;
     // all samples of this call stay in grid_samples when they fit one chunk: an adjoint with the
     // same arguments may take the paths' radiance from there
-    auto& f = s->grid_forward;
     f.valid = chunk >= spp;
     f.rho = rho;
     f.prop = prop;

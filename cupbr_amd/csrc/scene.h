@@ -46,6 +46,7 @@ struct cupbr_scene {
     // arguments of the last grid forward render whose per-sample radiance is all in grid_samples
     struct GridForward {
         bool valid = false;
+        uint64_t id = 0;  // counts the renders
         const float *rho = nullptr, *prop = nullptr, *alb = nullptr;
         cupbr_camera cam{};
         cupbr_grid_medium medium{};
@@ -91,6 +92,7 @@ int trace_closest_launch(const cupbr_scene* s, const float* rays, size_t n, int3
 // heterogeneous medium + adjoint (grid.hip)
 int grid_set_counting(cupbr_scene* s, bool enable);
 int grid_get_counts(const cupbr_scene* s, uint64_t out[4]);
+uint64_t grid_forward_id(const cupbr_scene* s);  // of the render whose samples are kept, 0: none
 int grid_validate(const cupbr_scene* s, const cupbr_camera* cam, const cupbr_grid_medium* m, uint32_t w, uint32_t h,
                   uint32_t spp, uint32_t max_depth);
 int grid_render_device(const cupbr_scene* s, const cupbr_camera* cam, const cupbr_grid_medium* m, const float* rho,

@@ -437,6 +437,11 @@ int cupbr_grid_adjoint_from_forward_device(const cupbr_scene* scene, const cupbr
                                            uint32_t height, uint32_t frame0, uint32_t spp, uint32_t max_depth,
                                            const float* d_image, float* grad_density, float* grad_albedo,
                                            void* hip_stream);
+/* Number of the forward render whose paths' radiance the scene keeps: other than 0, and another one
+ * for every render; 0 when the last render's is not kept (none yet, or more than 2^24 samples). The
+ * entry above compares buffers by address, and an address can serve another tensor later: a caller
+ * with several renders under way compares this number, taken right after its own render. */
+int cupbr_grid_forward_id(const cupbr_scene* scene, uint64_t* id);
 /* instrumentation: with counting on, the grid kernels add their work to four counters of the
  * scene: closest-hit rays, shadow rays, grid stencil reads (8 voxels each) and gradient atomics.
  * Enabling resets them; cupbr_grid_get_counts synchronizes the device and reads them. */

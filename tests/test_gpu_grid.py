@@ -212,6 +212,56 @@ def test_grid_full_size_workload():
     torch.testing.assert_close(ga3, -0.5 * ga, rtol=1e-4, atol=1e-5 * float(ga.abs().max()))
 
 
+@pytest.mark.parametrize("kind", ["slice", "float64", "transposed", "contiguous"])
+def test_autograd_of_two_forwards_under_way(kind):
+    """Two renders of one renderer before both of their backwards: the first gradient is that of the
+    first density, also where the kernels read a converted copy whose memory could serve both."""
+    torch = pytest.importorskip("torch")
+    from cupbr_amd.autograd import GridRender
+
+    G = scenes.grid_medium_scene(res=16)
+    ca = G["camera"]
+    cam = cb.Camera.look_at(ca["eye"], ca["target"], ca["up"], ca["vfov"], 32, 32)
+    scene = cb.Scene.from_desc(G["desc"])
+    med = cb.GridMedium.from_dict(G["density"].shape, G["medium"])
+    alb = torch.from_numpy(G["albedo"]).cuda()
+    weight = torch.from_numpy(np.random.default_rng(5).normal(size=(32, 32, 3)).astype(np.float32)).cuda()
+
+    def leaf_and_density(values):
+        v = torch.from_numpy(values).cuda()
+        if kind == "slice":  # as a network with several output channels leaves it
+            leaf = torch.stack([v, torch.zeros_like(v)], -1).requires_grad_(True)
+            return leaf, leaf[..., 0]
+        if kind == "float64":
+            leaf = v.double().requires_grad_(True)
+            return leaf, leaf
+        if kind == "transposed":
+            leaf = v.permute(2, 1, 0).contiguous().requires_grad_(True)
+            return leaf, leaf.permute(2, 1, 0)
+        leaf = v.requires_grad_(True)
+        return leaf, leaf
+
+    def render():
+        return GridRender(scene, cam, med, 32, 32, spp=4, max_depth=4)
+
+    first, second = G["density"] * np.float32(0.9) + np.float32(0.05), G["target_density"] * np.float32(0.5) + np.float32(0.1)
+    want = []
+    for values in (first, second):
+        leaf, rho = leaf_and_density(values)
+        want.append(torch.autograd.grad(render()(rho, alb), leaf, weight)[0])
+    R = render()
+    leaves, images = [], []
+    for values in (first, second):
+        leaf, rho = leaf_and_density(values)
+        leaves.append(leaf)
+        images.append(R(rho, alb))
+    for image, leaf, w in zip(images, leaves, want):
+        got = torch.autograd.grad(image, leaf, weight)[0]
+        assert got.shape == w.shape and got.dtype == w.dtype
+        # the same terms by atomic adds in another order
+        assert float(torch.linalg.norm(got - w)) <= 1e-4 * float(torch.linalg.norm(w))
+
+
 @pytest.mark.parametrize("shape,size,spp", [
     ((1, 1, 1), 24, 8),      # every lookup clamped on all axes
     ((1, 5, 2), 24, 8),
