@@ -512,6 +512,7 @@ int cupbr_render(cupbr_renderer* r, const cupbr_camera* cam, uint32_t spp) {
     if (int rc = scene_upload(r->scene)) return rc;
     if (cam->moved) r->frame_index = 0;  // :174-177
     r->stats = cupbr_render_stats{};
+    r->counted = false;
     r->timer.used = 0;
     CUPBR_HIP_CHECK(hipEventRecord(r->ev_start, r->stream));
     int rc = CUPBR_OK;
@@ -543,8 +544,8 @@ int cupbr_renderer_get_stats(const cupbr_renderer* cr, cupbr_render_stats* out) 
     float ms = 0.0f;
     if (hipEventElapsedTime(&ms, r->ev_start, r->ev_stop) == hipSuccess) r->stats.milliseconds = ms;
     Counters c{};
-    if (r->wf.counters.ptr) CUPBR_HIP_CHECK(hipMemcpy(&c, r->wf.counters.ptr, sizeof c, hipMemcpyDeviceToHost));
-    if (r->wf.counters.ptr && (r->method == CUPBR_PATHTRACER || r->method == CUPBR_VOLUME || r->method == CUPBR_GRADIENTDOMAIN)) {
+    if (r->counted) CUPBR_HIP_CHECK(hipMemcpy(&c, r->wf.counters.ptr, sizeof c, hipMemcpyDeviceToHost));
+    if (r->counted && (r->method == CUPBR_PATHTRACER || r->method == CUPBR_VOLUME || r->method == CUPBR_GRADIENTDOMAIN)) {
         r->stats.extension_rays = c.extension_rays;
         r->stats.shadow_rays = c.shadow_rays;
         r->stats.extension_node_visits = c.ext_nodes;

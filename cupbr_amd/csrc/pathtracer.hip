@@ -1231,6 +1231,7 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
     Wavefront& wf = r->wf;
     Counters* c = wf.counters.as<Counters>();
     CUPBR_HIP_CHECK(hipMemsetAsync(c, 0, sizeof(Counters), r->stream));
+    r->counted = true;
     uint32_t* spill = r->scene->stack_entries > (uint32_t)kPtLds ? wf.spill.as<uint32_t>() : nullptr;
     const DevScene& S = r->scene->dev;
     float* img = r->images[CUPBR_IMAGE_OUTPUT].as<float>();
@@ -1388,6 +1389,7 @@ int volume_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t 
     }
     Counters* c = wf.counters.as<Counters>();
     CUPBR_HIP_CHECK(hipMemsetAsync(c, 0, sizeof(Counters), r->stream));
+    r->counted = true;
     uint32_t* spill = r->scene->stack_entries > (uint32_t)kPtLds ? wf.spill.as<uint32_t>() : nullptr;
     const DevScene& S = r->scene->dev;
     float* img = r->images[CUPBR_IMAGE_OUTPUT].as<float>();
@@ -1464,6 +1466,7 @@ int gdpt_paths_wavefront(cupbr_renderer* r, const cupbr_camera& cam, uint32_t fr
     uint32_t* slots[2] = {wf.gdpt_slot.as<uint32_t>(), wf.gdpt_slot.as<uint32_t>() + (size_t)batch * n_int};
     Counters* c = wf.counters.as<Counters>();
     CUPBR_HIP_CHECK(hipMemsetAsync(c, 0, sizeof(Counters), r->stream));
+    r->counted = true;
     uint32_t* spill = r->scene->stack_entries > (uint32_t)kPtLds ? wf.spill.as<uint32_t>() : nullptr;
     const DevScene& S = r->scene->dev;
     float* im[kNumImages];

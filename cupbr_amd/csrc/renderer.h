@@ -141,6 +141,7 @@ struct cupbr_renderer {
     float nrc_camera_min_roughness = __builtin_inff();  // camera-hit cache vertices (+inf: none)
     uint32_t nrc_max_rows = 1u << 18;     // training rows kept per frame
     cupbr::DevBuf nrc_queries, nrc_pending, nrc_rows;
+    bool counted = false;  // the last cupbr_render call launched paths, and wf.counters holds its counts
     // second stream for cache inference that overlaps the training paths' later bounces
     hipStream_t side_stream = nullptr;
     hipEvent_t ev_queries = nullptr, ev_side_done = nullptr;

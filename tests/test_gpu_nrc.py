@@ -319,3 +319,28 @@ def test_cache_lowers_equal_time_error_on_the_cornell_box():
     print(f"cornell 256^2: NRC frame {t_nrc:.3f} ms rel-MSE {e_nrc:.4f}; PT 1 spp {t_pt:.3f} ms -> {k} spp at equal "
           f"time, rel-MSE {e_pt:.4f}; ratio {e_pt / e_nrc:.2f}", flush=True)
     assert e_nrc * 1.5 < e_pt
+
+
+def test_stats_of_calls_that_launch_no_paths():
+    """The counts are those of the last call: after a cached frame, calls without paths report none."""
+    w = h = 32
+    scene, cam = _cornell(w, h)
+    cache = cb.RadianceCache((0, 0, 0), (1, 1, 1), seed=1)
+    r = _pt(scene, cam, w, h, 2, cache=cache, training_paths=w * h // 2, train_steps=0)
+    counts = ("extension_rays", "shadow_rays", "cache_queries", "cache_training_rows")
+    assert all(r.stats()[k] > 0 for k in counts)
+    r.render(cam, 0)
+    assert {k: r.stats()[k] for k in counts} == dict.fromkeys(counts, 0)
+    for method, size in ((cb.RenderingMethod.GRADIENTDOMAIN, 2), (cb.RenderingMethod.RAYTRACER, w),
+                         (cb.RenderingMethod.VOLUME, w)):
+        r.set_method(cb.RenderingMethod.PATHTRACER)
+        r.set_output_size(w, h)
+        r.render(cam, 1)
+        assert r.stats()["cache_queries"] > 0
+        r.set_method(method)
+        r.set_output_size(size, size)
+        r.render(cam, 1)
+        st = r.stats()
+        assert st["cache_queries"] == 0 and st["cache_training_rows"] == 0, method
+        if method != cb.RenderingMethod.VOLUME:
+            assert st["extension_rays"] == 0 and st["shadow_rays"] == 0, method
