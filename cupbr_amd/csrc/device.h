@@ -28,14 +28,19 @@ struct DevBuf {
     void* ptr = nullptr;
     size_t bytes = 0;
     int ensure(size_t n) {
-        if (n <= bytes) return CUPBR_OK;
-        if (ptr) (void)hipFree(ptr);
-        ptr = nullptr;
-        bytes = 0;
-        if (n == 0) return CUPBR_OK;
-        if (hipMalloc(&ptr, n) != hipSuccess) return set_error(CUPBR_ERR_OUT_OF_MEMORY, "hipMalloc failed", false);
+        return try_ensure(n) ? CUPBR_OK : set_error(CUPBR_ERR_OUT_OF_MEMORY, "hipMalloc failed", false);
+    }
+    // ensure for a caller that can go on without: no error is left behind
+    bool try_ensure(size_t n) {
+        if (n <= bytes) return true;
+        release();
+        if (hipMalloc(&ptr, n) != hipSuccess) {
+            ptr = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
         bytes = n;
-        return CUPBR_OK;
+        return true;
     }
     void release() {
         if (ptr) (void)hipFree(ptr);

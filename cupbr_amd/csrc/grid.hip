@@ -38,6 +38,7 @@
 #include <cmath>
 
 #include "device.h"
+#include "grid_cells.h"
 #include "scene.h"
 #include "shading.h"
 #include "traverse.h"
@@ -65,9 +66,7 @@ constexpr uint32_t kMaxTrackSteps = 1u << 22;
 // 64^3 voxels, 256x256, 64 spp (101 M stencils a launch): 39.0 ms adding voxel by voxel to copies of the
 // gradient (20.5 G adds/s, the request rate), 11.8 ms in cells (68 G adds/s, 8.5 G requests: the
 // divergence of the paths bounds it now); clearing, folding and gathering the 140 MB take 35 us. 256^3, 512x512, 16 spp: 39.4 -> 19.2 ms.
-constexpr uint32_t kGradCopies = 8;
-constexpr size_t kMaxGradCopyBytes = (size_t)8 << 30;  // fewer copies above; grids of one such copy add to the output
-// Cells per path above which clearing and folding the cells (64 bytes each, per copy) cost more than the
+// Cells per path above which clearing and folding the cells (32 bytes each, per copy) cost more than the
 // requests they save: those add to the output too. 64^3 cells, 32 k paths (8 cells a path): 474 us in cells,
 // 485 voxel by voxel; 16 k paths (17): 487 and 473; 128^3 cells, 32 k paths (65): 801 and 511.
 constexpr size_t kCellsPerPath = 16;
@@ -597,6 +596,17 @@ int grid_get_counts(const cupbr_scene* s, uint64_t out[4]) {
     return CUPBR_OK;
 }
 
+// cell_copies, with the memory for them: fewer where the device does not grant it. The free memory is asked for
+// (10 us) only when the scene does not hold all the copies that could be used.
+static uint32_t ensure_cells(DevBuf& cells, size_t bytes) {
+    uint32_t copies = cell_copies(bytes, cells.bytes, SIZE_MAX);
+    if (bytes * copies <= cells.bytes) return copies;
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) == hipSuccess) copies = cell_copies(bytes, cells.bytes, free_b);
+    while (copies > 0 && !cells.try_ensure(bytes * copies)) copies >>= 1;
+    return copies;
+}
+
 uint64_t grid_forward_id(const cupbr_scene* s) { return s->grid_forward.valid ? s->grid_forward.id : 0; }
 
 int grid_render_device(const cupbr_scene* cs, const cupbr_camera* cam, const cupbr_grid_medium* m, const float* rho,
@@ -670,13 +680,8 @@ int grid_adjoint_device(const cupbr_scene* cs, const cupbr_camera* cam, const cu
     if (int rc = scene_stream_acquire(s, stream)) return rc;
     // copies of the gradient's cells (cleared by a kernel, not a memset, so that a captured graph replays it)
     const size_t n_cells = ((size_t)m->nx + 1) * (m->ny + 1) * (m->nz + 1), cell_floats = n_cells * 8;
-    uint32_t copies = kGradCopies;
-    while (copies > 0 && cell_floats * copies * sizeof(float) > kMaxGradCopyBytes) copies >>= 1;
-    bool in_cells = copies > 0 && (size_t)w * h * spp * kCellsPerPath >= n_cells;
-    if (in_cells && s->grid_grad.ensure(cell_floats * copies * sizeof(float))) {
-        (void)hipGetLastError();  // no memory for them
-        in_cells = false;
-    }
+    const uint32_t copies = (size_t)w * h * spp * kCellsPerPath < n_cells ? 0u : ensure_cells(s->grid_grad, cell_floats * sizeof(float));
+    const bool in_cells = copies > 0;
     float* target = grad_rho;
     if (in_cells) {
         target = s->grid_grad.as<float>();

@@ -41,7 +41,7 @@ struct cupbr_scene {
     cupbr::DevBuf grid_spill;          // traversal stack spill of the grid-medium kernels
     cupbr::DevBuf grid_samples;        // per-sample radiance of the grid-medium forward pass
     cupbr::DevBuf grid_counts;         // 4 x u64 work counters of the grid-medium kernels
-    cupbr::DevBuf grid_grad;           // per-XCD density-gradient copies of the adjoint
+    cupbr::DevBuf grid_grad;           // cells of the adjoint's density gradient, in up to 8 copies
     bool grid_counting = false;
     // arguments of the last grid forward render whose per-sample radiance is all in grid_samples
     struct GridForward {

@@ -420,7 +420,10 @@ int cupbr_grid_render_device(const cupbr_scene* scene, const cupbr_camera* camer
                              uint32_t width, uint32_t height, uint32_t frame0, uint32_t spp, uint32_t max_depth,
                              float* image, void* hip_stream);
 /* Adjoint: ADDS dLoss/d(density) and dLoss/d(surface_albedo) for the image's cotangent d_image
- * (width*height*3 floats) to grad_density and grad_albedo (same sizes as density and albedo). */
+ * (width*height*3 floats) to grad_density and grad_albedo (same sizes as density and albedo).
+ * The scene keeps a workspace of 32 (nx+1)(ny+1)(nz+1) bytes in up to 8 copies until it is destroyed
+ * (64^3: 70 MB, 256^3: 4.3 GB); as many copies as fit 8 GiB and a quarter of the memory that is free
+ * when it grows. With none, or with few paths for the grid (16 cells per path), it adds without. */
 int cupbr_grid_adjoint_device(const cupbr_scene* scene, const cupbr_camera* camera, const cupbr_grid_medium* medium,
                               const float* density, const float* proposal, const float* surface_albedo,
                               uint32_t width, uint32_t height, uint32_t frame0, uint32_t spp, uint32_t max_depth,

@@ -288,3 +288,29 @@ def test_grid_adjoint_shapes_against_fp64_oracle(shape, size, spp):
     # the bars of the other oracle comparisons here
     assert np.linalg.norm(gr - rr) <= 1e-3 * np.linalg.norm(rr)
     assert np.linalg.norm(ga - ra) <= 1e-3 * np.linalg.norm(ra)
+
+
+@pytest.mark.parametrize("shape", [(350, 350, 350), (511, 512, 510), (511, 512, 511)])
+def test_grid_adjoint_with_fewer_copies_of_the_cells(shape):
+    """Grids whose cells fit the workspace limit four times, twice and once: the gradient of a 64-spp call is the
+    sum over its frames of 1-spp calls, which have too few paths for the cells and add without."""
+    torch = pytest.importorskip("torch")
+    G = scenes.grid_medium_scene(res=8)
+    ca = G["camera"]
+    cam = cb.Camera.look_at(ca["eye"], ca["target"], ca["up"], ca["vfov"], 512, 512)
+    scene = cb.Scene.from_desc(G["desc"])
+    med = cb.GridMedium.from_dict(shape, G["medium"])
+    g = torch.Generator(device="cuda").manual_seed(1)
+    rho = 0.05 + 0.9 * torch.rand(shape, generator=g, device="cuda")
+    alb = torch.from_numpy(G["albedo"]).cuda()
+    weight = torch.randn(512, 512, 3, generator=g, device="cuda")
+    gr, ga = cb.GridRenderer(scene, cam, med, 512, 512, spp=64, max_depth=3).adjoint(rho, alb, weight)
+    sr, sa = torch.zeros_like(rho), torch.zeros_like(alb)
+    for k in range(64):
+        cb.GridRenderer(scene, cam, med, 512, 512, spp=1, max_depth=3, frame0=k).adjoint(
+            rho, alb, weight, grad_density=sr, grad_albedo=sa)
+    sr, sa = sr / 64, sa / 64
+    assert float(torch.linalg.norm(sr)) > 0
+    # the same terms in FP32 sums of other orders
+    assert float(torch.linalg.norm(gr - sr)) <= 1e-4 * float(torch.linalg.norm(sr))
+    assert float(torch.linalg.norm(ga - sa)) <= 1e-4 * float(torch.linalg.norm(sa))
