@@ -1246,10 +1246,11 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
     auto raygen = pcg ? k_pt_raygen<Pcg32> : k_pt_raygen<uint32_t>;
     auto camera = pcg ? k_pt_camera<Pcg32> : k_pt_camera<uint32_t>;
     const auto packet_blocks = [](uint32_t n) { return ((n + kPtBlock - 1) / kPtBlock + 7u) / 8u * 8u; };
-    // a small batch in one launch (not when the stages of a frame are timed)
+    // a small batch in one launch (not when the stages of a frame are timed, and only as the call's one batch: the
+    // kernel counts on from the call's cleared counters, where bounce 0 of the queues starts each batch at 0)
     const uint32_t cus = (uint32_t)device_cu_count();
     const bool deep = r->scene->stack_entries > kDeepStack;
-    const bool whole = packet && !r->profiling &&
+    const bool whole = packet && !r->profiling && batch == spp &&
                        (size_t)batch * npix <= (size_t)cus * (deep || nrc ? kWholePaths : kWholeShallow);
     uint32_t per_wave = 8;
     while (per_wave < 64u && (size_t)per_wave * cus * (deep ? 16u : 8u) < (size_t)batch * npix) per_wave *= deep ? 2u : 8u;
