@@ -151,15 +151,24 @@ __global__ __launch_bounds__(kNrcBlock, 2) void k_nrc_infer(const bf16x8* __rest
                                                             const float* __restrict__ rec, uint32_t n,
                                                             const uint32_t* __restrict__ n_dev, uint32_t stride,
                                                             float* __restrict__ out,
-                                                            const uint32_t* __restrict__ begin_dev) {
+                                                            const uint32_t* __restrict__ begin_dev, NrcParts parts) {
     const int lane = threadIdx.x & 63, g = lane >> 4;
     bf16x8 w[kFwdSize / 512];  // loaded while the counts are
 #pragma unroll
     for (int i = 0; i < kFwdSize / 512; ++i) w[i] = packed[i * 64 + lane];
-    if (n_dev) n = min(n, *n_dev);  // count written by an earlier kernel on the stream
-    const uint32_t begin = begin_dev ? min(*begin_dev, n) : 0u;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t n_waves = (gridDim.x * blockDim.x) >> 6;
+    uint32_t blk = blockIdx.x, blks = gridDim.x, begin = 0;
+    if (kAccumulate && parts.size != 0u) {  // an XCD's part by its own blocks
+        const uint32_t x = blk & 7u;
+        blk >>= 3;
+        blks >>= 3;
+        begin = x * parts.size;
+        n = begin + min(parts.size, n_dev[x * parts.stride]);
+    } else {
+        if (n_dev) n = min(n, *n_dev);  // count written by an earlier kernel on the stream
+        begin = begin_dev ? min(*begin_dev, n) : 0u;
+    }
+    const uint32_t wave = (blk * blockDim.x + threadIdx.x) >> 6;
+    const uint32_t n_waves = (blks * blockDim.x) >> 6;
     const uint32_t pairs = (n - begin + 31) / 32;  // two tiles of 16 queries per wave and step
     if (wave >= pairs) return;
     for (uint32_t t = wave; t < pairs; t += n_waves) {
@@ -617,16 +626,17 @@ int nrc_create(const float lo[3], const float hi[3], uint32_t seed, cupbr_nrc** 
 }
 
 int nrc_infer(cupbr_nrc* c, const float* rec, uint32_t n, const uint32_t* n_dev, uint32_t stride, float* out,
-              bool accumulate, hipStream_t stream, const uint32_t* begin_dev) {
+              bool accumulate, hipStream_t stream, const uint32_t* begin_dev, NrcParts parts) {
     if (n == 0) return CUPBR_OK;
     const uint32_t pairs = (n + 31) / 32;  // a wave takes two 16-query tiles at a time
-    const int blocks = (int)std::max<uint32_t>(1, std::min<uint32_t>((pairs + 3) / 4, (uint32_t)device_cu_count() * 2));
+    uint32_t blocks = std::max<uint32_t>(1, std::min<uint32_t>((pairs + 3) / 4, (uint32_t)device_cu_count() * 2));
+    if (parts.size != 0) blocks = (blocks + 7) / 8 * 8;
     if (accumulate)
         hipLaunchKernelGGL(k_nrc_infer<true>, dim3(blocks), dim3(kNrcBlock), 0, stream, c->packed_fwd.as<bf16x8>(),
-                           c->box, rec, n, n_dev, stride, out, begin_dev);
+                           c->box, rec, n, n_dev, stride, out, begin_dev, parts);
     else
         hipLaunchKernelGGL(k_nrc_infer<false>, dim3(blocks), dim3(kNrcBlock), 0, stream, c->packed_fwd.as<bf16x8>(),
-                           c->box, rec, n, n_dev, stride, out, begin_dev);
+                           c->box, rec, n, n_dev, stride, out, begin_dev, parts);
     CUPBR_HIP_CHECK(hipGetLastError());
     return CUPBR_OK;
 }

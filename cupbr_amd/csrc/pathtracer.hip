@@ -389,16 +389,54 @@ __global__ void k_snapshot_queries(Counters* c) { c->query_early.v = c->cache.qu
 
 // training rows from the pending rows of finished training paths: target = (final radiance -
 // radiance before the vertex's reflection) / throughput at the vertex (0 where the throughput is 0);
-// also counts the batch's queries and rows
+// also counts the batch's queries and rows. part_rows: whole paths leave their rows in parts of so many, one per XCD
+// (0: in one list).
 __device__ __forceinline__ void nrc_rows(uint32_t first, uint32_t stride, const float4* __restrict__ pending, Counters* c,
-                                         uint32_t max_rows, const float4* __restrict__ rad, float4* __restrict__ rows) {
-    const uint32_t n = min(c->cache.rows, max_rows);
+                                         uint32_t max_rows, uint32_t part_rows, const float4* __restrict__ rad,
+                                         float4* __restrict__ rows) {
+    uint32_t part[8], total = 0, queries = 0;
+    if (part_rows != 0u) {
+#pragma unroll
+        for (uint32_t x = 0; x < 8; ++x) {
+            part[x] = min(c->cache_part[x].rows, part_rows);
+            total += part[x];
+            queries += c->cache_part[x].queries;
+        }
+    } else {
+        total = c->cache.rows;
+        queries = c->cache.queries;
+    }
+    const uint32_t n = min(total, max_rows);
+    if (part_rows != 0u && total > n) {  // too many: as large a share of every part, its first rows
+        uint32_t before = 0, kept = 0;
+#pragma unroll
+        for (uint32_t x = 0; x < 8; ++x) {
+            before += part[x];
+            const uint32_t upto = (uint32_t)((unsigned long long)before * n / total);
+            part[x] = upto - kept;
+            kept = upto;
+        }
+    }
     if (first == 0) {
-        c->cache_queries += c->cache.queries;
+        c->cache_queries += queries;
         c->cache_rows += n;
+        if (part_rows != 0u) c->cache.rows = total;  // for the training steps
     }
     for (uint32_t i = first; i < n; i += stride) {
-        const float4* r = pending + (size_t)i * 6;
+        uint32_t slot = i;
+        if (part_rows != 0u) {
+            uint32_t left = i;
+            bool found = false;
+#pragma unroll
+            for (uint32_t x = 0; x < 8; ++x) {
+                if (!found && left < part[x]) {
+                    slot = x * part_rows + left;
+                    found = true;
+                }
+                left -= found ? 0u : part[x];
+            }
+        }
+        const float4* r = pending + (size_t)slot * 6;
         const float4 a = r[4], b = r[5];
         const uint32_t p = __float_as_uint(b.z);
         const float4 R = rad[p];
@@ -614,9 +652,12 @@ __device__ __forceinline__ void wave_append2(bool want_lo, bool want_hi, unsigne
     hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) + (uint32_t)__popcll(mh & below);
 }
 
+// paths of one XCD in a k_pt_paths launch of so many blocks
+__host__ __device__ inline uint32_t part_paths(uint32_t blocks, uint32_t per_wave) { return (blocks >> 3) * kPtWaves * per_wave; }
+
 // Whole paths of a small batch: the camera rays as packets (camera_packets), then vertex, shadow ray and next ray in
 // turn, in the order of the kernels above, so that a path's radiance is the same sum. per_wave paths a wave; with
-// kFew its last 16 and fewer rays by 8 lanes each (trace_lanes).
+// kFew its last 16 and fewer rays by 8 lanes each (trace_lanes). nrc.max_rows: pending rows of one XCD's part.
 template <bool kNrc, bool kFew, class Seed>
 __global__ __launch_bounds__(kPtBlock)
 void k_pt_paths(DevScene S, uint32_t n, uint32_t per_wave, cupbr_camera cam, uint32_t w, uint32_t h, uint32_t frame0,
@@ -650,12 +691,16 @@ void k_pt_paths(DevScene S, uint32_t n, uint32_t per_wave, cupbr_camera cam, uin
             if (v.emits) L += v.emission;
         }
         if (kNrc) {
+            // an XCD's records go to its own part of the lists (a path asks the cache once, so its queries fit the
+            // range of its paths): a counter that all XCDs add to costs 8 of this kernel's 97 us in a 256x256
+            // frame of the Cornell box
+            const uint32_t xcd = blockIdx.x & 7u;
             uint32_t qs, rs;
-            wave_append2(v.query, v.row, &c->cache.both, qs, rs);
+            wave_append2(v.query, v.row, &c->cache_part[xcd].both, qs, rs);
             if (v.query)
-                for (int k = 0; k < 5; ++k) nrc.queries[(size_t)qs * 5 + k] = v.rec[k];
+                for (int k = 0; k < 5; ++k) nrc.queries[((size_t)xcd * part_paths(gridDim.x, per_wave) + qs) * 5 + k] = v.rec[k];
             if (v.row && rs < nrc.max_rows)
-                for (int k = 0; k < 6; ++k) nrc.pending[(size_t)rs * 6 + k] = v.rec[k];
+                for (int k = 0; k < 6; ++k) nrc.pending[((size_t)xcd * nrc.max_rows + rs) * 6 + k] = v.rec[k];
         }
         bool occluded = false;
         n_sh += v.shadow ? 1u : 0u;
@@ -732,12 +777,13 @@ __global__ __launch_bounds__(kPtBlock) void k_accumulate_rows(float* __restrict_
                                                               uint32_t w, uint32_t h, SampleOrder order, uint32_t frame0,
                                                               uint32_t nspp, uint32_t pix_blocks,
                                                               const float4* __restrict__ pending, Counters* c,
-                                                              uint32_t max_rows, float4* __restrict__ rows) {
+                                                              uint32_t max_rows, uint32_t part_rows,
+                                                              float4* __restrict__ rows) {
     if (blockIdx.x < pix_blocks)
         accumulate_pixel(blockIdx.x * blockDim.x + threadIdx.x, img, rad, w, h, order, frame0, nspp);
     else
         nrc_rows((blockIdx.x - pix_blocks) * blockDim.x + threadIdx.x, (gridDim.x - pix_blocks) * blockDim.x, pending, c,
-                 max_rows, rad, rows);
+                 max_rows, part_rows, rad, rows);
 }
 
 // ------------------------------------------------------------------ gradient-domain paths
@@ -1259,12 +1305,15 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
                                   : (pcg ? k_pt_paths<false, false, Pcg32> : k_pt_paths<false, false, uint32_t>);
     NrcShade ns{nullptr, nullptr, 0, __builtin_inff()};
     uint32_t train_thresh = 0;
+    const uint32_t path_blocks = packet_blocks((batch * npix + per_wave - 1) / per_wave * 64u);
+    uint32_t part_rows = 0;  // whole paths: room for the rows of one XCD's paths, one a vertex
     if (nrc) {
+        if (whole) part_rows = (uint32_t)std::min<size_t>(r->nrc_max_rows, (size_t)part_paths(path_blocks, per_wave) * bounces);
         if ((rc = r->nrc_queries.ensure((size_t)batch * npix * 80)) ||
-            (rc = r->nrc_pending.ensure((size_t)r->nrc_max_rows * 96)) ||
+            (rc = r->nrc_pending.ensure((size_t)(whole ? 8u * part_rows : r->nrc_max_rows) * 96)) ||
             (rc = r->nrc_rows.ensure((size_t)r->nrc_max_rows * 80)))
             return rc;
-        ns = NrcShade{r->nrc_queries.as<float4>(), r->nrc_pending.as<float4>(), r->nrc_max_rows,
+        ns = NrcShade{r->nrc_queries.as<float4>(), r->nrc_pending.as<float4>(), whole ? part_rows : r->nrc_max_rows,
                       r->nrc_camera_min_roughness};
         if (!r->side_stream) {
             if (hipStreamCreateWithFlags(&r->side_stream, hipStreamNonBlocking) != hipSuccess ||
@@ -1289,7 +1338,7 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
             if ((rc = stage_mark(r, 3))) return rc;
         }
         if (whole)
-            hipLaunchKernelGGL(paths, dim3(packet_blocks((npath + per_wave - 1) / per_wave * 64u)), dim3(kPtBlock), 0,
+            hipLaunchKernelGGL(paths, dim3(path_blocks), dim3(kPtBlock), 0,
                                r->stream, S, npath, per_wave, cam, w, h,
                                frame0 + s0, order, train_thresh, r->max_trace_depth, (int)r->russian_roulette,
                                wf.radiance.as<float4>(), c, ns, spill, grid_threads);
@@ -1335,9 +1384,10 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
         if (nrc) {
             // throughput * cache for the paths that ended at a cache vertex (those not already
             // inferred on the side stream), then the training rows
-            if ((rc = nrc_infer(r->nrc, r->nrc_queries.as<float>(), npath, &c->cache.queries, 20,
-                                wf.radiance.as<float>(), true, r->stream,
-                                side_pending ? &c->query_early.v : nullptr)))
+            const uint32_t* n_queries = whole ? &c->cache_part[0].queries : &c->cache.queries;
+            const NrcParts parts = whole ? NrcParts{part_paths(path_blocks, per_wave), (uint32_t)(sizeof c->cache_part[0] / 4)} : NrcParts{};
+            if ((rc = nrc_infer(r->nrc, r->nrc_queries.as<float>(), npath, n_queries, 20, wf.radiance.as<float>(), true,
+                                r->stream, side_pending ? &c->query_early.v : nullptr, parts)))
                 return rc;
             if (side_pending) {
                 CUPBR_HIP_CHECK(hipStreamWaitEvent(r->stream, r->ev_side_done, 0));
@@ -1347,7 +1397,7 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
             const uint32_t pix_blocks = (npix + kPtBlock - 1) / kPtBlock;
             hipLaunchKernelGGL(k_accumulate_rows, dim3(pix_blocks + (uint32_t)device_cu_count()), dim3(kPtBlock), 0,
                                r->stream, img, wf.radiance.as<float4>(), w, h, order, frame0 + s0, nb, pix_blocks,
-                               r->nrc_pending.as<float4>(), c, r->nrc_max_rows, r->nrc_rows.as<float4>());
+                               r->nrc_pending.as<float4>(), c, r->nrc_max_rows, part_rows, r->nrc_rows.as<float4>());
         } else {
             hipLaunchKernelGGL(k_accumulate, dim3((npix + kPtBlock - 1) / kPtBlock), dim3(kPtBlock), 0, r->stream, img,
                                wf.radiance.as<float4>(), w, h, order, frame0 + s0, nb);

@@ -56,12 +56,13 @@ struct Counters {
     CounterLine inside[2][8];    // volume renderer: rays inside an object, likewise
     CounterLine work[8];         // trace kernel: extension rays handed out beyond the dealt pieces, per XCD
     CounterLine swork[8];        // trace kernel: shadow rays handed out beyond the dealt pieces, per XCD
-    union alignas(128) {
+    union alignas(128) CacheCount {
         struct {
             uint32_t queries, rows;  // radiance-cache queries and training rows of the batch
         };
         unsigned long long both;
     } cache;
+    CacheCount cache_part[8];    // whole paths: those of each XCD's blocks
     CounterLine query_early;  // queries that existed after the second bounce's shade
     unsigned long long extension_rays;
     unsigned long long shadow_rays;

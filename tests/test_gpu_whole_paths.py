@@ -63,3 +63,34 @@ def test_cached_whole_paths_equal_queues(name, w, h):
     want, n_want = _frame(scene, ca, w, h, 2, 6, True, cache=cache)
     assert n_got == n_want and n_got["cache_queries"] > 0 and n_got["cache_training_rows"] > 0
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("name,w,h", [("cornell", 21, 13), ("cornell", 200, 161), ("boxes", 96, 64), ("cornell", 512, 512)])
+def test_whole_paths_leave_the_rows_of_the_queues(name, w, h):
+    """Every path a training path: the rows, gathered from one part per XCD, are as many as the queues' and the
+    Adam step on a million draws of them goes the same way. A weight's first step is lr against the sign of its
+    gradient, whose sampling error is 1e-3 of the rows' spread. Of the last size's rows 2^18 are kept, which ones
+    is up to their order (the queues keep the first bounces')."""
+    desc, ca = SCENES[name]()
+    scene = cb.Scene.from_desc(desc)
+    cam = cb.Camera.look_at(ca["eye"], ca["target"], ca["up"], ca["vfov"], w, h)
+    steps, rows, images = [], [], []
+    for queues in (False, True):
+        cache = cb.RadianceCache((-3, -3, -3), (3, 3, 3), seed=3)
+        w0 = cache.get_weights()
+        r = cb.PBRenderer(cb.RenderingMethod.PATHTRACER)
+        r.set_output_size(w, h)
+        r.register_scene(scene)
+        r.set_max_trace_depth(6)
+        r.set_radiance_cache(cache, training_paths=w * h, train_steps=1, batch=1 << 20, learning_rate=1e-3)
+        r.set_profiling(queues)
+        r.render(cam, 1)
+        rows.append(r.stats()["cache_training_rows"])
+        images.append(r.get_output_image())
+        steps.append((cache.get_weights() - w0).astype(np.float64))
+    print(f"{name} {w}x{h}: {rows} rows", flush=True)
+    assert rows[0] == rows[1] > 0 and (rows[0] == 1 << 18) == (w == 512)
+    assert np.array_equal(images[0], images[1])
+    assert np.isfinite(steps[0]).all()
+    a, b = steps
+    assert rows[0] == 1 << 18 or np.dot(a, b) >= 0.95 * np.linalg.norm(a) * np.linalg.norm(b)
