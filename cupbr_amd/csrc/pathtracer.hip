@@ -48,12 +48,16 @@ constexpr uint32_t kWholePaths = 1024;
 // Traversal stack entries (three per BVH4 level) above which a wave of such a batch holds only as many paths (8 to 32)
 // as 16 waves per CU need, so that 8 lanes walk the tree for each: 1M triangles, 64x64, 1 spp, 1310 -> 312 us, 256x256
 // 1318 -> 761. In a shallow tree that pays up to 64 paths per CU only (Cornell box, depth 5: 64x64 158 -> 100 us, but
-// 256x256 156 -> 225); cached frames take 64 paths a wave beyond it, plain ones the queues (kWholeShallow).
+// 256x256 156 -> 225); beyond it a wave takes 64 paths.
 constexpr uint32_t kDeepStack = 24;
-// The limit of plain frames in a shallow tree. Larger ones would still gain a little (Cornell box, 256x256, 152 -> 139
-// us a frame; mixed primitives 331x217, 6 spp, none), but a cached frame (190 us) would then cost 1.4 plain ones
-// instead of 1.25, and what the cache is for, less error in equal time, needs that to stay well below 1.5.
-constexpr uint32_t kWholeShallow = 64;
+// The limits of plain frames in a shallow tree, of more bounces than one and of one. There the queues' launches end
+// sooner, so that they catch up where the waves of whole paths no longer all start at once (us, queues / whole paths;
+// Cornell box, mixed primitives, spheres and boxes):
+//   depth 2:  160x160 84 / 71, 88 / 67, 71 / 55;  256x255 85 / 78, 88 / 68, 71 / 63;  362x362 89 / 94, 93 / 91, 71 / 83
+//   depth 5:  160x160 158 / 150, 184 / 146, 116 / 97;  256x255 160 / 147, 175 / 146, 118 / 102;
+//             362x362 170 / 163, 181 / 156, 122 / 113;  512x256 165 / 159, 182 / 153, 119 / 124
+//   depth 1:  200x200 52 / 50, 52 / 47, 44 / 44;  256x255 52 / 59, 53 / 54, 44 / 52
+constexpr uint32_t kWholeShallow = 256, kWholeShallowDirect = 192;
 
 // Block-wide append: every thread of the block calls it; lanes with `want` get consecutive
 // slots of the queue whose length is *count (one atomic per block).
@@ -1297,7 +1301,7 @@ int render_pathtracer(cupbr_renderer* r, const cupbr_camera& cam, uint32_t frame
     const uint32_t cus = (uint32_t)device_cu_count();
     const bool deep = r->scene->stack_entries > kDeepStack;
     const bool whole = packet && !r->profiling && batch == spp &&
-                       (size_t)batch * npix <= (size_t)cus * (deep || nrc ? kWholePaths : kWholeShallow);
+                       (size_t)batch * npix <= (size_t)cus * (deep || nrc ? kWholePaths : bounces > 1 ? kWholeShallow : kWholeShallowDirect);
     uint32_t per_wave = 8;
     while (per_wave < 64u && (size_t)per_wave * cus * (deep ? 16u : 8u) < (size_t)batch * npix) per_wave *= deep ? 2u : 8u;
     auto paths = nrc ? (pcg ? k_pt_paths<true, true, Pcg32> : k_pt_paths<true, true, uint32_t>)

@@ -1,6 +1,6 @@
 """Small path-tracer batches, traced in one launch, equal the wavefront queues bit for bit.
 
-A batch of up to 1024 paths per CU (262,144 on 256 CUs; 16,384 for plain frames in a shallow tree) runs each path in
+A batch of up to 1024 paths per CU (262,144 on 256 CUs; 65,536 for plain frames in a shallow tree) runs each path in
 registers, 64 paths a wave or, in small batches and deep trees, 8 to 32 with several lanes per ray. Timing a frame's
 stages keeps the queues; both add the same terms to a path in the same order.
 """
@@ -38,7 +38,7 @@ def _frame(scene, ca, w, h, spp, depth, queues, rr=False, rng=0, cache=None):
 @pytest.mark.parametrize("w,h,spp,depth,rr,rng", [
     (1, 1, 1, 5, False, 0), (7, 5, 1, 1, False, 0), (13, 11, 3, 9, True, 0),
     (128, 128, 1, 4, False, 1),   # the last batch of 8 paths a wave in a shallow tree
-    (113, 145, 1, 6, True, 0),    # one more: queues in a shallow tree
+    (113, 145, 1, 6, True, 0),    # one more: 64 a wave
     (256, 257, 1, 5, False, 0), (512, 512, 1, 3, True, 1),  # the largest batch
     (512, 513, 1, 3, False, 0),   # queues
 ])
@@ -50,6 +50,16 @@ def test_whole_paths_equal_queues(name, w, h, spp, depth, rr, rng):
     print(f"{name} {w}x{h} {spp} spp depth {depth}: {n_got}", flush=True)
     assert n_got == n_want and n_got["extension_rays"] >= w * h * spp
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("name", ["cornell", "mixed"])
+@pytest.mark.parametrize("w,h,spp,depth", [
+    (256, 256, 1, 2), (128, 64, 8, 5),    # the last whole paths of more bounces than one in a shallow tree
+    (331, 199, 1, 2),                     # queues
+    (256, 192, 1, 1), (223, 221, 1, 1),   # the last of one bounce, and queues
+])
+def test_limits_of_plain_frames_in_shallow_trees(name, w, h, spp, depth):
+    test_whole_paths_equal_queues(name, w, h, spp, depth, False, 0)
 
 
 @pytest.mark.parametrize("name", list(SCENES))
