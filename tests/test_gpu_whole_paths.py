@@ -104,3 +104,52 @@ def test_whole_paths_leave_the_rows_of_the_queues(name, w, h):
     assert np.isfinite(steps[0]).all()
     a, b = steps
     assert rows[0] == 1 << 18 or np.dot(a, b) >= 0.95 * np.linalg.norm(a) * np.linalg.norm(b)
+
+
+def _cached(scene, cam, w, h, calls, depth=6, weights=None, **kw):
+    """(image, counts, weights afterwards) of a cached render in calls of so many frames"""
+    cache = cb.RadianceCache((-3, -3, -3), (3, 3, 3), seed=3)
+    if weights is not None:
+        cache.set_weights(weights)
+    r = cb.PBRenderer(cb.RenderingMethod.PATHTRACER)
+    r.set_output_size(w, h)
+    r.register_scene(scene)
+    r.set_max_trace_depth(depth)
+    r.set_radiance_cache(cache, **kw)
+    counts = np.zeros(4, np.int64)
+    for spp in calls:
+        r.render(cam, spp)
+        st = r.stats()
+        counts += [st[k] for k in ("extension_rays", "shadow_rays", "cache_queries", "cache_training_rows")]
+    return r.get_output_image(), counts, cache.get_weights()
+
+
+@pytest.mark.parametrize("name", ["cornell", "mixed"])
+@pytest.mark.parametrize("training", [0, 8])
+def test_large_cached_batches_equal_smaller_ones(name, training):
+    """A batch of 2^20 paths asks the cache for the first queries on a second stream, the rest (behind mirrors and
+    glass) after the last bounce; two calls of half as many paths ask once. Their frames are the same."""
+    w, h = 1024, 600
+    desc, ca = SCENES[name]()
+    scene = cb.Scene.from_desc(desc)
+    cam = cb.Camera.look_at(ca["eye"], ca["target"], ca["up"], ca["vfov"], w, h)
+    kw = dict(training_paths=w * h * training // 64, train_steps=0)
+    a, n_a, _ = _cached(scene, cam, w, h, [2], **kw)
+    b, n_b, _ = _cached(scene, cam, w, h, [1, 1], **kw)
+    assert n_a[2] > 0 and (n_a[3] > 0) == (training > 0)
+    assert np.array_equal(n_a, n_b) and np.array_equal(a, b)
+
+
+def test_large_cached_batches_keep_the_estimator():
+    """The same size with a zero cache (every path ends at its second vertex) and with training paths alone."""
+    w, h = 1024, 600
+    desc, ca = SCENES["cornell"]()
+    scene = cb.Scene.from_desc(desc)
+    cam = cb.Camera.look_at(ca["eye"], ca["target"], ca["up"], ca["vfov"], w, h)
+    zero, counts, _ = _cached(scene, cam, w, h, [2], weights=np.zeros(cb.NRC_PARAMS, np.float32), training_paths=0,
+                              train_steps=0)
+    assert counts[2] > 0 and np.array_equal(zero, _frame(scene, ca, w, h, 2, 1, False)[0])
+    w0 = cb.RadianceCache((-3, -3, -3), (3, 3, 3), seed=3).get_weights()
+    full, counts, trained = _cached(scene, cam, w, h, [2], training_paths=w * h, train_steps=2, batch=4096)
+    assert counts[2] == 0 and counts[3] > 0 and np.array_equal(full, _frame(scene, ca, w, h, 2, 6, False)[0])
+    assert np.isfinite(trained).all() and not np.array_equal(trained, w0)
