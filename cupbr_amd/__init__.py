@@ -244,6 +244,7 @@ def lib():
             "cupbr_nrc_set_weights": (C.c_int, [P, P]),
             "cupbr_nrc_infer_device": (C.c_int, [P, P, U32, P, P]),
             "cupbr_nrc_train_device": (C.c_int, [P, P, U32, U32, U32, C.c_float, P, P]),
+            "cupbr_tone_byte_check": (C.c_int, [P]),
             "cupbr_nrc_matrix_core_product": (C.c_int, [P, P, P]),
             "cupbr_renderer_set_radiance_cache": (C.c_int, [P, P, U32, U32, U32, C.c_float]),
             "cupbr_renderer_set_radiance_cache_camera_hit": (C.c_int, [P, C.c_float]),
@@ -294,6 +295,13 @@ def measure_valu_peak(iterations: int = 20000) -> dict:
     _check(lib().cupbr_measure_valu_peak(iterations, C.byref(ms), C.byref(n)))
     return {"ms": ms.value, "wave_instructions": n.value,
             "wave_instructions_per_s": n.value / (ms.value * 1e-3) if ms.value > 0 else float("nan")}
+
+
+def tone_byte_check() -> list:
+    """cupbr_tone_byte_check: floats whose byte the tone maps' fast route decides differently, per curve."""
+    n = (C.c_uint64 * 4)()
+    _check(lib().cupbr_tone_byte_check(n))
+    return list(n)
 
 
 def measure_atomic_peak(iterations: int = 256, words_per_copy: int = 64 ** 3) -> dict:

@@ -783,6 +783,11 @@ int cupbr_tonemapper_tonemap_bloom(cupbr_tonemapper* t, cupbr_post* p, const flo
     return post_bloom(p, curve, t->rgba.as<uint8_t>(), t->type, t->exposure);
 }
 
+int cupbr_tone_byte_check(uint64_t differing[4]) {
+    CHECK_ARG(differing, "null argument");
+    return tone_byte_check(differing);
+}
+
 int cupbr_tonemapper_get_render_buffer_device(const cupbr_tonemapper* t, uint8_t** dev) {
     CHECK_ARG(t && dev, "null argument");
     if (!t->registered)

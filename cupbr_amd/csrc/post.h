@@ -32,6 +32,7 @@ int post_bloom(cupbr_post* p, const float curve[4], uint8_t* rgba, int32_t type,
 // level k (1..5) of the Gaussian pyramid of a w x h image: ((dim_{k-1} + 1) / 2) per axis
 constexpr int kGaussLevels = 5;
 int tonemap(cupbr_tonemapper* t);
+int tone_byte_check(uint64_t differing[4]);
 int write_bmp(const char* path, const uint8_t* rgba, uint32_t w, uint32_t h);
 
 }  // namespace cupbr

@@ -388,6 +388,10 @@ int cupbr_tonemapper_get_render_buffer_device(const cupbr_tonemapper* t, uint8_t
 int cupbr_tonemapper_set_type(cupbr_tonemapper* t, int32_t type);
 int cupbr_tonemapper_get_type(const cupbr_tonemapper* t, int32_t* type);
 int cupbr_tonemapper_set_exposure(cupbr_tonemapper* t, float exposure);
+/* self-check of the tone maps' bytes, which the hardware's log2 and exp2 decide away from the steps: how many
+ * of all 2^32 floats get another byte than powf's from the curves x^(1/2.2) (the two roundings of 1/2.2 that
+ * the channels have) and 1.055 x^(1/2.4) - 0.055, and another 1 - x than the rounded double difference */
+int cupbr_tone_byte_check(uint64_t differing[4]);
 /* saveToFile(path): 32-bit BMP, rows flipped so row 0 of the image is the bottom (ToneMapper.cu:183-198) */
 int cupbr_tonemapper_save_to_file(const cupbr_tonemapper* t, const char* path);
 

@@ -54,3 +54,8 @@ def test_tone_map_of_special_values():
         finite = np.isfinite(x)
         assert np.abs(got - ref)[:, finite].max() <= 1, kind
         assert got[0, 0, 0] == 0 and (got[..., 3] == 255).all()
+
+
+def test_bytes_of_every_float():
+    """The fast route's byte is powf's for each of the 2^32 floats, infinities and NaN among them."""
+    assert cb.tone_byte_check() == [0, 0, 0, 0]
