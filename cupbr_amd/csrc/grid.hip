@@ -165,8 +165,9 @@ __device__ __forceinline__ uint32_t scatter_grad(const GradOut& out, const Stenc
         for (int k = 0; k < 8; ++k)
             if (s.w[k] != 0.0f) atomicAdd(out.rho + s.idx[k], c * s.w[k]);
     }
-    // voxels with a weight (1 - f is never 0)
-    return (s.f[0] != 0.0f ? 2u : 1u) * (s.f[1] != 0.0f ? 2u : 1u) * (s.f[2] != 0.0f ? 2u : 1u);
+    // voxels with a weight (f is 1 just below a voxel's centre, where u - floor(u) rounds up)
+    const auto two = [](float f) { return f != 0.0f && f != 1.0f ? 2u : 1u; };
+    return two(s.f[0]) * two(s.f[1]) * two(s.f[2]);
 }
 
 // parametric range [t0, t1] of o + t d inside the medium box, clipped to [0, tmax]
