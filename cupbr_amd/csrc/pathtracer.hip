@@ -1,14 +1,17 @@
 // PT+NEE in wavefront form (pathtracer_kernel_nee, lib/src/Renderer/PathTracer.cu:97-169).
 //
 // Per batch of paths (one path = one pixel of one reference frame):
-//   raygen      camera rays into extension queue 0                    (PathTracer.cu:112-117)
-//   per bounce: trace    closest hit for the bounce's extension rays   (:126), and any-hit
+//   camera      the camera rays, made and traced as wave packets       (PathTracer.cu:112-126)
+//   per bounce: trace    (from bounce 1 on) closest hit for the bounce's extension rays (:126), and any-hit
 //                        visibility for the previous bounce's shadow rays, adding their
 //                        NEE terms (:64-73), in one launch
 //               shade    emission, NEE sample -> shadow queue,         (:127-158)
 //                        Russian roulette, BSDF sample -> next extension queue
 //   final trace the last bounce's shadow rays
 //   accumulate  the reference running mean, frame by frame             (:162-168)
+// A small batch runs its paths whole in one launch instead (k_pt_paths), then accumulate. Where the camera rays
+// cannot be packets (the visit-counting pass, no tree, a tree deeper than the packets' stack), raygen writes them
+// into extension queue 0 and bounce 0 is a trace like the others.
 // Queue lengths live on the device, so no host round trip happens between bounces.
 // trace is a persistent grid whose waves take pieces of their XCD's rays from its work counter
 // (traversal cost varies per ray; one launch per bounce keeps the GPU full
@@ -36,11 +39,12 @@ namespace cupbr {
 
 constexpr int kPtBlock = 256;
 constexpr int kPtWaves = kPtBlock / 64;
-// traversal stack entries per lane kept in LDS (16 KB per 256-thread block: the trace kernel's 61
+// traversal stack entries per lane kept in LDS (16 KB per 256-thread block: the trace kernel's 63
 // VGPRs, not LDS, then bound its occupancy at 8 waves per SIMD; deeper entries spill to memory)
 constexpr int kPtLds = 16;
-// Batches of up to this many paths per CU run whole paths in one launch (k_pt_paths): as many as are resident at
-// once, 4 waves per SIMD. What bounds a small batch is the longest path's chain of rays and, with a launch and a
+// Batches of up to this many paths per CU run whole paths in one launch (k_pt_paths): as many as plain frames have
+// resident at once with 64 paths a wave (113 VGPRs, 4 waves per SIMD; the 8-lane walk takes 144, 3 waves, and with
+// the cache 192, 2 waves). What bounds a small batch is the longest path's chain of rays and, with a launch and a
 // queue per bounce, the launches; a resident batch needs neither queues nor the path state in memory. Frames of
 // 256x256, 1 spp, depth 5, queues / whole paths (us): spheres and boxes 819 / 277, 1M triangles 1503 / 761; 512x512:
 // 994 / 590, 1623 / 1541. At 331x217, 6 spp (1.6 times the limit) 1003 / 738, but 1786 / 2371.
@@ -364,7 +368,7 @@ __device__ __forceinline__ void pt_shade(const DevScene& S, int cur, uint32_t bo
 
 // Shade without the radiance cache. amdgpu_waves_per_eu(5, 8): 96 VGPRs instead of 102 and 5
 // waves per SIMD instead of 4, without spills (23.7 -> 23.1 ms of shading per 1080p 64-spp step;
-// 6 and 8 waves spill and are slower). The cache variant keeps its 123 VGPRs (it would spill).
+// 6 and 8 waves spill and are slower). The cache variant keeps its 145 VGPRs, 3 waves (it would spill).
 template <class Seed>
 __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(5, 8)))
 void k_pt_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, int rr, const float4* __restrict__ q_o,
@@ -858,9 +862,9 @@ void k_gdpt_camera(DevScene S, uint32_t n, cupbr_camera cam, uint32_t w, uint32_
     });
 }
 
-// one bounce of collect_radiance (:121-156) for every queued path. amdgpu_waves_per_eu(4, 8): 102
-// VGPRs and 4 waves per SIMD (Cornell box 512², 128 spp: 504 Msamples/s; 496 at 5 waves with 96
-// VGPRs, 478 at 6 waves with 80 VGPRs and a 24-byte spill).
+// one bounce of collect_radiance (:121-156) for every queued path. amdgpu_waves_per_eu(4, 8): 95 VGPRs and 5 waves
+// per SIMD since it touches only the state that changes. (Before that, with 102 VGPRs at 4 waves, forcing 5 waves
+// cost 1.6%, and 6 waves, with a 24-byte spill, 5%: Cornell box 512², 128 spp, 504, 496 and 478 Msamples/s.)
 __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_gdpt_shade(DevScene S, int cur, uint32_t bounce, uint32_t max_depth, const float4* __restrict__ q_o,
                   const float4* __restrict__ q_d, const float2* __restrict__ q_hit, float4* __restrict__ nq_o,
